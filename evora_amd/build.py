@@ -5,12 +5,12 @@
 Every translation unit is compiled for gfx950 only.  The staged kernels, the
 exact builds of the fused and conduction kernels, and the gravity kernels are
 compiled without floating-point contraction so that their FP64 results follow
-the reference's operation order.  The FP32-mixed builds of the march are
-compiled without it too: the compiler fuses a product into a neighbouring add
-differently at different inlined call sites of the same FP32 code, and the
-march forms one cell's values at several (a ring lane or an interior lane, a
-z chunk's first planes or the plane ahead), so that a contracted FP32 result
-would depend on the launch shape.  Packed FP32 instructions are disabled for
+the reference's operation order.  The other builds of the march are compiled
+without it too, with their fused operations placed by hand: the compiler fuses
+a product into a neighbouring add differently at different inlined call sites
+of the same code, and the march forms one cell's values at several (a ring
+lane or an interior lane, a z chunk's first planes or the plane ahead), so
+that a contracted result would depend on the launch shape.  Packed FP32 instructions are disabled for
 all device code.  The library links hipFFT (ROCm) for the Poisson solve on
 grids whose sides are not all powers of two.
 """
@@ -37,14 +37,14 @@ COMMON = [
 UNITS = [
     ("api.o", "api.hip", []),
     ("staged.o", "staged.hip", ["-ffp-contract=off"]),
-    ("fused64.o", "fused.hip", ["-DEVH_FUSED_PREC=64"]),
+    ("fused64.o", "fused.hip", ["-DEVH_FUSED_PREC=64", "-ffp-contract=off"]),
     ("fused32.o", "fused.hip", ["-DEVH_FUSED_PREC=32", "-ffp-contract=off"]),
     ("fused64x.o", "fused.hip", ["-DEVH_FUSED_PREC=64", "-DEVH_FUSED_EXACT=1", "-ffp-contract=off"]),
     ("conduction.o", "conduction.hip", []),
     ("conductionx.o", "conduction.hip", ["-DEVH_COND_EXACT=1", "-ffp-contract=off"]),
     ("gravity.o", "gravity.hip", ["-ffp-contract=off"]),
     ("mathcheck.o", "mathcheck.hip", []),
-    ("batch64.o", "batch.hip", ["-DEVH_FUSED_PREC=64"]),
+    ("batch64.o", "batch.hip", ["-DEVH_FUSED_PREC=64", "-ffp-contract=off"]),
     ("batch32.o", "batch.hip", ["-DEVH_FUSED_PREC=32", "-ffp-contract=off"]),
 ]
 

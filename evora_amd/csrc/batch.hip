@@ -79,11 +79,11 @@ __device__ __forceinline__ int box_of(const BoxDev *boxes, int nbox, int item) {
   return lo;
 }
 
-template <typename T, typename S, int SOLVER, int LIMITER, int TY, int WPE>
-__global__ void __launch_bounds__(core::TileShape<TY>::NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, int WPE>
+__global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     k_batch_fused(const BoxDev *__restrict__ boxes, int nbox, S *__restrict__ q0, S *__restrict__ q1, BoxState bs,
                   Queues *qs) {
-  __shared__ core::Smem<T, TY> sm;
+  __shared__ core::Smem<T, TX, TY> sm;
   __shared__ int s_item;
   const int xcd = blockIdx.x % kXcds;
   for (;;) {
@@ -96,8 +96,10 @@ __global__ void __launch_bounds__(core::TileShape<TY>::NT) __attribute__((amdgpu
       // k_batch_dt has flipped the side of every box that steps: the new
       // state goes to that buffer, the current one is read from the other
       const BoxDev &bx = boxes[b];
+      const KParams P = bx.P;
+      const Geo G = bx.G;
       const bool to1 = bs.side[b] != 0;
-      core::march<T, S, SOLVER, LIMITER, TY, false>(bx.P, bx.G, to1 ? q0 : q1, to1 ? q1 : q0, bx.qoff, b, bs.dt[b],
+      core::march<T, S, SOLVER, LIMITER, TX, TY, false>(P, G, to1 ? q0 : q1, to1 ? q1 : q0, bx.qoff, b, bs.dt[b],
                                                     &bs.st[b], &bs.st[b].vmin_bits, item - bx.tile0, sm);
     }
     __syncthreads();  // s_item is rewritten only after every lane has used it
@@ -164,24 +166,22 @@ namespace evh {
 namespace batch {
 
 // launchers for this translation unit's precision
-template <typename T, typename S, int SOLVER, int LIMITER, int TY, int WPE>
+template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, int WPE>
 static void launch(const BoxDev *boxes, int nbox, void *q0, void *q1, const BoxState &bs, Queues *qs, int blocks,
                    hipStream_t stream) {
-  hipLaunchKernelGGL((k_batch_fused<T, S, SOLVER, LIMITER, TY, WPE>), dim3(blocks),
-                     dim3(core::TileShape<TY>::NT), 0, stream, boxes, nbox, (S *)q0, (S *)q1, bs, qs);
+  hipLaunchKernelGGL((k_batch_fused<T, S, SOLVER, LIMITER, TX, TY, WPE>), dim3(blocks),
+                     dim3((core::TileShape<TX, TY>::NT)), 0, stream, boxes, nbox, (S *)q0, (S *)q1, bs, qs);
 }
 
+// tx x ty: 16 x 8, 16 x 12 or, in FP32, 32 x 6; waves per SIMD as in the single-grid
+// kernel, FP64 2 and FP32 4
 template <typename T, typename S, int SOLVER, int LIMITER>
-static void launch_shape(int ty, bool hi, const BoxDev *boxes, int nbox, void *q0, void *q1, const BoxState &bs,
+static void launch_shape(int tx, int ty, const BoxDev *boxes, int nbox, void *q0, void *q1, const BoxState &bs,
                          Queues *qs, int blocks, hipStream_t stream) {
-  constexpr int LO = sizeof(T) == 8 ? 2 : 3, HI = LO + 1;
-  if (ty == 8) {
-    if (hi) launch<T, S, SOLVER, LIMITER, 8, HI>(boxes, nbox, q0, q1, bs, qs, blocks, stream);
-    else launch<T, S, SOLVER, LIMITER, 8, LO>(boxes, nbox, q0, q1, bs, qs, blocks, stream);
-  } else {
-    if (hi) launch<T, S, SOLVER, LIMITER, 12, HI>(boxes, nbox, q0, q1, bs, qs, blocks, stream);
-    else launch<T, S, SOLVER, LIMITER, 12, LO>(boxes, nbox, q0, q1, bs, qs, blocks, stream);
-  }
+  constexpr int W = sizeof(T) == 8 ? 2 : 4;
+  if (ty == 8) launch<T, S, SOLVER, LIMITER, 16, 8, W>(boxes, nbox, q0, q1, bs, qs, blocks, stream);
+  else if (tx == 16) launch<T, S, SOLVER, LIMITER, 16, 12, W>(boxes, nbox, q0, q1, bs, qs, blocks, stream);
+  else if constexpr (sizeof(T) == 4) launch<T, S, SOLVER, LIMITER, 32, 6, W>(boxes, nbox, q0, q1, bs, qs, blocks, stream);
 }
 
 #if EVH_FUSED_PREC == 32
@@ -192,9 +192,9 @@ using TT = float;
 using TT = double;
 #endif
 
-hipError_t EVH_BATCH_LAUNCH(int solver, int limiter, int ty, bool hi, const BoxDev *boxes, int nbox, void *q0,
+hipError_t EVH_BATCH_LAUNCH(int solver, int limiter, int tx, int ty, const BoxDev *boxes, int nbox, void *q0,
                             void *q1, const BoxState &bs, Queues *qs, int blocks, hipStream_t stream) {
-#define EVH_L(SV, LM) launch_shape<TT, TT, SV, LM>(ty, hi, boxes, nbox, q0, q1, bs, qs, blocks, stream)
+#define EVH_L(SV, LM) launch_shape<TT, TT, SV, LM>(tx, ty, boxes, nbox, q0, q1, bs, qs, blocks, stream)
   if (solver == 1 && limiter == 1) EVH_L(1, 1);
   else if (solver == 1 && limiter == 2) EVH_L(1, 2);
   else if (solver == 1 && limiter == 3) EVH_L(1, 3);
@@ -213,7 +213,7 @@ hipError_t EVH_BATCH_LAUNCH(int solver, int limiter, int ty, bool hi, const BoxD
 #if EVH_FUSED_PREC == 64
 namespace evh {
 namespace batch {
-hipError_t launch_batch_f32(int, int, int, bool, const BoxDev *, int, void *, void *, const BoxState &, Queues *, int,
+hipError_t launch_batch_f32(int, int, int, int, const BoxDev *, int, void *, void *, const BoxState &, Queues *, int,
                             hipStream_t);
 }  // namespace batch
 }  // namespace evh
@@ -242,6 +242,7 @@ struct evh_batch {
   std::vector<char> cfl_needed;
   // launch shape
   int tile_ty = 12, wpe_hi = 1, zchunk = 64, blocks_per_cu = 2;
+  int tx = 16, ty = 12;  // the column tile that tile_ty stands for (pick_tile)
   // one step of the ensemble, captured once (the kernels read each box's
   // buffer side from device memory)
   hipGraphExec_t gexec = nullptr;
@@ -314,11 +315,28 @@ int gridsz(long long work) {
   return (int)(g < 1 ? 1 : (g > 8192 ? 8192 : g));
 }
 
-// Descriptors of nbox boxes (box i at element offset 6 qoff[i]) for tile
-// height ty and z chunk zc, and the per-XCD work queues over their tiles;
+// The march's column tile for tile height tile_ty: 16 x 8 for 8, otherwise
+// 16 x 12 or, in FP32, 32 x 6, whichever suits the boxes together (tiling.h).
+void pick_tile(const evh_config *cfgs, int nbox, int tile_ty, int *tx, int *ty) {
+  *tx = 16;
+  *ty = tile_ty;
+  if (tile_ty == 8 || cfgs[0].precision != EVH_FP32_MIXED) return;
+  long long n32 = 0, n16 = 0;  // tiles of a plane, weighted by the box's planes
+  for (int i = 0; i < nbox; i++) {
+    n32 += tiles_of(cfgs[i].nx, cfgs[i].ny, 32, 6) * cfgs[i].nz;
+    n16 += tiles_of(cfgs[i].nx, cfgs[i].ny, 16, 12) * cfgs[i].nz;
+  }
+  if (wide_tile(n32, n16)) {
+    *tx = 32;
+    *ty = 6;
+  }
+}
+
+// Descriptors of nbox boxes (box i at element offset 6 qoff[i]) for tiles
+// of tx x ty columns and z chunk zc, and the per-XCD work queues over their tiles;
 // returns the number of work items.
 int describe_boxes(const evh_config *cfgs, const KParams *kps, const long long *ncell, const long long *qoff,
-                   int nbox, int ty, int zc, BoxDev *out, Queues *q) {
+                   int nbox, int tx, int ty, int zc, BoxDev *out, Queues *q) {
   int items = 0;
   for (int i = 0; i < nbox; i++) {
     const evh_config &c = cfgs[i];
@@ -328,7 +346,7 @@ int describe_boxes(const evh_config *cfgs, const KParams *kps, const long long *
     g.nz = c.nz;
     g.n = ncell[i];
     g.zchunk = zc > g.nz ? g.nz : zc;
-    g.tiles_x = (g.nx + core::TX - 1) / core::TX;
+    g.tiles_x = (g.nx + tx - 1) / tx;
     g.tiles_y = (g.ny + ty - 1) / ty;
     g.nchunks = (g.nz + g.zchunk - 1) / g.zchunk;
     g.ntiles = g.tiles_x * g.tiles_y * g.nchunks;
@@ -349,7 +367,8 @@ int describe_boxes(const evh_config *cfgs, const KParams *kps, const long long *
 int rebuild_items(evh_batch *b) {
   std::vector<BoxDev> h(b->nbox);
   Queues q;
-  b->nitems = describe_boxes(b->cfgs.data(), b->kps.data(), b->ncell.data(), b->qoff.data(), b->nbox, b->tile_ty,
+  pick_tile(b->cfgs.data(), b->nbox, b->tile_ty, &b->tx, &b->ty);
+  b->nitems = describe_boxes(b->cfgs.data(), b->kps.data(), b->ncell.data(), b->qoff.data(), b->nbox, b->tx, b->ty,
                              b->zchunk, h.data(), &q);
   BHIP(hipMemcpy(b->boxes_d, h.data(), sizeof(BoxDev) * b->nbox, hipMemcpyHostToDevice));
   BHIP(hipMemcpy(b->qs_d, &q, sizeof(Queues), hipMemcpyHostToDevice));
@@ -366,9 +385,9 @@ hipError_t launch_step(evh_batch *b) {
   const int blocks = b->blocks_per_cu * b->num_cu;
   const evh_config &c = b->cfgs[0];
   if (b->precision == EVH_FP32_MIXED)
-    return launch_batch_f32(c.solver, c.limiter, b->tile_ty, b->wpe_hi != 0, b->boxes_d, nb, b->qbuf[0], b->qbuf[1],
+    return launch_batch_f32(c.solver, c.limiter, b->tx, b->ty, b->boxes_d, nb, b->qbuf[0], b->qbuf[1],
                             b->bs, b->qs_d, blocks, b->stream);
-  return launch_batch_f64(c.solver, c.limiter, b->tile_ty, b->wpe_hi != 0, b->boxes_d, nb, b->qbuf[0], b->qbuf[1],
+  return launch_batch_f64(c.solver, c.limiter, b->tx, b->ty, b->boxes_d, nb, b->qbuf[0], b->qbuf[1],
                           b->bs, b->qs_d, blocks, b->stream);
 }
 
@@ -828,8 +847,10 @@ int evh_batch_run_noalloc(const evh_config *cfgs, int nbox, void *q0, void *q1, 
     off += ncell[i];
   }
   // the launch shape evh_batch_create starts with
-  const int ty = 12, zc = 64, wpe_hi = 1, bpc = f32 ? 4 : 2;
-  describe_boxes(cfgs, kps, ncell, qoff, nbox, ty, zc, img.boxes, &img.qs);
+  const int zc = 64, bpc = f32 ? 4 : 2;
+  int tx, ty;
+  pick_tile(cfgs, nbox, 12, &tx, &ty);
+  describe_boxes(cfgs, kps, ncell, qoff, nbox, tx, ty, zc, img.boxes, &img.qs);
   for (int i = 0; i < nbox; i++) {
     img.t[i] = t[i];
     img.tend[i] = tend[i];
@@ -874,10 +895,10 @@ int evh_batch_run_noalloc(const evh_config *cfgs, int nbox, void *q0, void *q1, 
     e = hipGetLastError();
     if (e != hipSuccess) break;
     if (f32)
-      e = launch_batch_f32(c0.solver, c0.limiter, ty, wpe_hi != 0, dev->boxes, nbox, q0, q1, bs, &dev->qs,
+      e = launch_batch_f32(c0.solver, c0.limiter, tx, ty, dev->boxes, nbox, q0, q1, bs, &dev->qs,
                            bpc * cu, 0);
     else
-      e = launch_batch_f64(c0.solver, c0.limiter, ty, wpe_hi != 0, dev->boxes, nbox, q0, q1, bs, &dev->qs,
+      e = launch_batch_f64(c0.solver, c0.limiter, tx, ty, dev->boxes, nbox, q0, q1, bs, &dev->qs,
                            bpc * cu, 0);
   }
   if (e == hipSuccess) e = hipDeviceSynchronize();

@@ -18,12 +18,13 @@ namespace evh {
 namespace fm {
 
 // ---- double
+// One third-order step on the hardware estimate (relative error e below
+// 2^-24): r (1 + e + e^2), the dropped terms e^3 below 2^-72.  The final fma
+// rounds once, as a second Newton step would, with one operation less.
 __device__ __forceinline__ double rcp(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  double e = __builtin_fma(-x, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-x, r, 1.0);
-  return __builtin_fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
 // The IEEE quotient a/d, rounded to nearest, from y = rcp(d) above or from
@@ -155,25 +156,23 @@ __device__ __forceinline__ double expm1_tiny(double c) {
   return __builtin_fma(__builtin_fma(c, 1.0 / 6.0, 0.5), c * c, c);
 }
 
-// 1/sqrt(x) for positive, normal x (two Newton steps on the rsq estimate)
-__device__ __forceinline__ double rsqrt_pos(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double hx = 0.5 * x;
-  double e = __builtin_fma(-hx * y, y, 0.5);
-  y = __builtin_fma(y, e, y);
-  e = __builtin_fma(-hx * y, y, 0.5);
-  return __builtin_fma(y, e, y);
+// n / sqrt(x) for positive, normal x: the rsq estimate y (relative error
+// below 2^-23) with the third-order step (1 - e)^(-1/2) = 1 + e/2 + 3e^2/8 of
+// e = 1 - x y^2 (the dropped term, 5e^3/16, is below 2^-68) applied to n y
+__device__ __forceinline__ double div_sqrt_pos(double n, double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x * y, y, 1.0);
+  const double a = n * y;
+  return __builtin_fma(a * e, __builtin_fma(e, 0.375, 0.5), a);
 }
 
-// a*b + c.  FP32: one fused instruction, placed here by hand (the FP32
-// build of the march is compiled without contraction, so that every inlined
-// call site rounds alike).  FP64: the expression itself, contracted by the
-// fast build and left unfused by the exact build.
-template <typename T>
-__device__ __forceinline__ T fmad(T a, T b, T c) {
-  if constexpr (sizeof(T) == 4) return __builtin_fmaf(a, b, c);
-  else return a * b + c;
-}
+// a*b + c fused, and |a|, in either type.  The builds of the march are
+// compiled without contraction and place every fused operation by hand, so
+// that each inlined call site of the same expression rounds alike.
+__device__ __forceinline__ double fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fabs(double a) { return __builtin_fabs(a); }
+__device__ __forceinline__ float fabs(float a) { return __builtin_fabsf(a); }
 
 // ---- float (hardware transcendentals; ~1-2 ulp)
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -181,7 +180,7 @@ __device__ __forceinline__ float sqrt_pos(float x) { return __builtin_amdgcn_sqr
 __device__ __forceinline__ float pow_pos(float x, float y) {
   return __builtin_amdgcn_exp2f(y * __builtin_amdgcn_logf(x));
 }
-__device__ __forceinline__ float rsqrt_pos(float x) { return __builtin_amdgcn_rsqf(x); }
+__device__ __forceinline__ float div_sqrt_pos(float n, float x) { return n * __builtin_amdgcn_rsqf(x); }
 
 }  // namespace fm
 }  // namespace evh

@@ -1,7 +1,7 @@
 // fused.hip -- the whole 3-D hydro step of one grid in one HBM pass.
 //
 // k_fused runs the tile march of fused_core.h over one grid: one block per
-// (16 x TY tile, z chunk), with the tiles of each XCD contiguous; on 2-D
+// (column tile, z chunk), with the tiles of each XCD contiguous; on 2-D
 // grids (nz = 1), k_fused2d marches row strips along y (march2d.h).  k_cfl
 // gives the first step's CFL limit.  The file is compiled three times:
 // EVH_FUSED_PREC=64 (FP64, fast arithmetic), EVH_FUSED_PREC=32 (FP32-mixed)
@@ -36,16 +36,16 @@ namespace {
 using core::Geo;
 
 // WPE: waves per SIMD the register allocation must leave room for
-// (512 / WPE VGPRs per lane); the tuning knob next to the tile height TY.
+// (512 / WPE VGPRs per lane).
 // SLAB: a z-slab whose ghost planes may come from halo buffers.
-template <typename T, typename S, int SOLVER, int LIMITER, int TY, int WPE, bool SLAB>
-__global__ void __launch_bounds__(core::TileShape<TY>::NT) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, int WPE, bool SLAB>
+__global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     K_FUSED(KParams P, Geo G, const S *__restrict__ qin, S *__restrict__ qout, double dt, Status *st,
             S *__restrict__ tout) {
-  __shared__ core::Smem<T, TY> sm;
+  __shared__ core::Smem<T, TX, TY> sm;
   const int lin = xcd_tile(blockIdx.x, G.ntiles);
   if (lin < 0) return;  // padding block (whole block exits before any barrier)
-  core::march<T, S, SOLVER, LIMITER, TY, kExact, SLAB>(P, G, qin, qout, 0, 0, dt, st, &st->vmin_bits, lin, sm,
+  core::march<T, S, SOLVER, LIMITER, TX, TY, kExact, SLAB>(P, G, qin, qout, 0, 0, dt, st, &st->vmin_bits, lin, sm,
                                                         tout);
 }
 
@@ -77,13 +77,13 @@ __global__ void __launch_bounds__(256) k_cfl(KParams P, Geo G, const S *__restri
   if ((threadIdx.x & 63) == 0) atomic_min_pos(&st->vmin_bits, vmin);
 }
 
-Geo make_geo(const evh_ctx *h, int ty) {
+Geo make_geo(const evh_ctx *h, int tx, int ty) {
   Geo g;
   g.nx = h->grid.nx;
   g.ny = h->grid.ny;
   g.nz = h->grid.nz;
   g.n = h->grid.n();
-  g.tiles_x = (g.nx + core::TX - 1) / core::TX;
+  g.tiles_x = (g.nx + tx - 1) / tx;
   g.tiles_y = (g.ny + ty - 1) / ty;
   g.zchunk = h->zchunk > 0 ? h->zchunk : z_chunk((long long)g.tiles_x * g.tiles_y, g.nz, 64);
   if (g.zchunk > g.nz) g.zchunk = g.nz;
@@ -94,11 +94,11 @@ Geo make_geo(const evh_ctx *h, int ty) {
   return g;
 }
 
-template <typename T, typename S, int SOLVER, int LIMITER, int TY, int WPE, bool SLAB = false>
+template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, int WPE, bool SLAB = false>
 void launch_ty(evh_ctx *h, double dt) {
-  const Geo g = make_geo(h, TY);
+  const Geo g = make_geo(h, TX, TY);
   const int blocks = xcd_blocks(g.ntiles);
-  hipLaunchKernelGGL((K_FUSED<T, S, SOLVER, LIMITER, TY, WPE, SLAB>), dim3(blocks), dim3(core::TileShape<TY>::NT), 0,
+  hipLaunchKernelGGL((K_FUSED<T, S, SOLVER, LIMITER, TX, TY, WPE, SLAB>), dim3(blocks), dim3((core::TileShape<TX, TY>::NT)), 0,
                      h->stream, h->kp, g, (const S *)h->qbuf[h->cur], (S *)h->qbuf[1 - h->cur], dt, h->st,
                      (S *)h->tbuf);
 }
@@ -123,32 +123,34 @@ void launch_2d(evh_ctx *h, double dt) {
                      (S *)h->tbuf);
 }
 
-// tuning variants: tile height 8 or 12, waves per SIMD (FP64: 2 or 3, FP32: 3
-// or 4); 2-D grids take the row-strip march in its one shape
+// The register budget is 2 waves per SIMD in FP64 (a column's values take
+// about 220 of the 256 registers it leaves; 168 for 3 waves spill 64: 12.4 ms
+// against 5.8 at 512^3) and 4 in FP32.  2-D grids take the row-strip march in
+// its one shape.
 template <typename T, typename S, int SOLVER, int LIMITER>
 void launch_fused_t(evh_ctx *h, double dt) {
-  constexpr int LO = sizeof(T) == 8 ? 2 : 3, HI = LO + 1;
+  constexpr int W = sizeof(T) == 8 ? 2 : 4;
+  const int nx = h->grid.nx, ny = h->grid.ny;
   if (h->grid.nz == 1) {
-    // 2-D: FP64 at 3 waves per SIMD (its row carry in LDS, 16 B/lane
-    // spilled: 3% faster than 2 waves at 8192^2), FP32 at 4 without spills
-    // (5 spill 32 B/lane and measured 4% slower)
+    // 2-D: FP64 at 3 waves per SIMD (its row carry in LDS: 3% faster than 2
+    // waves at 8192^2), FP32 at 4
     launch_2d<T, S, SOLVER, LIMITER, sizeof(T) == 8 ? 3 : 4>(h, dt);
     return;
   }
-  if (h->zslab[0] || h->zslab[1]) {
-    // a z-slab with halo buffers: the default tile shape (the z chunk is
-    // still the tuning's)
-    launch_ty<T, S, SOLVER, LIMITER, 12, HI, true>(h, dt);
+  const bool slab = h->zslab[0] || h->zslab[1];  // with halo buffers: tile height 12 (the z chunk is the tuning's)
+  if (!slab && h->tile_ty == 8) {
+    launch_ty<T, S, SOLVER, LIMITER, 16, 8, W>(h, dt);
     return;
   }
-  const bool hi = h->wpe_hi;
-  if (h->tile_ty == 8) {
-    if (hi) launch_ty<T, S, SOLVER, LIMITER, 8, HI>(h, dt);
-    else launch_ty<T, S, SOLVER, LIMITER, 8, LO>(h, dt);
-  } else {
-    if (hi) launch_ty<T, S, SOLVER, LIMITER, 12, HI>(h, dt);
-    else launch_ty<T, S, SOLVER, LIMITER, 12, LO>(h, dt);
+  if constexpr (sizeof(T) == 4) {
+    if (wide_tile(tiles_of(nx, ny, 32, 6), tiles_of(nx, ny, 16, 12))) {
+      if (slab) launch_ty<T, S, SOLVER, LIMITER, 32, 6, W, true>(h, dt);
+      else launch_ty<T, S, SOLVER, LIMITER, 32, 6, W>(h, dt);
+      return;
+    }
   }
+  if (slab) launch_ty<T, S, SOLVER, LIMITER, 16, 12, W, true>(h, dt);
+  else launch_ty<T, S, SOLVER, LIMITER, 16, 12, W>(h, dt);
 }
 
 template <typename T, typename S>
@@ -171,7 +173,7 @@ hipError_t launch_fused_prec(evh_ctx *h, double dt) {
 bool fused_supported(const evh_config &c) { return c.nx >= 2 && c.ny >= 2 && c.nz >= 1; }
 
 hipError_t launch_cfl(evh_ctx *h) {
-  const Geo g = make_geo(h, 12);
+  const Geo g = make_geo(h, 16, 12);
   long long b = (g.n + 255) / 256;
   if (b > 8192) b = 8192;
   if (h->cfg.precision == EVH_FP32_MIXED)

@@ -2,33 +2,46 @@
 // single-grid kernel (fused.hip) and the batched persistent kernel
 // (batch.hip).
 //
-// A block owns a 16 x TY column tile of one box and marches up a chunk of z
+// A block owns a TX x TY column tile of one box and marches up a chunk of z
 // planes, reading q^n once and writing q^{n+1} once; w, evo and s never
-// exist in HBM.  Waves 0..TY/4-1 own the 16*TY interior columns one to one;
-// the last wave (the "ring wave") owns the 2*(16+TY) columns of the first
-// halo ring and loads the second ring and the four corners, so every
-// interior lane does useful work in every stage.  Per plane k:
-//   S1  primitive (comp.f90:26-85) of plane k+1 for every owned column, with
-//       the ghost cells of `bound` (boundary.f90) folded into the load index
-//       (a column's x-y offset is formed once per march); plane k goes to
-//       LDS with both halo rings.  The ring wave's second-ring cells of
-//       plane k were formed in its idle time of S2 of plane k-1.
-//   S2  limited slopes in x, y, z and the predictor evo (muscl.f90:45-169)
-//       of plane k; the x/y face states go to LDS per face; the interior
+// exist in HBM.  The interior waves (TX TY / 64 of them) own the tile's
+// columns one to one; the last wave (the "ring wave") owns the 2 (TX + TY)
+// columns of the first halo ring, one or two per lane, and loads the second
+// ring and the four corners, so every interior lane does useful work in every
+// stage.  The two roles run loops of their own with the same barriers.  Per
+// plane k:
+//   S1  w of plane k goes to LDS with both halo rings.
+//   S2  primitive (comp.f90:26-85) of plane k+1, with the ghost cells of
+//       `bound` (boundary.f90) folded into the load index (a column's x-y
+//       offset is formed once per march; the ring wave forms its own ahead,
+//       in S3, and its second-ring cells' here); limited slopes in x, y, z
+//       and the predictor evo (muscl.f90:45-169) of plane k; the x/y face states go to LDS per face; the interior
 //       lanes solve their z face k-1/2 (riemann.f90) and finish plane k-1
 //       as (q + dtx*(Fx) + dty*(Fy)) + dtz*(Fz), the reference's x, y, z
-//       order (muscl.f90:191-272, integration :287), and store it.
+//       order (muscl.f90:191-272, integration :287), store it, and take the
+//       primitive and the CFL limit of those of its cells that can change
+//       the minimum for the next hydrostep (timestep.f90:26-57; CflMin).
 //   S3  x and y faces of plane k: interior lane (i,j) solves its left and
-//       bottom faces, the ring wave the TY right-edge and 16 top-edge faces
+//       bottom faces, the ring wave the TY right-edge and TX top-edge faces
 //       in one solve.  Each flux overwrites the two states it came from.
-//   S4  q(k) + dtx*(Fx) + dty*(Fy) of plane k, kept for S2 of plane k+1;
-//       then the primitive and the CFL limit of the stored plane k-1, which
-//       feed a min reduction for the next hydrostep (timestep.f90:26-57).
-//       They sit where the interior waves have the least to do.
+//   S4  q(k) + dtx*(Fx) + dty*(Fy) of plane k, carried in registers with the
+//       z flux and the top z state to S2 of plane k+1.
 // Template parameters: T compute type, S storage type of q (double/double
 // for the FP64 form, float/float for the FP32-mixed form), SOLVER, LIMITER,
-// TY the tile height (4, 8 or 12).  2-D grids march along y instead
-// (march2d.h).
+// TX x TY the tile.  2-D grids march along y instead (march2d.h).
+//
+// What bounds it: FP64, the issue of vector instructions (a wave64 FP64
+// instruction takes about 5 cycles of its SIMD, and the SIMDs that hold
+// interior waves only have one to issue 98% of the time); FP32-mixed, the
+// L1's requests to L2 for the ring.  512^3 HLLC blast, FP64: 6.36 ms with both
+// roles in one loop (219 VGPRs), the carry in LDS and every cell's limit
+// formed; 5.62 ms (23.9 G cell updates/s) with a loop per role, so that
+// neither holds the other's values (205 VGPRs with the carry in registers,
+// 32 of 135 LDS operations per plane gone, 46 KB of LDS instead of 72),
+// third-order reciprocals and roots, the star flux from its jump conditions,
+// the predictor from shared factors, and the limit only where it can count.
+// FP32-mixed: 3.33 -> 2.95 ms (45.5 G), with its constants in scalar
+// registers (16 B/lane of spills gone).
 #pragma once
 
 #include "evh_internal.h"
@@ -37,19 +50,20 @@
 namespace evh {
 namespace core {
 
-constexpr int TX = 16;
-
-template <int TY>
+template <int TX_, int TY_>
 struct TileShape {
-  static constexpr int NI = TX * TY;          // interior lanes
-  static constexpr int NT = NI + 64;          // + the ring wave
-  static constexpr int NR1 = 2 * TX + 2 * TY; // first-ring columns
-  static constexpr int EW = TX + 4;           // extended plane pitch (x from -2 to TX+1)
-  static constexpr int EA = EW * (TY + 4);    // extended plane area
-  static constexpr int NFX = (TX + 1) * TY;   // x faces of a plane
-  static constexpr int NFY = TX * (TY + 1);   // y faces of a plane
+  static constexpr int TX = TX_, TY = TY_;
+  static constexpr int NI = TX * TY;              // interior lanes
+  static constexpr int NT = NI + 64;              // + the ring wave
+  static constexpr int NR1 = 2 * TX + 2 * TY;     // first-ring columns
+  static constexpr int NP = (NR1 + 4 + 63) / 64;  // columns and corners per ring lane
+  static constexpr int EW = TX + 4;               // extended plane pitch (x from -2 to TX+1)
+  static constexpr int EA = EW * (TY + 4);        // extended plane area
+  static constexpr int NFX = (TX + 1) * TY;       // x faces of a plane
+  static constexpr int NFY = TX * (TY + 1);       // y faces of a plane
   static_assert(NI % 64 == 0, "interior lanes must fill whole wavefronts");
-  static_assert(NR1 + 4 <= 64, "ring columns and corners must fit one wavefront");
+  static_assert(TX + TY <= 64, "the edge faces must fit one wavefront");
+  __device__ static __forceinline__ int eidx(int x, int y) { return (x + 2) + EW * (y + 2); }
 };
 
 struct Geo {
@@ -64,9 +78,6 @@ struct Geo {
   const void *zlo, *zhi;
 };
 
-template <int TY>
-__device__ __forceinline__ int eidx(int x, int y) { return (x + 2) + TileShape<TY>::EW * (y + 2); }
-
 // mixed form: FP64 pressure recovery where the flow is fast
 template <typename T>
 struct Prim;
@@ -80,6 +91,11 @@ struct Prim<double> {
 
 template <>
 struct Prim<float> {
+  // 0.5 m^2 / rho in FP64, an IEEE quotient
+  __device__ static __forceinline__ double kin64(const float q[6]) {
+    const double r = q[0];
+    return fm::div_cr(0.5 * (double(q[1]) * q[1] + double(q[2]) * q[2] + double(q[3]) * q[3]), r, fm::rcp(r));
+  }
   // FP32 recovery, except where the subtraction E - kin cancels: there
   // (kin/E above the Mach threshold) p = g1 (E - kin) is evaluated in FP64.
   // With dualenergy on, the entropy branch (kin/E > de_thresh1,
@@ -90,13 +106,13 @@ struct Prim<float> {
     w[1] = q[1] * rinv;
     w[2] = q[2] * rinv;
     w[3] = q[3] * rinv;
-    const float m2 = fm::fmad(q[3], q[3], fm::fmad(q[2], q[2], q[1] * q[1]));
+    const float m2 = fm::fma(q[3], q[3], fm::fma(q[2], q[2], q[1] * q[1]));
     const float kin = 0.5f * m2 * rinv;
-    const bool fast_flow = kin > float(P.kin_frac64) * q[4];
+    const bool fast_flow = kin > P.f.kin_frac64 * q[4];
     float pr;
-    if (P.dualenergy && kin * fm::rcp(q[4]) > float(P.de_thresh1)) {
+    if (P.dualenergy && kin * fm::rcp(q[4]) > P.f.de_thresh1) {
       const double r64 = double(q[0]);
-      const double k64 = 0.5 * (double(q[1]) * q[1] + double(q[2]) * q[2] + double(q[3]) * q[3]) / r64;
+      const double k64 = kin64(q);
       // (the Newton form of the power: this rare branch must not raise the
       // register count of the whole FP32 kernel)
       const double p64 = double(q[5]) * fast::pow_g1<false>(P, r64);
@@ -104,10 +120,9 @@ struct Prim<float> {
       pr = float(p64);
     } else {
       if (fast_flow) {
-        const double k64 = 0.5 * (double(q[1]) * q[1] + double(q[2]) * q[2] + double(q[3]) * q[3]) / double(q[0]);
-        pr = float(P.g1 * (double(q[4]) - k64));
+        pr = float(P.g1 * (double(q[4]) - kin64(q)));
       } else {
-        pr = float(P.g1) * (q[4] - kin);
+        pr = P.f.g1 * (q[4] - kin);
       }
       if (P.dualenergy) q[5] = pr * fast::rpow_g1(P, q[0]);
     }
@@ -117,10 +132,10 @@ struct Prim<float> {
 };
 
 // Arithmetic of the march.  Phys<false> is the fast form (physics_fast.h:
-// refined hardware reciprocals and roots, cube-root powers, FMA contraction
-// in the Riemann solvers; in FP64 the primitive recovery and the predictor
-// keep the reference's roundings, with IEEE quotients from shared
-// reciprocals).
+// refined hardware reciprocals and roots, cube-root powers, fused operations
+// in the predictor, the Riemann solvers and the update; in FP64 the primitive
+// recovery and the sum of a face state keep the reference's roundings, with
+// IEEE quotients from shared reciprocals).
 // Phys<true> is the reference's own arithmetic (physics.h: IEEE division
 // and square root, the reference's operation order; its translation unit is
 // compiled without FMA contraction), so that every face state, flux and
@@ -139,9 +154,25 @@ struct Phys<false> {
   __device__ static __forceinline__ T slope3(T wl, T wc, T wr) {
     return fast::slope3<LIMITER>(wl, wc, wr);
   }
-  template <int D, typename T>
-  __device__ static __forceinline__ void predictor_dir(const KParams &P, const T w[5], T rinv, const T s[5], T a[5]) {
-    fast::predictor_dir<D>(P, w, rinv, s, a);
+  template <typename T>
+  __device__ static __forceinline__ T mad(T a, T b, T c) {
+    return fm::fma(a, b, c);
+  }
+  template <int LIMITER, typename T>
+  __device__ static __forceinline__ T slope2(T dwl, T dwr) {
+    return fast::slope2<LIMITER>(dwl, dwr);
+  }
+  template <typename T>
+  using Evo = fast::EvoFactors<T>;
+  template <typename T>
+  __device__ static __forceinline__ void evo3d(const fast::EvoFactors<T> &F, const KParams &P, const T w[5], T rinv, const T sx[5],
+                                               const T sy[5], const T sz[5], T ev[5]) {
+    fast::evo3d(F, P, w, rinv, sx, sy, sz, ev);
+  }
+  template <typename T>
+  __device__ static __forceinline__ void evo2d(const fast::EvoFactors<T> &F, const KParams &P, const T w[5], T rinv, const T sx[5],
+                                               const T sy[5], T ev[5]) {
+    fast::evo2d(F, P, w, rinv, sx, sy, ev);
   }
   template <int SOLVER, int DIR, typename T>
   __device__ static __forceinline__ int riemann(const KParams &P, const T wl[5], const T wr[5], T f[6]) {
@@ -154,7 +185,7 @@ struct Phys<false> {
   // temperature p / rho * temp0 (for thermal conduction)
   template <typename T>
   __device__ static __forceinline__ T temp(const KParams &P, const T w[5], T rinv) {
-    return w[4] * rinv * T(P.temp0);
+    return w[4] * rinv * consts(P, T()).temp0;
   }
 };
 
@@ -193,6 +224,37 @@ __device__ __forceinline__ void state(const KParams &P, const double w[5], doubl
 // sqrt(g p / rho) with y the refined reciprocal of rho
 __device__ __forceinline__ double sound(const KParams &P, double rho, double p, double y) {
   return fm::sqrt_pos(fm::div_cr(P.g * p, rho, y));
+}
+// predictor terms (muscl.f90:100-104) and evo (muscl.f90:68,86,106-107); s(5)/rho
+// is the IEEE quotient from the correctly rounded rinv
+template <int D>
+__device__ __forceinline__ void predictor_dir(const KParams &P, const double w[5], double rinv, const double s[5],
+                                              double a[5]) {
+#pragma unroll
+  for (int i = 0; i < 5; i++) a[i] = w[D + 1] * s[i];
+  a[4] = a[4] + P.g * w[4] * s[D + 1];
+  a[D + 1] = a[D + 1] + fm::div_cr(s[4], w[0], rinv);
+}
+struct EvoFactors {
+  double dt2;
+  __device__ EvoFactors(const KParams &, double dt) : dt2(-0.5 * dt) {}
+};
+__device__ __forceinline__ void evo3d(const EvoFactors &F, const KParams &P, const double w[5], double rinv,
+                                      const double sx[5], const double sy[5], const double sz[5], double ev[5]) {
+  double a1[5], a2[5], a3[5];
+  predictor_dir<0>(P, w, rinv, sx, a1);
+  predictor_dir<1>(P, w, rinv, sy, a2);
+  predictor_dir<2>(P, w, rinv, sz, a3);
+#pragma unroll
+  for (int m = 0; m < 5; m++) ev[m] = F.dt2 * (a1[m] * P.dxinv + a2[m] * P.dyinv + a3[m] * P.dzinv);
+}
+__device__ __forceinline__ void evo2d(const EvoFactors &F, const KParams &P, const double w[5], double rinv,
+                                      const double sx[5], const double sy[5], double ev[5]) {
+  double a1[5], a2[5];
+  predictor_dir<0>(P, w, rinv, sx, a1);
+  predictor_dir<1>(P, w, rinv, sy, a2);
+#pragma unroll
+  for (int m = 0; m < 5; m++) ev[m] = F.dt2 * (a1[m] * P.dxinv + a2[m] * P.dyinv);
 }
 template <int DIR>
 __device__ __forceinline__ int hll(const KParams &P, const double wl[5], const double wr[5], double f[6]) {
@@ -276,11 +338,21 @@ struct Phys<true> {
   __device__ static __forceinline__ double slope3(double wl, double wc, double wr) {
     return evh::slope3<LIMITER>(wl, wc, wr);
   }
-  // muscl.f90:100-104: s(5)/rho is the IEEE quotient from rinv
-  template <int D>
-  __device__ static __forceinline__ void predictor_dir(const KParams &P, const double w[5], double rinv,
-                                                       const double s[5], double a[5]) {
-    fast::predictor_dir<D>(P, w, rinv, s, a);
+  __device__ static __forceinline__ double mad(double a, double b, double c) { return a * b + c; }
+  template <int LIMITER>
+  __device__ static __forceinline__ double slope2(double dwl, double dwr) {
+    return evh::limited_slope<LIMITER>(dwl, dwr);
+  }
+  template <typename T>
+  using Evo = exact_bf::EvoFactors;
+  __device__ static __forceinline__ void evo3d(const exact_bf::EvoFactors &F, const KParams &P, const double w[5],
+                                               double rinv, const double sx[5], const double sy[5],
+                                               const double sz[5], double ev[5]) {
+    exact_bf::evo3d(F, P, w, rinv, sx, sy, sz, ev);
+  }
+  __device__ static __forceinline__ void evo2d(const exact_bf::EvoFactors &F, const KParams &P, const double w[5],
+                                               double rinv, const double sx[5], const double sy[5], double ev[5]) {
+    exact_bf::evo2d(F, P, w, rinv, sx, sy, ev);
   }
   template <int SOLVER, int DIR>
   __device__ static __forceinline__ int riemann(const KParams &P, const double wl[5], const double wr[5], double f[6]) {
@@ -306,22 +378,25 @@ struct Phys<true> {
 // in z the prefetch of plane nz + 2 after the last plane (never used; it
 // would fall outside the grid for nz = 2).  A column's offset is fixed for
 // the whole march, so only the plane's is formed per plane.
-__device__ __forceinline__ long long col_offset(const KParams &P, const Geo &G, int gx, int gy) {
+// (An element index below 2^31: a plane of more cells would not leave room for
+// the state in device memory.)
+__device__ __forceinline__ int col_offset(const KParams &P, const Geo &G, int gx, int gy) {
   const bool per = P.boundtype == 2;
   const int cx = gx < -2 ? -2 : (gx > G.nx + 1 ? G.nx + 1 : gx);
   const int cy = gy < -2 ? -2 : (gy > G.ny + 1 ? G.ny + 1 : gy);
-  return (long long)ghost_src(cx, G.nx, per) + (long long)G.nx * ghost_src(cy, G.ny, per);
+  return ghost_src(cx, G.nx, per) + G.nx * ghost_src(cy, G.ny, per);
 }
 __device__ __forceinline__ long long plane_offset(const KParams &P, const Geo &G, int gz) {
   const int cz = gz < -2 ? -2 : (gz > G.nz + 1 ? G.nz + 1 : gz);
   return (long long)G.nx * G.ny * ghost_src(cz, G.nz, P.boundtype == 2);
 }
 
-// raw q of the cell at offset c
+// raw q of the column at offset c of the plane at offset `plane` (the same in
+// all lanes)
 template <typename S>
-__device__ __forceinline__ void fetch_at(const Geo &G, const S *__restrict__ q, long long c, S raw[6]) {
+__device__ __forceinline__ void fetch_at(const Geo &G, const S *__restrict__ q, long long plane, int c, S raw[6]) {
 #pragma unroll
-  for (int m = 0; m < 6; m++) raw[m] = q[m * G.n + c];
+  for (int m = 0; m < 6; m++) raw[m] = (q + (m * G.n + plane))[c];
 }
 
 // raw q of column offset c in plane gz (clamped as plane_offset does).
@@ -332,7 +407,7 @@ __device__ __forceinline__ void fetch_at(const Geo &G, const S *__restrict__ q, 
 // the kernels without the test.
 template <bool SLAB, typename S>
 __device__ __forceinline__ void fetch_plane(const KParams &P, const Geo &G, const S *__restrict__ q, int gz,
-                                            long long c, S raw[6]) {
+                                            int c, S raw[6]) {
   if constexpr (SLAB) {
     const long long pl = (long long)G.nx * G.ny;
     const S *h = nullptr;
@@ -340,41 +415,35 @@ __device__ __forceinline__ void fetch_plane(const KParams &P, const Geo &G, cons
     else if (gz >= G.nz && G.zhi) h = (const S *)G.zhi + pl * (gz > G.nz ? 1 : 0);
     if (h) {
 #pragma unroll
-      for (int m = 0; m < 6; m++) raw[m] = h[m * 2 * pl + c];
+      for (int m = 0; m < 6; m++) raw[m] = (h + m * 2 * pl)[c];
       return;
     }
   }
-  fetch_at(G, q, c + plane_offset(P, G, gz), raw);
+  fetch_at(G, q, plane_offset(P, G, gz), c, raw);
 }
 
-// raw q at (gx, gy, gz), ghost-mapped
-template <bool SLAB, typename S>
-__device__ __forceinline__ void fetch_raw(const KParams &P, const Geo &G, const S *__restrict__ q, int gx, int gy,
-                                          int gz, S raw[6]) {
-  fetch_plane<SLAB>(P, G, q, gz, col_offset(P, G, gx, gy), raw);
+// A copy of v in a register of its own.  Without it the compiler lets the
+// prefetched value and its copy share a register, loads the next plane
+// elsewhere and moves it back at the end of the iteration, which waits for
+// the load (and for the stores before it) there instead of a plane later.
+template <typename S>
+__device__ __forceinline__ S own_copy(S v) {
+  asm("" : "+v"(v));
+  return v;
 }
 
-// primitive of a fetched cell at column gx (for the reflecting wall)
+// primitive of a fetched cell; wall: a ghost column beyond the reflecting
+// upper x (boundary.f90:57-64)
 template <bool EXACT, typename S, typename T>
-__device__ __forceinline__ void prim_cell(const KParams &P, const Geo &G, const S raw[6], int gx, T qc[6], T wc[5],
-                                          T &rinv) {
+__device__ __forceinline__ void prim_cell(const KParams &P, bool wall, const S raw[6], T qc[6], T wc[5], T &rinv) {
 #pragma unroll
-  for (int m = 0; m < 6; m++) qc[m] = T(raw[m]);
+  for (int m = 0; m < 6; m++) qc[m] = T(own_copy(raw[m]));
   Phys<EXACT>::q2w(P, qc, wc, rinv);
-  if (P.boundtype == 3 && gx >= G.nx) {  // reflecting upper x (boundary.f90:57-64)
+  if (wall) {
     wc[1] = -wc[1];
     wc[2] = -wc[2];
     wc[3] = -wc[3];
   }
-}
-
-// load q at (gx, gy, gz) (ghost-mapped) and recover w
-template <bool EXACT, bool SLAB, typename S, typename T>
-__device__ __forceinline__ void load_cell(const KParams &P, const Geo &G, const S *__restrict__ q, int gx, int gy,
-                                          int gz, T qc[6], T wc[5], T &rinv) {
-  S raw[6];
-  fetch_raw<SLAB>(P, G, q, gx, gy, gz, raw);
-  prim_cell<EXACT>(P, G, raw, gx, qc, wc, rinv);
 }
 
 template <typename T, int EA>
@@ -383,14 +452,411 @@ __device__ __forceinline__ void store_w(T (*W)[EA], int slot, const T w[5]) {
   for (int m = 0; m < 5; m++) W[m][slot] = w[m];
 }
 
-// LDS of one block
-template <typename T, int TY>
-struct Smem {
-  T W[5][TileShape<TY>::EA];    // w of plane k, both halo rings
-  T XB[10][TileShape<TY>::NFX]; // x face (fi, j), fi = 0..TX: [0,5) left state, [5,10) right state; then flux
-  T YB[10][TileShape<TY>::NFY]; // y face (i, fj), fj = 0..TY
-  T CR[17][TileShape<TY>::NI];  // per interior column: partial update [0,6), z flux below [6,12), z state below [12,17)
+// ---- the CFL minimum of the new state
+// Most cells cannot set the step's CFL minimum: their fastest signal is
+// slower than one already found.  `slower` tells so without the primitive:
+// with a lower bound thr of the largest signal speed max_d (|u_d| + a) / dx_d
+// found so far in this step, a cell whose |m_d| + a rho < thr dx_d rho in
+// every direction, with (a rho)^2 = g p rho = g g1 (rho E - m^2/2), changes
+// neither the minimum nor the error state (p > 0, by a margin above the
+// rounding of any form; with dual energy also p from E, not from the
+// entropy).  About 16 operations against 50 for the primitive and the limit;
+// thr carries a margin of 5e-6, far above the rounding of this test, so
+// the minimum is the same to the last bit.  false for NaN.
+template <typename T>
+__device__ __forceinline__ bool slower(const KParams &P, const T q[6], T thr) {
+  const auto &C = consts(P, T());
+  const T er = q[4] * q[0];
+  const T m2 = fm::fma(q[3], q[3], fm::fma(q[2], q[2], q[1] * q[1]));
+  const T x = fm::fma(T(-0.5), m2, er);
+  const T a = thr * q[0];
+  const T d = dmin(dmin(fm::fma(a, C.dx, -fm::fabs(q[1])), fm::fma(a, C.dy, -fm::fabs(q[2]))),
+                   fm::fma(a, C.dz, -fm::fabs(q[3])));
+  return x > C.calm * er && d > T(0) && d * d > C.ggm * fm::fma(T(1e-6), er, x);
+}
+
+// the largest of the wave's positive values, as a scalar
+__device__ __forceinline__ float wave_max_pos(float v) {
+  int x = __builtin_bit_cast(int, v);
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false));  // row_shr 1, 2, 4, 8
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false));  // row_bcast 15, 31
+  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false));
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(x, 63));
+}
+
+// The running minimum of one lane, min_c 1 / max_d (|u_d| + a) / dx_d, and
+// the wave's bound for `slower`.  The FP64 fast form keeps -max_d (..) per
+// cell and inverts once per lane; a lane without cells gives 1e6 either way.
+template <typename T, bool EXACT>
+struct CflMin {
+  static constexpr bool kSpeedKey = !EXACT && sizeof(T) == 8;
+  static constexpr float kMargin = 0.999995f;
+  double v = kSpeedKey ? -1e-6 : 1e6;
+  T thr = T(1e-6f * kMargin);
+  __device__ __forceinline__ void add(const KParams &P, const T w[5], T rinv) {
+    if constexpr (kSpeedKey) v = dmin(v, -fast::cfl_speed(P, w, rinv));
+    else v = dmin(v, Phys<EXACT>::cfl_cell(P, w, rinv));
+  }
+  __device__ __forceinline__ void raise() {  // all lanes of the wave
+    const float s = kSpeedKey ? float(-v) : fm::rcp(float(v));
+    const T t = T(wave_max_pos(s) * kMargin);
+    thr = t > thr ? t : thr;
+  }
+  // the wave's minimum, in every lane
+  __device__ __forceinline__ double wave_min() {
+    if constexpr (kSpeedKey) v = fm::rcp(-v);
+    for (int off = 32; off > 0; off >>= 1) v = dmin(v, __shfl_xor(v, off));
+    return v;
+  }
 };
+
+// LDS of one block
+template <typename T, int TX, int TY>
+struct Smem {
+  using TS = TileShape<TX, TY>;
+  T W[5][TS::EA];    // w of plane k, both halo rings
+  T XB[10][TS::NFX]; // x face (fi, j), fi = 0..TX: [0,5) left state, [5,10) right state; then flux
+  T YB[10][TS::NFY]; // y face (i, fj), fj = 0..TY
+  double vmin[TS::NI / 64];  // the interior waves' CFL minima
+};
+
+// the first Riemann error (err, in plane err_k) and the first negative
+// pressure of the new state (nerr, nerr_k) a lane sees; reported once after
+// the march, with the lane's own column (gx, gy)
+struct LaneErrors {
+  int err = 0, err_k = 0, nerr = 0, nerr_k = 0;
+};
+
+// The tile's place: columns from (x0, y0), output planes z0 <= k < z1.
+struct Place {
+  int x0, y0, z0, z1;
+};
+
+// ---- the interior waves of the march: lane tid owns column tid of the tile
+template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, bool EXACT, bool SLAB>
+__device__ __forceinline__ void march_columns(const KParams &P, const Geo &G, const Place &L,
+                                              const S *__restrict__ qin, S *__restrict__ qout, double dt,
+                                              Smem<T, TX, TY> &sm, S *__restrict__ tout, CflMin<T, EXACT> &cfl,
+                                              LaneErrors &er, int tid) {
+  using TS = TileShape<TX, TY>;
+  constexpr int EW = TS::EW;
+  auto &W = sm.W;
+  auto &XB = sm.XB;
+  auto &YB = sm.YB;
+  const int cx = tid % TX, cy = tid / TX;
+  const int gx = L.x0 + cx, gy = L.y0 + cy;
+  const bool inside = gx < G.nx && gy < G.ny;
+  const bool wall = P.boundtype == 3 && gx >= G.nx;
+  const int me = TS::eidx(cx, cy);
+  const int fxl = cx + (TX + 1) * cy, fyb = cx + TX * cy;  // the left x face and the bottom y face
+  const int z0 = L.z0, z1 = L.z1;
+
+  const typename Phys<EXACT>::template Evo<T> evof(P, dt);
+  const T dtx = uniform(T(dt * P.dxinv)), dty = uniform(T(dt * P.dyinv)), dtz = uniform(T(dt * P.dzinv));
+
+  // w of planes k and k+1 and (wm) of plane k-1 or, where the limiter takes
+  // one-sided differences only, its difference from plane k; qc, qn: the (dual-energy corrected) q of planes
+  // k and k+1, the base of the update, kept in registers so that q is read
+  // from HBM once; pre: the raw q of the plane after, loaded one plane ahead,
+  // so that no wave stalls on memory right after issuing a load
+  T wm[5], wc[5], wp[5], qc[6], qn[6];
+  T rc, rp;
+  S pre[6];
+  const int own_xy = col_offset(P, G, gx, gy);
+  {
+    S ra[6], rb[6];  // all three planes in flight together
+    fetch_plane<SLAB>(P, G, qin, z0 - 2, own_xy, ra);
+    fetch_plane<SLAB>(P, G, qin, z0 - 1, own_xy, rb);
+    fetch_plane<SLAB>(P, G, qin, z0, own_xy, pre);
+    prim_cell<EXACT>(P, wall, ra, qn, wm, rc);
+    prim_cell<EXACT>(P, wall, rb, qn, wc, rc);
+  }
+  constexpr bool kDiff = LIMITER != 2;
+  if constexpr (kDiff) {
+#pragma unroll
+    for (int m = 0; m < 5; m++) wm[m] = wc[m] - wm[m];
+  }
+#pragma unroll
+  for (int m = 0; m < 6; m++) qc[m] = T(0);
+  // carried from plane k-1: its partial update, the flux of its bottom z
+  // face and its top z state
+  T part[6], fzb[6], zrp[5];
+#pragma unroll
+  for (int m = 0; m < 6; m++) { part[m] = T(0); fzb[m] = T(0); }
+#pragma unroll
+  for (int m = 0; m < 5; m++) zrp[m] = T(0);
+
+  for (int k = z0 - 1; k <= z1; k++) {
+    const bool out_plane = k >= z0 && k < z1;
+    // ---- S1: w of plane k to LDS
+    store_w(W, me, wc);
+    __syncthreads();
+
+    // ---- S2: primitive of plane k+1; slopes, predictor and face states of
+    // plane k
+    prim_cell<EXACT>(P, wall, pre, qn, wp, rp);
+    fetch_plane<SLAB>(P, G, qin, k + 2, own_xy, pre);
+    T sx[5], sy[5], sz[5], ev[5];
+#pragma unroll
+    for (int m = 0; m < 5; m++) {
+      sx[m] = Phys<EXACT>::template slope3<LIMITER>(W[m][me - 1], wc[m], W[m][me + 1]);
+      sy[m] = Phys<EXACT>::template slope3<LIMITER>(W[m][me - EW], wc[m], W[m][me + EW]);
+      if constexpr (kDiff) {
+        const T dz = wp[m] - wc[m];
+        sz[m] = Phys<EXACT>::template slope2<LIMITER>(wm[m], dz);
+        wm[m] = dz;
+      } else {
+        sz[m] = Phys<EXACT>::template slope3<LIMITER>(wm[m], wc[m], wp[m]);
+        wm[m] = wc[m];
+      }
+    }
+    if (P.secondorder) {
+      Phys<EXACT>::evo3d(evof, P, wc, rc, sx, sy, sz, ev);
+    } else {
+#pragma unroll
+      for (int m = 0; m < 5; m++) { ev[m] = T(0); sx[m] = T(0); sy[m] = T(0); sz[m] = T(0); }
+    }
+    {
+      T zl[5], zr[5];
+#pragma unroll
+      for (int m = 0; m < 5; m++) {
+        XB[5 + m][fxl] = fast::face_state(wc[m], T(-0.5), sx[m], ev[m]);   // right state of the left face
+        XB[m][fxl + 1] = fast::face_state(wc[m], T(0.5), sx[m], ev[m]);   // left state of the right face
+        YB[5 + m][fyb] = fast::face_state(wc[m], T(-0.5), sy[m], ev[m]);
+        YB[m][fyb + TX] = fast::face_state(wc[m], T(0.5), sy[m], ev[m]);
+        zl[m] = fast::face_state(wc[m], T(-0.5), sz[m], ev[m]);
+        zr[m] = fast::face_state(wc[m], T(0.5), sz[m], ev[m]);
+      }
+      // z face k-1/2 and the end of plane k-1; the scheduling barrier keeps
+      // this solve apart from the x/y solves
+      __builtin_amdgcn_sched_barrier(0);
+      if (k >= z0) {
+        T fz[6];
+        const int e = Phys<EXACT>::template riemann<SOLVER, 3>(P, zrp, zl, fz);
+        if (e && inside && !er.err) { er.err = e; er.err_k = k; }
+        if (k - 1 >= z0) {
+          T o[6];
+#pragma unroll
+          for (int m = 0; m < 6; m++) o[m] = Phys<EXACT>::mad(dtz, fzb[m] - fz[m], part[m]);
+          const long long op = (long long)G.nx * G.ny * (k - 1);  // the plane; own_xy is the cell's place in it
+          if (inside) {
+#pragma unroll
+            for (int m = 0; m < 6; m++) (qout + (m * G.n + op))[own_xy] = S(o[m]);
+          }
+          // the limits of the new state, for the cells that can change them
+          const bool need = inside && (tout || !slower(P, o, cfl.thr));
+          if (__builtin_amdgcn_ballot_w64(need)) {
+            if (need) {
+              T wn[5], rn;
+              const int ep = Phys<EXACT>::q2w(P, o, wn, rn);
+              if (ep && !er.nerr) { er.nerr = ep; er.nerr_k = k - 1; }
+              cfl.add(P, wn, rn);
+              if (tout) (tout + op)[own_xy] = S(Phys<EXACT>::temp(P, wn, rn));
+            }
+            if (!tout) cfl.raise();
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < 6; m++) fzb[m] = fz[m];
+      }
+#pragma unroll
+      for (int m = 0; m < 5; m++) zrp[m] = zr[m];
+    }
+    __syncthreads();
+
+    // ---- S3: the left x face and the bottom y face of plane k, as one
+    // straight-line block so that the two solves interleave
+    if (out_plane) {
+      T xl[5], xr[5], fx[6], yl[5], yr[5], fy[6];
+#pragma unroll
+      for (int m = 0; m < 5; m++) {
+        xl[m] = XB[m][fxl];
+        xr[m] = XB[5 + m][fxl];
+        yl[m] = YB[m][fyb];
+        yr[m] = YB[5 + m][fyb];
+      }
+      const int ex = Phys<EXACT>::template riemann<SOLVER, 1>(P, xl, xr, fx);
+      const int ey = Phys<EXACT>::template riemann<SOLVER, 2>(P, yl, yr, fy);
+      // faces of cells outside the box (partial tiles) do not count
+      const int e = (gy < G.ny && gx <= G.nx && ex) ? ex : ((gx < G.nx && gy <= G.ny) ? ey : 0);
+      const bool take = e && !er.err;
+      er.err = take ? e : er.err;
+      er.err_k = take ? k : er.err_k;
+#pragma unroll
+      for (int m = 0; m < 6; m++) {
+        XB[m][fxl] = fx[m];
+        YB[m][fyb] = fy[m];
+      }
+    }
+    __syncthreads();
+
+    // ---- S4: x/y differences of plane k
+    if (out_plane) {
+#pragma unroll
+      for (int m = 0; m < 6; m++) part[m] = Phys<EXACT>::mad(dtx, XB[m][fxl] - XB[m][fxl + 1], qc[m]);
+#pragma unroll
+      for (int m = 0; m < 6; m++) part[m] = Phys<EXACT>::mad(dty, YB[m][fyb] - YB[m][fyb + TX], part[m]);
+    }
+    // rotate the column window
+#pragma unroll
+    for (int m = 0; m < 5; m++) wc[m] = wp[m];
+    rc = rp;
+#pragma unroll
+    for (int m = 0; m < 6; m++) qc[m] = qn[m];
+  }
+}
+
+// ---- the ring wave of the march: lane `lane` owns first-ring columns (or
+// corners) lane, lane + 64, ... and the second-ring cell beyond each.  The
+// same barriers as march_columns.
+template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, bool EXACT, bool SLAB>
+__device__ __forceinline__ void march_ring(const KParams &P, const Geo &G, const Place &L, const S *__restrict__ qin,
+                                           double dt, Smem<T, TX, TY> &sm, LaneErrors &er, int lane) {
+  using TS = TileShape<TX, TY>;
+  constexpr int EW = TS::EW, NP = TS::NP;
+  auto &W = sm.W;
+  const int z0 = L.z0, z1 = L.z1;
+  const typename Phys<EXACT>::template Evo<T> evof(P, dt);
+
+  // per column: the state's place (the face it belongs to), the slots of its
+  // w and of its second-ring cell, its q offsets
+  bool owns[NP], second[NP], wall[NP], wall2[NP], isx[NP];
+  T half[NP], *out[NP];
+  int ostride[NP], me[NP], slot2[NP];
+  int own_xy[NP], r2_xy[NP];
+  T wm[NP][5], wc[NP][5], wp[NP][5], rc[NP], rp[NP], rw2[NP][5], tq[6], tr;
+  S pre[NP][6], pre2[NP][6];
+#pragma unroll
+  for (int p = 0; p < NP; p++) {
+    const int c = lane + 64 * p;
+    int cx, cy, r2x, r2y;
+    owns[p] = c < TS::NR1;
+    second[p] = c < TS::NR1 + 4;
+    isx[p] = c < 2 * TY;
+    half[p] = T(0.5);
+    if (c < TY) {  // left of the tile: the left state of the left-edge faces
+      cx = -1; cy = c; r2x = -2; r2y = c;
+      out[p] = &sm.XB[0][(TX + 1) * cy];
+    } else if (c < 2 * TY) {  // right: the right state of the right-edge faces
+      cx = TX; cy = c - TY; r2x = TX + 1; r2y = cy;
+      out[p] = &sm.XB[5][TX + (TX + 1) * cy];
+      half[p] = T(-0.5);
+    } else if (c < 2 * TY + TX) {  // below
+      cx = c - 2 * TY; cy = -1; r2x = cx; r2y = -2;
+      out[p] = &sm.YB[0][cx];
+    } else if (c < TS::NR1) {  // above
+      cx = c - 2 * TY - TX; cy = TY; r2x = cx; r2y = TY + 1;
+      out[p] = &sm.YB[5][cx + TX * TY];
+      half[p] = T(-0.5);
+    } else {  // the four corners of the first ring; lanes without a job load one too
+      cx = (c & 1) ? TX : -1;
+      cy = (c & 2) ? TY : -1;
+      r2x = cx;
+      r2y = cy;
+      out[p] = &sm.XB[0][0];
+    }
+    ostride[p] = isx[p] ? TS::NFX : TS::NFY;
+    me[p] = TS::eidx(cx, cy);
+    slot2[p] = TS::eidx(r2x, r2y);
+    own_xy[p] = col_offset(P, G, L.x0 + cx, L.y0 + cy);
+    r2_xy[p] = col_offset(P, G, L.x0 + r2x, L.y0 + r2y);
+    wall[p] = P.boundtype == 3 && L.x0 + cx >= G.nx;
+    wall2[p] = P.boundtype == 3 && L.x0 + r2x >= G.nx;
+    S ra[6], rb[6], rd[6], r2[6];
+    fetch_plane<SLAB>(P, G, qin, z0 - 2, own_xy[p], ra);
+    fetch_plane<SLAB>(P, G, qin, z0 - 1, own_xy[p], rb);
+    fetch_plane<SLAB>(P, G, qin, z0 - 1, r2_xy[p], r2);
+    fetch_plane<SLAB>(P, G, qin, z0, own_xy[p], rd);
+    fetch_plane<SLAB>(P, G, qin, z0, r2_xy[p], pre2[p]);
+    fetch_plane<SLAB>(P, G, qin, z0 + 1, own_xy[p], pre[p]);
+    prim_cell<EXACT>(P, wall[p], ra, tq, wm[p], tr);
+    prim_cell<EXACT>(P, wall[p], rb, tq, wc[p], rc[p]);
+    prim_cell<EXACT>(P, wall2[p], r2, tq, rw2[p], tr);
+    prim_cell<EXACT>(P, wall[p], rd, tq, wp[p], rp[p]);
+  }
+
+  for (int k = z0 - 1; k <= z1; k++) {
+    const bool out_plane = k >= z0 && k < z1;
+    // ---- S1
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      if (owns[p]) store_w(W, me[p], wc[p]);
+      if (second[p]) store_w(W, slot2[p], rw2[p]);
+    }
+    __syncthreads();
+
+    // ---- S2: the face state of each column
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      if (owns[p]) {
+        T sx[5], sy[5], sz[5], ev[5];
+        const int i = me[p];
+#pragma unroll
+        for (int m = 0; m < 5; m++) {
+          sx[m] = Phys<EXACT>::template slope3<LIMITER>(W[m][i - 1], wc[p][m], W[m][i + 1]);
+          sy[m] = Phys<EXACT>::template slope3<LIMITER>(W[m][i - EW], wc[p][m], W[m][i + EW]);
+          sz[m] = Phys<EXACT>::template slope3<LIMITER>(wm[p][m], wc[p][m], wp[p][m]);
+        }
+        if (P.secondorder) {
+          Phys<EXACT>::evo3d(evof, P, wc[p], rc[p], sx, sy, sz, ev);
+        } else {
+#pragma unroll
+          for (int m = 0; m < 5; m++) { ev[m] = T(0); sx[m] = T(0); sy[m] = T(0); }
+        }
+#pragma unroll
+        for (int m = 0; m < 5; m++) out[p][m * ostride[p]] = fast::face_state(wc[p][m], half[p], isx[p] ? sx[m] : sy[m], ev[m]);
+      }
+      // the second ring's w of plane k+1
+      prim_cell<EXACT>(P, wall2[p], pre2[p], tq, rw2[p], tr);
+      fetch_plane<SLAB>(P, G, qin, k + 2, r2_xy[p], pre2[p]);
+    }
+    __syncthreads();
+
+    // ---- S3: the TY right-edge x faces (lanes 0..TY-1) and the TX top-edge
+    // y faces (lanes TY..TY+TX-1) in one solve, so that the wave does not run
+    // two: a y face is the x face of the states with u and v exchanged.  The
+    // solvers are bit-symmetric under that exchange: |u|^2 is formed
+    // symmetrically and every other term by its role.
+    if (out_plane && lane < TY + TX) {
+      const bool isy = lane >= TY;
+      T *fb = isy ? &sm.YB[0][(lane - TY) + TX * TY] : &sm.XB[0][TX + (TX + 1) * lane];
+      const int st_ = isy ? TS::NFY : TS::NFX;
+      T wl[5], wr[5], f[6];
+#pragma unroll
+      for (int m = 0; m < 5; m++) { wl[m] = fb[m * st_]; wr[m] = fb[(5 + m) * st_]; }
+      const T l1 = wl[1], r1 = wr[1];
+      wl[1] = isy ? wl[2] : wl[1];
+      wl[2] = isy ? l1 : wl[2];
+      wr[1] = isy ? wr[2] : wr[1];
+      wr[2] = isy ? r1 : wr[2];
+      const int e = Phys<EXACT>::template riemann<SOLVER, 1>(P, wl, wr, f);
+      const T f1 = f[1];
+      f[1] = isy ? f[2] : f[1];
+      f[2] = isy ? f1 : f[2];
+      const bool counts = isy ? (L.x0 + lane - TY < G.nx && L.y0 + TY <= G.ny)
+                              : (L.x0 + TX <= G.nx && L.y0 + lane < G.ny);
+      if (e && !er.err && counts) { er.err = e; er.err_k = k; }
+#pragma unroll
+      for (int m = 0; m < 6; m++) fb[m * st_] = f[m];
+    }
+    // rotate the column windows and form the primitive of plane k+2 here, where
+    // the interior waves run two solves: S1 comes between two barriers, and
+    // the ring wave's primitives there made every wave wait (512^3 FP64: 6.19
+    // against 5.54 ms with the second ring's in S1 too)
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+#pragma unroll
+      for (int m = 0; m < 5; m++) { wm[p][m] = wc[p][m]; wc[p][m] = wp[p][m]; }
+      rc[p] = rp[p];
+      prim_cell<EXACT>(P, wall[p], pre[p], tq, wp[p], rp[p]);
+      fetch_plane<SLAB>(P, G, qin, k + 3, own_xy[p], pre[p]);
+    }
+    __syncthreads();
+  }
+}
 
 // One tile `lin` (x fastest, then y, then z chunk) of the box whose q starts
 // at element qoff of qin_all/qout_all.  vmin_dst receives the CFL minimum of
@@ -398,292 +864,58 @@ struct Smem {
 // With tout (single box only), the temperature of each new cell is stored
 // there too, for the conduction pass that follows the sweep.  SLAB: the grid
 // is a z-slab whose ghost planes may come from halo buffers (Geo::zlo, zhi).
-template <typename T, typename S, int SOLVER, int LIMITER, int TY, bool EXACT, bool SLAB = false>
-__device__ __forceinline__ void march(const KParams P, const Geo G, const S *__restrict__ qin_all,
+// The two roles run loops of their own, so that neither holds the other's
+// values in registers.
+template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, bool EXACT, bool SLAB = false>
+__device__ __forceinline__ void march(const KParams &P, const Geo &G, const S *__restrict__ qin_all,
                                       S *__restrict__ qout_all, long long qoff, int box, double dt, Status *st,
-                                      unsigned long long *vmin_dst, int lin, Smem<T, TY> &sm,
+                                      unsigned long long *vmin_dst, int lin, Smem<T, TX, TY> &sm,
                                       S *__restrict__ tout = nullptr) {
-  using TS = TileShape<TY>;
-  constexpr int NI = TS::NI, NR1 = TS::NR1, EW = TS::EW, EA = TS::EA;
-  T(&W)[5][EA] = sm.W;
-  T(&XB)[10][TS::NFX] = sm.XB;
-  T(&YB)[10][TS::NFY] = sm.YB;
-  T(&CR)[17][NI] = sm.CR;
-  const int tid = threadIdx.x;
-  const bool ring = tid >= NI;
+  using TS = TileShape<TX, TY>;
+  constexpr int NI = TS::NI;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int tid = (int)(threadIdx.x & 63) + 64 * wave;
   const int tile = lin % (G.tiles_x * G.tiles_y);
   const int chunk = lin / (G.tiles_x * G.tiles_y);
-  const int x0 = (tile % G.tiles_x) * TX, y0 = (tile / G.tiles_x) * TY;
-  const int z0 = chunk * G.zchunk;
-  const int z1 = min(z0 + G.zchunk, G.nz);
+  Place L;
+  L.x0 = (tile % G.tiles_x) * TX;
+  L.y0 = (tile / G.tiles_x) * TY;
+  L.z0 = chunk * G.zchunk;
+  L.z1 = min(L.z0 + G.zchunk, G.nz);
   const S *__restrict__ qin = qin_all + qoff;
   S *__restrict__ qout = qout_all + qoff;
-  const unsigned long long tag = (unsigned long long)box << 40;  // box index above the cell index
 
-  // owned column (interior cell, or first-ring cell for the ring wave); the
-  // ring wave also loads one second-ring cell or first-ring corner per lane
-  int cx, cy, side = -1, r2x = 0, r2y = 0;
-  const int lane = tid - NI;
-  if (!ring) {
-    cx = tid % TX;
-    cy = tid / TX;
-  } else if (lane < TY) {
-    side = 0; cx = -1; cy = lane; r2x = -2; r2y = lane;
-  } else if (lane < 2 * TY) {
-    side = 1; cx = TX; cy = lane - TY; r2x = TX + 1; r2y = cy;
-  } else if (lane < 2 * TY + TX) {
-    side = 2; cx = lane - 2 * TY; cy = -1; r2x = cx; r2y = -2;
-  } else if (lane < NR1) {
-    side = 3; cx = lane - 2 * TY - TX; cy = TY; r2x = cx; r2y = TY + 1;
-  } else {  // lanes NR1..NR1+3 load the first-ring corners, the rest idle
-    const int c = lane - NR1;
-    cx = (c & 1) ? TX : -1;
-    cy = (c & 2) ? TY : -1;
-    r2x = cx;
-    r2y = cy;
-    if (c >= 4) r2x = -3;  // no second-ring job
+  LaneErrors er;
+  int gx, gy;  // the lane's own column, which locates its errors
+  if (wave < NI / 64) {
+    CflMin<T, EXACT> cfl;
+    march_columns<T, S, SOLVER, LIMITER, TX, TY, EXACT, SLAB>(P, G, L, qin, qout, dt, sm, tout, cfl, er, tid);
+    const double v = cfl.wave_min();
+    if ((tid & 63) == 0) sm.vmin[wave] = v;
+    gx = L.x0 + tid % TX;
+    gy = L.y0 + tid / TX;
+  } else {
+    const int lane = tid - NI;
+    march_ring<T, S, SOLVER, LIMITER, TX, TY, EXACT, SLAB>(P, G, L, qin, dt, sm, er, lane);
+    // its last faces are the right-edge x faces, then the top-edge y faces
+    gx = L.x0 + (lane < TY ? TX : lane - TY);
+    gy = L.y0 + (lane < TY ? lane : TY);
   }
-  const bool owns_col = !ring || side >= 0;
-  const int gx = x0 + cx, gy = y0 + cy;
-  const bool inside = !ring && gx < G.nx && gy < G.ny;
-  const int me = eidx<TY>(cx, cy);
-
-  const T dt2 = T(-0.5 * dt);
-  const T dtx = T(dt * P.dxinv), dty = T(dt * P.dyinv), dtz = T(dt * P.dzinv);
-  const T half = T(0.5);
-
-  // qc, qn: the (dual-energy corrected) q of planes k and k+1, the base of
-  // the update, kept in registers so that q is read from HBM once
-  T wm[5], wc[5], wp[5], qn[6], qc[6], tq[6];
-  T rm, rc, rp;
-  // The CFL minimum min_c 1 / max_d (|u_d| + a) / dx_d.  The FP64 fast
-  // form reduces -max_d (..) per cell and inverts once per lane; a lane
-  // without cells gives 1e6 either way.
-  constexpr bool kSpeedKey = !EXACT && sizeof(T) == 8;
-  double vmin = kSpeedKey ? -1e-6 : 1e6;
-  // first Riemann error and first negative pressure of the new state seen by
-  // this lane (code, plane); reported once after the march
-  int err = 0, err_k = 0, nerr = 0, nerr_k = 0;
-  // q^{n+1} of plane k-1, stored in S2; its primitive, CFL limit and
-  // temperature are formed after the x/y solves (S4), where the interior
-  // waves would otherwise wait for the ring wave
-  T o[6];
-  bool pend = false;
-  long long oc = 0;
-
-  // global loads run one plane ahead: pre holds the raw q of this column's
-  // next plane and pre2 the ring wave's second-ring cell, so that no wave
-  // stalls on memory right after issuing a load
-  S pre[6], pre2[6];
-  const long long own_xy = col_offset(P, G, gx, gy);
-  const long long r2_xy = col_offset(P, G, x0 + r2x, y0 + r2y);
-  // the ring wave's second-ring cell: its w of the current plane (rw2) is
-  // formed one plane ahead, in the ring wave's idle time of S2
-  T rw2[5];
+  // one atomic per block: the waves of all blocks meet at one address
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double v = sm.vmin[0];
 #pragma unroll
-  for (int m = 0; m < 6; m++) { qc[m] = T(0); qn[m] = T(0); }
-  load_cell<EXACT, SLAB, S, T>(P, G, qin, gx, gy, z0 - 2, tq, wm, rm);
-  load_cell<EXACT, SLAB, S, T>(P, G, qin, gx, gy, z0 - 1, tq, wc, rc);
-  fetch_plane<SLAB>(P, G, qin, z0, own_xy, pre);
-  {
-    T rr2;
-    fetch_plane<SLAB>(P, G, qin, z0 - 1, r2_xy, pre2);
-    prim_cell<EXACT>(P, G, pre2, x0 + r2x, tq, rw2, rr2);
-    fetch_plane<SLAB>(P, G, qin, z0, r2_xy, pre2);
+    for (int i = 1; i < NI / 64; i++) v = dmin(v, sm.vmin[i]);
+    atomic_min_pos(vmin_dst, v);
   }
-
-  for (int k = z0 - 1; k <= z1; k++) {
-    const bool out_plane = k >= z0 && k < z1;
-    // ---- S1: primitive of plane k+1 (own column); rings of plane k to LDS.
-    // Every lane forms and fetches (the ring wave's corner and idle lanes on
-    // clamped coordinates), so that no branch makes a load wait for the
-    // fetches issued after it.
-    prim_cell<EXACT>(P, G, pre, gx, qn, wp, rp);
-    fetch_plane<SLAB>(P, G, qin, k + 2, own_xy, pre);
-    if (ring && r2x > -3) store_w<T, EA>(W, eidx<TY>(r2x, r2y), rw2);
-    if (owns_col) store_w<T, EA>(W, me, wc);
-    __syncthreads();
-
-    // ---- S2: slopes, predictor and face states of plane k
-    T sx[5], sy[5], sz[5], ev[5];
-    if (owns_col) {
-#pragma unroll
-    for (int m = 0; m < 5; m++) {
-      sx[m] = Phys<EXACT>::template slope3<LIMITER>(W[m][me - 1], wc[m], W[m][me + 1]);
-      sy[m] = Phys<EXACT>::template slope3<LIMITER>(W[m][me - EW], wc[m], W[m][me + EW]);
-      sz[m] = Phys<EXACT>::template slope3<LIMITER>(wm[m], wc[m], wp[m]);
-    }
-    if (P.secondorder) {
-      T a1[5], a2[5], a3[5];
-      Phys<EXACT>::template predictor_dir<0>(P, wc, rc, sx, a1);
-      Phys<EXACT>::template predictor_dir<1>(P, wc, rc, sy, a2);
-      Phys<EXACT>::template predictor_dir<2>(P, wc, rc, sz, a3);
-      fast::evo5(P, dt2, a1, a2, a3, ev);  // muscl.f90:106-107
-    } else {
-#pragma unroll
-      for (int m = 0; m < 5; m++) { ev[m] = T(0); sx[m] = T(0); sy[m] = T(0); sz[m] = T(0); }
-    }
-    // face states (muscl.f90:207-210) in the reference's order:
-    // (w + 0.5 s) + evo on the high side, (w - 0.5 s) + evo on the low side
-    if (!ring) {
-      const int fxl = cx + (TX + 1) * cy, fyb = cx + TX * cy;
-#pragma unroll
-      for (int m = 0; m < 5; m++) {
-        XB[5 + m][fxl] = fm::fmad(-half, sx[m], wc[m]) + ev[m];       // right state of the left face
-        XB[m][fxl + 1] = fm::fmad(half, sx[m], wc[m]) + ev[m];       // left state of the right face
-        YB[5 + m][fyb] = fm::fmad(-half, sy[m], wc[m]) + ev[m];
-        YB[m][fyb + TX] = fm::fmad(half, sy[m], wc[m]) + ev[m];
-      }
-    } else if (side == 0) {
-#pragma unroll
-      for (int m = 0; m < 5; m++) XB[m][(TX + 1) * cy] = fm::fmad(half, sx[m], wc[m]) + ev[m];
-    } else if (side == 1) {
-#pragma unroll
-      for (int m = 0; m < 5; m++) XB[5 + m][TX + (TX + 1) * cy] = fm::fmad(-half, sx[m], wc[m]) + ev[m];
-    } else if (side == 2) {
-#pragma unroll
-      for (int m = 0; m < 5; m++) YB[m][cx] = fm::fmad(half, sy[m], wc[m]) + ev[m];
-    } else {
-#pragma unroll
-      for (int m = 0; m < 5; m++) YB[5 + m][cx + TX * TY] = fm::fmad(-half, sy[m], wc[m]) + ev[m];
-    }
-    // z face k-1/2 (interior lanes) and the end of plane k-1; the
-    // scheduling barrier keeps this solve apart from the x/y solves
-    __builtin_amdgcn_sched_barrier(0);
-    if (!ring) {
-      T zl[5], zr[5];
-#pragma unroll
-      for (int m = 0; m < 5; m++) {
-        zl[m] = fm::fmad(-half, sz[m], wc[m]) + ev[m];
-        zr[m] = fm::fmad(half, sz[m], wc[m]) + ev[m];
-      }
-      if (k >= z0) {
-        T zrp[5], fz[6];
-#pragma unroll
-        for (int m = 0; m < 5; m++) zrp[m] = CR[12 + m][tid];
-        const int e = Phys<EXACT>::template riemann<SOLVER, 3>(P, zrp, zl, fz);
-        if (e && inside && !err) { err = e; err_k = k; }
-        if (k - 1 >= z0 && inside) {
-#pragma unroll
-          for (int m = 0; m < 6; m++) o[m] = fm::fmad(dtz, CR[6 + m][tid] - fz[m], CR[m][tid]);
-          oc = (long long)gx + (long long)G.nx * ((long long)gy + (long long)G.ny * (k - 1));
-#pragma unroll
-          for (int m = 0; m < 6; m++) qout[m * G.n + oc] = S(o[m]);
-          pend = true;
-        }
-#pragma unroll
-        for (int m = 0; m < 6; m++) CR[6 + m][tid] = fz[m];
-      }
-#pragma unroll
-      for (int m = 0; m < 5; m++) CR[12 + m][tid] = zr[m];
-    }
-    }  // owns_col
-    if (ring) {  // second-ring w of plane k+1, stored in S1 of plane k+1
-      T rr2;
-      prim_cell<EXACT>(P, G, pre2, x0 + r2x, tq, rw2, rr2);
-      fetch_plane<SLAB>(P, G, qin, k + 2, r2_xy, pre2);
-    }
-    __syncthreads();
-
-    // ---- S3: x and y faces of plane k
-    if (out_plane) {
-      if (!ring) {
-        // interior lane (i,j): its left x face and bottom y face, as one
-        // straight-line block so that the two solves interleave
-        const int fxi = cx + (TX + 1) * cy, fyi = cx + TX * cy;
-        T xl[5], xr[5], fx[6], yl[5], yr[5], fy[6];
-#pragma unroll
-        for (int m = 0; m < 5; m++) {
-          xl[m] = XB[m][fxi];
-          xr[m] = XB[5 + m][fxi];
-          yl[m] = YB[m][fyi];
-          yr[m] = YB[5 + m][fyi];
-        }
-        const int ex = Phys<EXACT>::template riemann<SOLVER, 1>(P, xl, xr, fx);
-        const int ey = Phys<EXACT>::template riemann<SOLVER, 2>(P, yl, yr, fy);
-        // faces of cells outside the box (partial tiles) do not count
-        const int e = (gy < G.ny && gx <= G.nx && ex) ? ex : ((gx < G.nx && gy <= G.ny) ? ey : 0);
-        const bool take = e && !err;
-        err = take ? e : err;
-        err_k = take ? k : err_k;
-#pragma unroll
-        for (int m = 0; m < 6; m++) {
-          XB[m][fxi] = fx[m];
-          YB[m][fyi] = fy[m];
-        }
-      } else {
-        // ring wave: the TY right-edge x faces (lanes 0..TY-1) and the 16
-        // top-edge y faces (lanes TY..TY+15) in one solve, so that the wave
-        // does not run two: a y face is the x face of the states with u and
-        // v exchanged.  The solvers are bit-symmetric under that exchange:
-        // |u|^2 is formed symmetrically and every other term by its role
-        // (the FP32 build has no contraction).
-        if (lane < TY + TX) {
-          const bool isy = lane >= TY;
-          T *fb = isy ? &YB[0][(lane - TY) + TX * TY] : &XB[0][TX + (TX + 1) * lane];
-          const int st_ = isy ? TS::NFY : TS::NFX;
-          T wl[5], wr[5], f[6];
-#pragma unroll
-          for (int m = 0; m < 5; m++) { wl[m] = fb[m * st_]; wr[m] = fb[(5 + m) * st_]; }
-          const T l1 = wl[1], r1 = wr[1];
-          wl[1] = isy ? wl[2] : wl[1];
-          wl[2] = isy ? l1 : wl[2];
-          wr[1] = isy ? wr[2] : wr[1];
-          wr[2] = isy ? r1 : wr[2];
-          const int e = Phys<EXACT>::template riemann<SOLVER, 1>(P, wl, wr, f);
-          const T f1 = f[1];
-          f[1] = isy ? f[2] : f[1];
-          f[2] = isy ? f1 : f[2];
-          const bool counts = isy ? (x0 + lane - TY < G.nx && y0 + TY <= G.ny) : (x0 + TX <= G.nx && y0 + lane < G.ny);
-          if (e && !err && counts) { err = e; err_k = k; }
-#pragma unroll
-          for (int m = 0; m < 6; m++) fb[m * st_] = f[m];
-        }
-      }
-    }
-    __syncthreads();
-
-    // ---- S4: x/y differences of plane k
-    if (!ring && out_plane) {
-      const int fxl = cx + (TX + 1) * cy, fyb = cx + TX * cy;
-      T part[6];
-#pragma unroll
-      for (int m = 0; m < 6; m++) part[m] = fm::fmad(dtx, XB[m][fxl] - XB[m][fxl + 1], qc[m]);
-#pragma unroll
-      for (int m = 0; m < 6; m++) CR[m][tid] = fm::fmad(dty, YB[m][fyb] - YB[m][fyb + TX], part[m]);
-    }
-    // the end of plane k-1: primitive of the new state for the CFL minimum
-    // of the next step, its first negative pressure, its temperature
-    if (pend) {
-      T on[6], wn[5], rn;
-#pragma unroll
-      for (int m = 0; m < 6; m++) on[m] = T(S(o[m]));
-      const int ep = Phys<EXACT>::q2w(P, on, wn, rn);
-      if (ep && !nerr) { nerr = ep; nerr_k = k - 1; }
-      if constexpr (kSpeedKey) vmin = dmin(vmin, -fast::cfl_speed(P, wn, rn));
-      else vmin = dmin(vmin, Phys<EXACT>::cfl_cell(P, wn, rn));
-      if (tout) tout[oc] = S(Phys<EXACT>::temp(P, wn, rn));
-      pend = false;
-    }
-    // rotate the column window
-#pragma unroll
-    for (int m = 0; m < 5; m++) { wm[m] = wc[m]; wc[m] = wp[m]; }
-    rm = rc;
-    rc = rp;
-#pragma unroll
-    for (int m = 0; m < 6; m++) qc[m] = qn[m];
-  }
-
-  if (err || nerr) {  // the lane's own column (clamped into the box) locates the error
+  if (er.err || er.nerr) {  // clamped into the box
+    const unsigned long long tag = (unsigned long long)box << 40;  // box index above the cell index
     const long long ex = min(max(gx, 0), G.nx - 1), ey = min(max(gy, 0), G.ny - 1);
-    if (err) report(st, err, tag | (unsigned long long)(ex + G.nx * (ey + (long long)G.ny * err_k)));
-    if (nerr) report_next(st, nerr, tag | (unsigned long long)(ex + G.nx * (ey + (long long)G.ny * nerr_k)));
+    if (er.err) report(st, er.err, tag | (unsigned long long)(ex + G.nx * (ey + (long long)G.ny * er.err_k)));
+    if (er.nerr) report_next(st, er.nerr, tag | (unsigned long long)(ex + G.nx * (ey + (long long)G.ny * er.nerr_k)));
   }
-  if constexpr (kSpeedKey) vmin = fm::rcp(-vmin);
-  for (int off = 32; off > 0; off >>= 1) vmin = dmin(vmin, __shfl_xor(vmin, off));
-  if ((tid & 63) == 0) atomic_min_pos(vmin_dst, vmin);
 }
-
 
 }  // namespace core
 }  // namespace evh

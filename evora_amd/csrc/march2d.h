@@ -101,9 +101,8 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
   const bool face = l >= 1 && l < NL - 2;       // solves the face (l, l+1)
   const bool face_counts = gx >= -1 && gx < G.nx;  // that face is one the reference solves
 
-  const T dt2 = T(-0.5 * dt);
-  const T dtx = T(dt * P.dxinv), dty = T(dt * P.dyinv);
-  const T half = T(0.5);
+  const typename Ph::template Evo<T> evof(P, dt);
+  const T dtx = uniform(T(dt * P.dxinv)), dty = uniform(T(dt * P.dyinv));
 
   // rows k-1, k, k+1 of the column; qc, qn: q of rows k and k+1 (the base of
   // the update, kept in registers so that q is read from HBM once)
@@ -160,30 +159,25 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
         sy[m] = Ph::template slope3<LIMITER>(wm[m], wc[m], wp[m]);
       }
       if (P.secondorder) {
-        T a1[5], a2[5];
-        Ph::template predictor_dir<0>(P, wc, rc, sx, a1);
-        Ph::template predictor_dir<1>(P, wc, rc, sy, a2);
-        fast::evo5_2d(P, dt2, a1, a2, ev);  // muscl.f90:79-85
+        Ph::evo2d(evof, P, wc, rc, sx, sy, ev);
       } else {
 #pragma unroll
         for (int m = 0; m < 5; m++) { ev[m] = T(0); sx[m] = T(0); sy[m] = T(0); }
       }
-      // face states (muscl.f90:207-210): (w + 0.5 s) + evo on the high side,
-      // (w - 0.5 s) + evo on the low side
       if (face) {
 #pragma unroll
-        for (int m = 0; m < 5; m++) XB[m][l] = fm::fmad(half, sx[m], wc[m]) + ev[m];
+        for (int m = 0; m < 5; m++) XB[m][l] = fast::face_state(wc[m], T(0.5), sx[m], ev[m]);
       }
       if (l >= 2) {
 #pragma unroll
-        for (int m = 0; m < 5; m++) XB[5 + m][l - 1] = fm::fmad(-half, sx[m], wc[m]) + ev[m];
+        for (int m = 0; m < 5; m++) XB[5 + m][l - 1] = fast::face_state(wc[m], T(-0.5), sx[m], ev[m]);
       }
       if (inner) {
         T yb[5], yt[5];
 #pragma unroll
         for (int m = 0; m < 5; m++) {
-          yb[m] = fm::fmad(-half, sy[m], wc[m]) + ev[m];
-          yt[m] = fm::fmad(half, sy[m], wc[m]) + ev[m];
+          yb[m] = fast::face_state(wc[m], T(-0.5), sy[m], ev[m]);
+          yt[m] = fast::face_state(wc[m], T(0.5), sy[m], ev[m]);
         }
         if (k >= y0) {
           T fy[6], yt0[5];
@@ -197,8 +191,8 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
           if (k - 1 >= y0 && inside) {
 #pragma unroll
             for (int m = 0; m < 6; m++) {
-              if constexpr (LC) o[m] = fm::fmad(dty, sm.F[m][l] - fy[m], part[m]);
-              else o[m] = fm::fmad(dty, fyb[m] - fy[m], part[m]);
+              if constexpr (LC) o[m] = Ph::mad(dty, sm.F[m][l] - fy[m], part[m]);
+              else o[m] = Ph::mad(dty, fyb[m] - fy[m], part[m]);
             }
             oc = (long long)gx + (long long)G.nx * (k - 1);
 #pragma unroll
@@ -238,7 +232,7 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
     // ---- S4: q(k) + dtx*(Fx) of row k; the end of row k-1
     if (out_row && inner) {
 #pragma unroll
-      for (int m = 0; m < 6; m++) part[m] = fm::fmad(dtx, XB[m][l - 1] - XB[m][l], qc[m]);
+      for (int m = 0; m < 6; m++) part[m] = Ph::mad(dtx, XB[m][l - 1] - XB[m][l], qc[m]);
     }
     if (pend) {
       T on[6], wn[5], rn;

@@ -41,7 +41,25 @@ struct KParams {
   int g1_third;       // |2/3 - g1| <= 1e-6: powers of g1 via the cube root
   int conduction;     // thermal conduction (simplekappa) on
   double c_cond, temp0, kappa0;
+  double ggm;   // g g1: (a rho)^2 = ggm (rho E - m^2/2)
+  double calm;  // share of rho E that rho E - m^2/2 exceeds where p > 0 comes from E in every form
+  // the same rounded to single precision, for the FP32-mixed kernels: read
+  // from here they stay in scalar registers, where a conversion in the kernel
+  // (the vector unit's) would hold a vector register each for its whole loop
+  struct Single {
+    float g, g1, g1inv, gg1, de_thresh1, kin_frac64, temp0, dxinv, dyinv, dzinv, dx, dy, dz, ggm, calm;
+  } f;
 };
+
+// the constants in the compute type
+__host__ __device__ __forceinline__ const KParams &consts(const KParams &P, double) { return P; }
+__host__ __device__ __forceinline__ const KParams::Single &consts(const KParams &P, float) { return P.f; }
+
+// a value that is the same in every lane, moved to scalar registers
+__device__ __forceinline__ float uniform(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double uniform(double v) { return v; }  // FP64 kernels have no scalar registers to spare
 
 // Device status block: first error (code, linear cell) and min reductions.
 struct Status {

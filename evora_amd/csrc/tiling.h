@@ -25,6 +25,19 @@ __device__ __forceinline__ int xcd_tile(int b, int ntiles) {
 // blocks to launch for ntiles tiles (a multiple of the XCD count)
 inline int xcd_blocks(int ntiles) { return kXcds * ((ntiles + kXcds - 1) / kXcds); }
 
+// The column tile of the 3-D march for tile height 12, 192 columns either way:
+// 16 x 12, or in FP32 32 x 6 (wide) where that takes at most 5% more tiles to
+// cover a plane of the grid (or of all boxes together).  The wide tile's ring
+// has half the columns beyond its x sides, each of which costs the L1 a
+// request of a whole line for one value, and more columns in all.  FP32 is
+// bound by those requests: 512^3 2.51 ms wide against 2.78, 384^3 1.15 against
+// 1.26, 256^3 0.361 against 0.387.  FP64 is bound by instruction issue, the
+// ring's included: 512^3 5.55 ms wide against 5.39, 256^3 0.765 against 0.735.
+inline long long tiles_of(int nx, int ny, int tx, int ty) {
+  return (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
+}
+inline bool wide_tile(long long tiles32x6, long long tiles16x12) { return 20 * tiles32x6 <= 21 * tiles16x12; }
+
 // Chunk lengths when the tuning leaves them open.  A block's march is
 // serial, so on a small grid long chunks leave most of the GPU idle and a
 // pass takes the march's latency; short chunks cost a few planes more of

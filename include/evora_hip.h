@@ -172,13 +172,14 @@ int evh_event_elapsed(evh_ctx *h, int a, int b, float *ms); /* syncs on slot b *
 int evh_synchronize(evh_ctx *h);
 
 /* Launch shape of the fused kernel (no counterpart in the reference; set by
- * the autotuner): tile height 8 or 12 columns, occupancy target (0: the
- * lower, 1: the higher of the two register budgets compiled per precision),
- * z planes per block (rows on 2-D grids; 0, the default: 64 planes or 32
- * rows, halved down to 4 while the grid gives fewer than 1024 blocks).
- * Invalid values are rejected.  A z-slab with halo buffers (evh_slab) runs
- * tile height 12 at the higher budget; its z chunk is the tuning's.  The
- * results do not depend on the launch shape. */
+ * the autotuner): tile height 8 (tiles of 16 x 8 columns) or 12 (192 columns,
+ * 16 x 12 or, in FP32-mixed, 32 x 6 where that covers the grid as well),
+ * occupancy target (0 or 1; kept for callers, both give the one register
+ * budget compiled per precision), z planes per block (rows on 2-D grids; 0,
+ * the default: 64 planes or 32 rows, halved down to 4 while the grid gives
+ * too few blocks).  Invalid values are rejected.  A z-slab with halo buffers
+ * (evh_slab) runs tile height 12; its z chunk is the tuning's.  The results
+ * do not depend on the launch shape. */
 int evh_set_tuning(evh_ctx *h, int tile_ty, int wpe_hi, int zchunk);
 int evh_get_tuning(evh_ctx *h, int *tile_ty, int *wpe_hi, int *zchunk);
 
@@ -234,7 +235,8 @@ int evh_batch_set_time(evh_batch *b, const double *t, const double *tend);
 int evh_batch_run(evh_batch *b, int nsteps, int use_graph, float *ms);
 /* per-box t, last dt, steps done and go flag; any pointer may be NULL */
 int evh_batch_times(evh_batch *b, double *t, double *dt, int *steps, int *go);
-/* launch shape: tile height 8|12, occupancy target 0|1, z chunk, blocks per CU */
+/* launch shape as evh_set_tuning: tile height 8|12, occupancy target 0|1 (one
+ * register budget either way), z chunk, blocks per CU */
 int evh_batch_set_tuning(evh_batch *b, int tile_ty, int wpe_hi, int zchunk, int blocks_per_cu);
 int evh_batch_get_tuning(evh_batch *b, int *tile_ty, int *wpe_hi, int *zchunk, int *blocks_per_cu);
 /* time every launch shape for trial_steps steps on a snapshot of the state,
