@@ -83,6 +83,14 @@ __global__ void k_clear_code(Status *st) {
   }
 }
 
+__global__ void k_clear_statuses(Status *st, int n) {
+  if ((int)threadIdx.x < n) clear_status(st + threadIdx.x);
+}
+
+__global__ void k_run_start(RunSlot *r, double t) {
+  if (threadIdx.x == 0) *r = RunSlot{t, 1e99, 1, 0, 0, 0};
+}
+
 // AoS chunk (cells x 6, double) -> SoA storage at cell offset `base`
 template <typename S>
 __global__ void k_aos_to_soa(const double *__restrict__ src, S *__restrict__ dst, long long cells, long long base,
@@ -180,13 +188,8 @@ hipError_t timer_end(evh_ctx *h, int stage) {
   return e;
 }
 
-// Sync and surface device-side errors.  Errors stay sticky until read here.
-int check_status(evh_ctx *h) {
-  // the status block is read behind the queued work (pinned host copy, one
-  // wait instead of a wait and a blocking copy)
-  HIP_TRY(hipMemcpyAsync(h->st_host, h->st, sizeof(Status), hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  accumulate_timing(h);
+// Surface the device-side errors of a status block read into st_host.
+int surface_errors(evh_ctx *h) {
   if (h->st_host->code) {
     const int code = h->st_host->code;
     const long long cell = (long long)h->st_host->cell;
@@ -196,6 +199,24 @@ int check_status(evh_ctx *h) {
     return fail(h, code, "device", cell);
   }
   return EVH_OK;
+}
+
+// Sync and surface device-side errors.  Errors stay sticky until read here.
+int check_status(evh_ctx *h) {
+  // the status block is read behind the queued work (pinned host copy, one
+  // wait instead of a wait and a blocking copy)
+  HIP_TRY(hipMemcpyAsync(h->st_host, h->st, sizeof(Status), hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  accumulate_timing(h);
+  return surface_errors(h);
+}
+
+// the control block of a kernel that the host gives dt, on the current status
+StepCtl plain_ctl(const evh_ctx *h, double dt) {
+  StepCtl c = {};
+  c.dt = dt;
+  c.st = c.lim = h->st;
+  return c;
 }
 
 int ensure_staged_arrays(evh_ctx *h) {
@@ -324,11 +345,14 @@ int evh_create(const evh_config *cfg, evh_ctx **out) {
   }
   if (h->cfg.gravity && (e = gravity_init(h)) != hipSuccess) return bail(e);
   if ((e = h->xfer.init(n)) != hipSuccess) return bail(e);
-  if ((e = hipMalloc(&h->st, sizeof(Status))) != hipSuccess) return bail(e);
+  if ((e = hipMalloc(&h->st_all, 4 * sizeof(Status))) != hipSuccess) return bail(e);
+  h->st = h->st_all;
+  if ((e = hipMalloc(&h->runs, 2 * sizeof(RunSlot))) != hipSuccess) return bail(e);
   if ((e = hipHostMalloc(&h->st_host, sizeof(Status))) != hipSuccess) return bail(e);
+  if ((e = hipHostMalloc(&h->run_host, sizeof(evh_ctx::RunHost))) != hipSuccess) return bail(e);
   if ((e = hipMalloc(&h->partials, sizeof(double) * 6 * kSumBlocks)) != hipSuccess) return bail(e);
-  h->dev_bytes += h->xfer.device_bytes() + (long long)sizeof(Status) + (long long)sizeof(double) * 6 * kSumBlocks;
-  hipLaunchKernelGGL(k_clear_code, dim3(1), dim3(64), 0, h->stream, h->st);
+  h->dev_bytes += h->xfer.device_bytes() + (long long)(4 * sizeof(Status) + 2 * sizeof(RunSlot)) + (long long)sizeof(double) * 6 * kSumBlocks;
+  hipLaunchKernelGGL(k_clear_statuses, dim3(1), dim3(64), 0, h->stream, h->st_all, 4);
   if ((e = hipStreamSynchronize(h->stream)) != hipSuccess) return bail(e);
   *out = h;
   return EVH_OK;
@@ -344,8 +368,10 @@ int evh_destroy(evh_ctx *h) {
   if (h->evo) hipFree(h->evo);
   if (h->s) hipFree(h->s);
   h->xfer.release();
-  if (h->st) hipFree(h->st);
+  if (h->st_all) hipFree(h->st_all);
+  if (h->runs) hipFree(h->runs);
   if (h->st_host) hipHostFree(h->st_host);
+  if (h->run_host) hipHostFree(h->run_host);
   if (h->partials) hipFree(h->partials);
   for (auto p : h->zhalo) if (p) hipFree(p);
   for (auto p : h->thalo) if (p) hipFree(p);
@@ -495,10 +521,14 @@ int evh_sweep(evh_ctx *h, double dt) {
     return check_status(h);
   }
   if (!h->v_valid) return fail(h, EVH_ERR_STATE, "sweep before primitive");
-  HIP_TRY(launch_reset_status(h, false));
+  StepCtl c = plain_ctl(h, dt);
+  c.prev = h->st;
+  c.st = c.lim = next_status(h, 1);
+  c.reset = next_status(h, 2);
   HIP_TRY(timer_begin(h, EVH_STAGE_SWEEP));
-  HIP_TRY(launch_fused_step(h, dt));
+  HIP_TRY(launch_fused_step(h, c));
   HIP_TRY(timer_end(h, EVH_STAGE_SWEEP));
+  h->st = c.st;
   h->cur = 1 - h->cur;
   h->v_valid = true;
   h->tv_valid = false;
@@ -537,7 +567,7 @@ int evh_thermalconduction(evh_ctx *h, double dt) {
   if (!h->t_valid) HIP_TRY(launch_temp(h));
   HIP_TRY(launch_reset_status(h, false));
   HIP_TRY(timer_begin(h, EVH_STAGE_CONDUCTION));
-  HIP_TRY(launch_conduction(h, dt));
+  HIP_TRY(launch_conduction(h, plain_ctl(h, dt)));
   HIP_TRY(timer_end(h, EVH_STAGE_CONDUCTION));
   h->v_valid = true;
   h->tv_valid = true;
@@ -553,7 +583,7 @@ int evh_gravpotential(evh_ctx *h, double cosmo) {
   if (!h->cfg.gravity) return fail(h, EVH_ERR_STATE, "gravpotential without gravity");
   h->cosmo = cosmo;
   HIP_TRY(timer_begin(h, EVH_STAGE_GRAVPOTENTIAL));
-  HIP_TRY(launch_gravpotential(h, cosmo));
+  HIP_TRY(launch_gravpotential(h, cosmo, plain_ctl(h, 0.0)));
   HIP_TRY(timer_end(h, EVH_STAGE_GRAVPOTENTIAL));
   h->phi_valid = true;
   return EVH_OK;
@@ -566,7 +596,7 @@ int evh_gravintegration(evh_ctx *h, double dt) {
   if (!h->phi_valid) return fail(h, EVH_ERR_STATE, "gravintegration before gravpotential");
   HIP_TRY(launch_reset_status(h, false));
   HIP_TRY(timer_begin(h, EVH_STAGE_GRAVINTEGRATION));
-  HIP_TRY(launch_gravintegration(h, dt));
+  HIP_TRY(launch_gravintegration(h, plain_ctl(h, dt)));
   HIP_TRY(timer_end(h, EVH_STAGE_GRAVINTEGRATION));
   h->v_valid = true;                // the kernel formed the CFL minimum of the new state
   h->tv_valid = false;
@@ -613,10 +643,98 @@ int evh_step(evh_ctx *h, double *t, double tend, double *dt, int *go) {
   return EVH_OK;
 }
 
+// evh_run without a wait per step: the kernels form dt and t themselves
+// (stepctl.h), the host launches up to kRunBatch steps and reads what became
+// of them.
+static int run_on_device(evh_ctx *h, int nsteps, double *t, double tend, double *dt, int *done) {
+  constexpr int kRunBatch = 64;
+  const bool hydro = !h->cfg.hydro_off, grav = h->cfg.gravity, cond = h->cfg.conduction;
+  int r;
+  if ((r = evh_primitive(h))) return r;
+  if (cond && !h->tv_valid) {
+    HIP_TRY(launch_thermal_min(h));
+    h->tv_valid = true;
+  }
+  hipLaunchKernelGGL(k_run_start, dim3(1), dim3(64), 0, h->stream, h->runs, *t);
+  Status *const st0 = h->st;
+  const int slot0 = (int)(st0 - h->st_all), cur0 = h->cur;
+  const bool sums0 = h->rho_sums_valid;
+  RunSlot end = {};
+  for (int j = 0; j < nsteps && !end.stop;) {
+    const int batch = nsteps - j < kRunBatch ? nsteps - j : kRunBatch;
+    for (int i = 0; i < batch; i++, j++) {
+      StepCtl c = {};
+      c.prev = h->st;
+      c.st = next_status(h, 1);
+      c.reset = next_status(h, 2);
+      c.in = h->runs + (j & 1);
+      c.out = h->runs + ((j + 1) & 1);
+      c.tend = tend;
+      c.hydro = hydro ? 1 : 0;
+      c.head = 1;
+      Status *const replaced = h->st_all + 3;  // limits that a later kernel of the step replaces
+      if (hydro) {
+        c.lim = grav || cond ? replaced : c.st;
+        HIP_TRY(launch_fused_step(h, c));
+        h->cur = 1 - h->cur;
+        c.head = 0;
+      }
+      if (grav) {
+        HIP_TRY(launch_gravpotential(h, h->cosmo, c));
+        c.lim = cond ? replaced : c.st;
+        HIP_TRY(launch_gravintegration(h, c));
+        c.head = 0;
+      }
+      if (cond) {
+        if (!hydro) HIP_TRY(launch_temp(h));
+        c.lim = c.st;
+        HIP_TRY(launch_conduction(h, c));
+      }
+      h->st = c.st;
+    }
+    HIP_TRY(hipMemcpyAsync(h->run_host->st, h->st_all, 3 * sizeof(Status), hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipMemcpyAsync(h->run_host->runs, h->runs, 2 * sizeof(RunSlot), hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    end = h->run_host->runs[j & 1];
+  }
+  // the steps that were taken, and the state and limits they left
+  h->st = h->st_all + (slot0 + end.done) % 3;
+  *h->st_host = h->run_host->st[h->st - h->st_all];
+  if (hydro) h->cur = (cur0 + end.done) & 1;
+  if (end.done > 0) {
+    h->v_valid = true;
+    h->tv_valid = cond;
+    h->t_valid = !cond && h->tbuf != nullptr;
+    if (grav) h->phi_valid = true;
+    h->evo_valid = false;
+    h->w_valid = false;
+    h->bound_done = false;
+  } else {
+    h->rho_sums_valid = sums0;
+  }
+  *t = end.t;
+  *dt = end.dt;
+  *done = end.done;
+  if (end.why == kRunNext) {
+    if ((r = surface_errors(h))) return r;
+    h->v_valid = false;
+    if (!hydro) h->tv_valid = false;
+    return fail(h, (int)h->st_host->next_code, hydro ? "primitive" : "thermalstep", (long long)h->st_host->next_cell);
+  }
+  if (end.why == kRunDt) return fail(h, EVH_ERR_DT);
+  return surface_errors(h);
+}
+
 int evh_run(evh_ctx *h, int nsteps, double *t, double tend, double *dt, int *done) {
   if (!h || !t || !dt || !done) return EVH_ERR_STATE;
   int go = 1;
   *done = 0;
+  // one wait at the end where every kernel of a step can take its dt from the
+  // device: not with the staged kernels, nor hipFFT's transforms; with the
+  // stages timed, each step is waited for as its events are
+  const bool device = h->mode != EVH_MODE_STAGED && !h->timing && !h->zslab[0] && !h->zslab[1] &&
+                      (!h->cfg.gravity || h->xyz_pencils) && nsteps > 1;
+  if (device) return run_on_device(h, nsteps, t, tend, dt, done);
   for (int k = 0; k < nsteps && go; k++) {
     int r = evh_step(h, t, tend, dt, &go);
     if (r) return r;

@@ -100,7 +100,7 @@ __global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((
       const Geo G = bx.G;
       const bool to1 = bs.side[b] != 0;
       core::march<T, S, SOLVER, LIMITER, TX, TY, false>(P, G, to1 ? q0 : q1, to1 ? q1 : q0, bx.qoff, b, bs.dt[b],
-                                                    &bs.st[b], &bs.st[b].vmin_bits, item - bx.tile0, sm);
+                                                    &bs.st[b], &bs.st[b], item - bx.tile0, sm);
     }
     __syncthreads();  // s_item is rewritten only after every lane has used it
   }

@@ -194,10 +194,11 @@ using M = CondMath<kExact>;
 
 template <typename S>
 __global__ void __launch_bounds__(CT) k_conduct(KParams P, CGeo G, S *__restrict__ q, const S *__restrict__ tb,
-                                                double dt, Status *st) {
+                                                StepCtl C) {
   __shared__ double T[RY * RX];
   const int lin = xcd_tile(blockIdx.x, G.ntiles);
-  if (lin < 0) return;  // padding block (whole block exits before any barrier)
+  double dt;
+  if (!step_begin(P, C, dt) || lin < 0) return;  // no step, or a padding block (whole blocks, before any barrier)
   const int tile = lin % (G.tiles_x * G.tiles_y), chunk = lin / (G.tiles_x * G.tiles_y);
   const int x0 = (tile % G.tiles_x) * CX, y0 = (tile / G.tiles_x) * CY;
   const int z0 = chunk * G.zchunk, z1 = min(z0 + G.zchunk, G.nz);
@@ -243,7 +244,7 @@ __global__ void __launch_bounds__(CT) k_conduct(KParams P, CGeo G, S *__restrict
       // the primitive of main.f90:171 before thermalconduction stops on a
       // non-positive pressure of this cell
       const int e = M::update(P, G, kc, qc, tc, T[me - 1], T[me + 1], T[me - RX], T[me + RX], tm, tn);
-      if (e) report(st, e, (unsigned long long)c);
+      if (e) report(C.st, e, (unsigned long long)c);
       q[4 * G.n + c] = S(qc[4]);
       q[5 * G.n + c] = S(qc[5]);
       // the next step's limits from the new state (as stored)
@@ -251,7 +252,7 @@ __global__ void __launch_bounds__(CT) k_conduct(KParams P, CGeo G, S *__restrict
 #pragma unroll
       for (int m = 0; m < 6; m++) qs[m] = double(S(qc[m]));
       const int ep = M::limits(P, qs, v, tv);
-      if (ep) report_next(st, ep, (unsigned long long)c);
+      if (ep) report_next(C.lim, ep, (unsigned long long)c);
       vmin = dmin(vmin, v);
       tvmin = dmin(tvmin, tv);
     }
@@ -264,8 +265,8 @@ __global__ void __launch_bounds__(CT) k_conduct(KParams P, CGeo G, S *__restrict
     tvmin = dmin(tvmin, __shfl_xor(tvmin, off));
   }
   if ((tid & 63) == 0) {
-    atomic_min_pos(&st->vmin_bits, vmin);
-    atomic_min_pos(&st->tvmin_bits, tvmin);
+    atomic_min_pos(&C.lim->vmin_bits, vmin);
+    atomic_min_pos(&C.lim->tvmin_bits, tvmin);
   }
 }
 
@@ -337,12 +338,12 @@ void launch_thermal_min_s(evh_ctx *h) {
 // q[cur] in place, with T of q[cur] in tbuf; the caller resets the CFL
 // minimum before
 template <typename S>
-void launch_conduction_s(evh_ctx *h, double dt) {
-  hipLaunchKernelGGL(k_reset_tv, dim3(1), dim3(64), 0, h->stream, h->st);
+void launch_conduction_s(evh_ctx *h, const StepCtl &c) {
+  if (!c.in) hipLaunchKernelGGL(k_reset_tv, dim3(1), dim3(64), 0, h->stream, c.lim);
   const CGeo g = make_cgeo(h);
   const int blocks = xcd_blocks(g.ntiles);
   hipLaunchKernelGGL(k_conduct<S>, dim3(blocks), dim3(CT), 0, h->stream, h->kp, g, (S *)h->qbuf[h->cur],
-                     (const S *)h->tbuf, dt, h->st);
+                     (const S *)h->tbuf, c);
 }
 
 }  // namespace
@@ -357,8 +358,8 @@ hipError_t launch_temp_exact(evh_ctx *h) {
   launch_temp_s<double>(h);
   return hipGetLastError();
 }
-hipError_t launch_conduction_exact(evh_ctx *h, double dt) {
-  launch_conduction_s<double>(h, dt);
+hipError_t launch_conduction_exact(evh_ctx *h, const StepCtl &c) {
+  launch_conduction_s<double>(h, c);
   return hipGetLastError();
 }
 #else
@@ -377,10 +378,10 @@ hipError_t launch_temp(evh_ctx *h) {
   else launch_temp_s<double>(h);
   return hipGetLastError();
 }
-hipError_t launch_conduction(evh_ctx *h, double dt) {
-  if (use_exact(h)) return launch_conduction_exact(h, dt);
-  if (h->cfg.precision == EVH_FP32_MIXED) launch_conduction_s<float>(h, dt);
-  else launch_conduction_s<double>(h, dt);
+hipError_t launch_conduction(evh_ctx *h, const StepCtl &c) {
+  if (use_exact(h)) return launch_conduction_exact(h, c);
+  if (h->cfg.precision == EVH_FP32_MIXED) launch_conduction_s<float>(h, c);
+  else launch_conduction_s<double>(h, c);
   return hipGetLastError();
 }
 #endif

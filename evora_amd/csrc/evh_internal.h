@@ -7,6 +7,7 @@
 
 #include "../../include/evora_hip.h"
 #include "physics.h"
+#include "stepctl.h"
 #include "tiling.h"
 #include "transfer.h"
 
@@ -85,8 +86,15 @@ struct evh_ctx {
   evh::Xfer xfer;
 
   // reductions
-  evh::Status *st = nullptr;      // device
-  evh::Status *st_host = nullptr; // pinned
+  // status blocks on the device: three that take turns and one for what a
+  // later kernel of the same step replaces; st: the current state's
+  evh::Status *st_all = nullptr, *st = nullptr;
+  evh::Status *st_host = nullptr;  // pinned
+  evh::RunSlot *runs = nullptr;    // device: the two slots of a run of several steps
+  struct RunHost {
+    evh::Status st[3];
+    evh::RunSlot runs[2];
+  } *run_host = nullptr;  // pinned
   double *partials = nullptr;     // per-block sums
   int npartials = 0;
 
@@ -125,30 +133,32 @@ hipError_t launch_sweep(evh_ctx *h, double dt);
 
 // fused kernels (fused.hip)
 hipError_t launch_cfl(evh_ctx *h);                 // primitive + CFL min over cur q
-hipError_t launch_fused_step(evh_ctx *h, double dt);  // cur -> other, CFL of the result
-hipError_t launch_fused_f64(evh_ctx *h, double dt);
-hipError_t launch_fused_f32(evh_ctx *h, double dt);
-hipError_t launch_fused_exact(evh_ctx *h, double dt);  // FP64, reference arithmetic
+hipError_t launch_fused_step(evh_ctx *h, const StepCtl &c);  // cur -> other, CFL of the result
+hipError_t launch_fused_f64(evh_ctx *h, const StepCtl &c);
+hipError_t launch_fused_f32(evh_ctx *h, const StepCtl &c);
+hipError_t launch_fused_exact(evh_ctx *h, const StepCtl &c);  // FP64, reference arithmetic
 // conduction kernels (conduction.hip)
 hipError_t launch_thermal_min(evh_ctx *h);              // conduction limit of cur q
 hipError_t launch_temp(evh_ctx *h);                     // tbuf from cur q
-hipError_t launch_conduction(evh_ctx *h, double dt);    // cur q in place (tbuf valid), limits of the result
+hipError_t launch_conduction(evh_ctx *h, const StepCtl &c);    // cur q in place (tbuf valid), limits of the result
 hipError_t launch_thermal_min_exact(evh_ctx *h);        // the same with the reference's arithmetic
 hipError_t launch_temp_exact(evh_ctx *h);
-hipError_t launch_conduction_exact(evh_ctx *h, double dt);
+hipError_t launch_conduction_exact(evh_ctx *h, const StepCtl &c);
 bool fused_supported(const evh_config &c);
 
 // gravity (gravity.hip)
 hipError_t gravity_init(evh_ctx *h);     // buffers, tables and FFT plans
 void gravity_release(evh_ctx *h);
-hipError_t launch_gravpotential(evh_ctx *h, double cosmo);  // phi of cur q
-hipError_t launch_gravintegration(evh_ctx *h, double dt);   // cur q in place with phi, limits (and T) of the result
+hipError_t launch_gravpotential(evh_ctx *h, double cosmo, const StepCtl &c);  // phi of cur q
+hipError_t launch_gravintegration(evh_ctx *h, const StepCtl &c);              // cur q in place with phi, limits (and T) of the result
 
 // KParams of a configuration (api.hip)
 KParams make_kparams(const evh_config &c);
 
 // transfers and reductions (api.hip)
 hipError_t launch_reset_status(evh_ctx *h, bool keep_next);
+// the status block the next step's new state takes (steps = 1), or the one after
+inline Status *next_status(const evh_ctx *h, int steps) { return h->st_all + (h->st - h->st_all + steps) % 3; }
 hipError_t launch_sums(evh_ctx *h, double *out3);
 
 }  // namespace evh

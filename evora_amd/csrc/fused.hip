@@ -40,24 +40,24 @@ using core::Geo;
 // SLAB: a z-slab whose ghost planes may come from halo buffers.
 template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, int WPE, bool SLAB>
 __global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-    K_FUSED(KParams P, Geo G, const S *__restrict__ qin, S *__restrict__ qout, double dt, Status *st,
-            S *__restrict__ tout) {
+    K_FUSED(KParams P, Geo G, const S *__restrict__ qin, S *__restrict__ qout, StepCtl C, S *__restrict__ tout) {
   __shared__ core::Smem<T, TX, TY> sm;
   const int lin = xcd_tile(blockIdx.x, G.ntiles);
-  if (lin < 0) return;  // padding block (whole block exits before any barrier)
-  core::march<T, S, SOLVER, LIMITER, TX, TY, kExact, SLAB>(P, G, qin, qout, 0, 0, dt, st, &st->vmin_bits, lin, sm,
-                                                        tout);
+  double dt;
+  if (!step_begin(P, C, dt) || lin < 0) return;  // no step, or a padding block (whole blocks, before any barrier)
+  core::march<T, S, SOLVER, LIMITER, TX, TY, kExact, SLAB>(P, G, qin, qout, 0, 0, dt, C.st, C.lim, lin, sm, tout);
 }
 
 // 2-D grids (nz = 1): row strips marching along y (march2d.h)
 template <typename T, typename S, int SOLVER, int LIMITER, int WPE>
 __global__ void __launch_bounds__(core2d::NL) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-    K_FUSED2D(KParams P, core2d::Geo2 G, const S *__restrict__ qin, S *__restrict__ qout, double dt, Status *st,
+    K_FUSED2D(KParams P, core2d::Geo2 G, const S *__restrict__ qin, S *__restrict__ qout, StepCtl C,
               S *__restrict__ tout) {
   __shared__ core2d::Smem2<T> sm;
   const int lin = xcd_tile(blockIdx.x, G.ntiles);
-  if (lin < 0) return;  // padding block (whole block exits before any barrier)
-  core2d::march2d<T, S, SOLVER, LIMITER, kExact>(P, G, qin, qout, dt, st, &st->vmin_bits, lin, sm, tout);
+  double dt;
+  if (!step_begin(P, C, dt) || lin < 0) return;  // no step, or a padding block (whole blocks, before any barrier)
+  core2d::march2d<T, S, SOLVER, LIMITER, kExact>(P, G, qin, qout, dt, C.st, C.lim, lin, sm, tout);
 }
 
 // primitive + CFL min over q without materialising w (first step, after
@@ -95,18 +95,18 @@ Geo make_geo(const evh_ctx *h, int tx, int ty) {
 }
 
 template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, int WPE, bool SLAB = false>
-void launch_ty(evh_ctx *h, double dt) {
+void launch_ty(evh_ctx *h, const StepCtl &c) {
   const Geo g = make_geo(h, TX, TY);
   const int blocks = xcd_blocks(g.ntiles);
   hipLaunchKernelGGL((K_FUSED<T, S, SOLVER, LIMITER, TX, TY, WPE, SLAB>), dim3(blocks), dim3((core::TileShape<TX, TY>::NT)), 0,
-                     h->stream, h->kp, g, (const S *)h->qbuf[h->cur], (S *)h->qbuf[1 - h->cur], dt, h->st,
+                     h->stream, h->kp, g, (const S *)h->qbuf[h->cur], (S *)h->qbuf[1 - h->cur], c,
                      (S *)h->tbuf);
 }
 
 // the 2-D form: strips of 252 columns, chunks of up to 32 rows (the z chunk
 // of the tuning, when set), WPE waves per SIMD
 template <typename T, typename S, int SOLVER, int LIMITER, int WPE>
-void launch_2d(evh_ctx *h, double dt) {
+void launch_2d(evh_ctx *h, const StepCtl &c) {
   core2d::Geo2 g;
   g.nx = h->grid.nx;
   g.ny = h->grid.ny;
@@ -119,7 +119,7 @@ void launch_2d(evh_ctx *h, double dt) {
   g.nchunks = (g.ny + g.ychunk - 1) / g.ychunk;
   g.ntiles = g.strips * g.nchunks;
   hipLaunchKernelGGL((K_FUSED2D<T, S, SOLVER, LIMITER, WPE>), dim3(xcd_blocks(g.ntiles)), dim3(core2d::NL), 0,
-                     h->stream, h->kp, g, (const S *)h->qbuf[h->cur], (S *)h->qbuf[1 - h->cur], dt, h->st,
+                     h->stream, h->kp, g, (const S *)h->qbuf[h->cur], (S *)h->qbuf[1 - h->cur], c,
                      (S *)h->tbuf);
 }
 
@@ -128,40 +128,40 @@ void launch_2d(evh_ctx *h, double dt) {
 // against 5.8 at 512^3) and 4 in FP32.  2-D grids take the row-strip march in
 // its one shape.
 template <typename T, typename S, int SOLVER, int LIMITER>
-void launch_fused_t(evh_ctx *h, double dt) {
+void launch_fused_t(evh_ctx *h, const StepCtl &c) {
   constexpr int W = sizeof(T) == 8 ? 2 : 4;
   const int nx = h->grid.nx, ny = h->grid.ny;
   if (h->grid.nz == 1) {
     // 2-D: FP64 at 3 waves per SIMD (its row carry in LDS: 3% faster than 2
     // waves at 8192^2), FP32 at 4
-    launch_2d<T, S, SOLVER, LIMITER, sizeof(T) == 8 ? 3 : 4>(h, dt);
+    launch_2d<T, S, SOLVER, LIMITER, sizeof(T) == 8 ? 3 : 4>(h, c);
     return;
   }
   const bool slab = h->zslab[0] || h->zslab[1];  // with halo buffers: tile height 12 (the z chunk is the tuning's)
   if (!slab && h->tile_ty == 8) {
-    launch_ty<T, S, SOLVER, LIMITER, 16, 8, W>(h, dt);
+    launch_ty<T, S, SOLVER, LIMITER, 16, 8, W>(h, c);
     return;
   }
   if constexpr (sizeof(T) == 4) {
     if (wide_tile(tiles_of(nx, ny, 32, 6), tiles_of(nx, ny, 16, 12))) {
-      if (slab) launch_ty<T, S, SOLVER, LIMITER, 32, 6, W, true>(h, dt);
-      else launch_ty<T, S, SOLVER, LIMITER, 32, 6, W>(h, dt);
+      if (slab) launch_ty<T, S, SOLVER, LIMITER, 32, 6, W, true>(h, c);
+      else launch_ty<T, S, SOLVER, LIMITER, 32, 6, W>(h, c);
       return;
     }
   }
-  if (slab) launch_ty<T, S, SOLVER, LIMITER, 16, 12, W, true>(h, dt);
-  else launch_ty<T, S, SOLVER, LIMITER, 16, 12, W>(h, dt);
+  if (slab) launch_ty<T, S, SOLVER, LIMITER, 16, 12, W, true>(h, c);
+  else launch_ty<T, S, SOLVER, LIMITER, 16, 12, W>(h, c);
 }
 
 template <typename T, typename S>
-hipError_t launch_fused_prec(evh_ctx *h, double dt) {
+hipError_t launch_fused_prec(evh_ctx *h, const StepCtl &c) {
   const int s = h->kp.solver, l = h->kp.limiter;
-  if (s == 1 && l == 1) launch_fused_t<T, S, 1, 1>(h, dt);
-  else if (s == 1 && l == 2) launch_fused_t<T, S, 1, 2>(h, dt);
-  else if (s == 1 && l == 3) launch_fused_t<T, S, 1, 3>(h, dt);
-  else if (s == 2 && l == 1) launch_fused_t<T, S, 2, 1>(h, dt);
-  else if (s == 2 && l == 2) launch_fused_t<T, S, 2, 2>(h, dt);
-  else if (s == 2 && l == 3) launch_fused_t<T, S, 2, 3>(h, dt);
+  if (s == 1 && l == 1) launch_fused_t<T, S, 1, 1>(h, c);
+  else if (s == 1 && l == 2) launch_fused_t<T, S, 1, 2>(h, c);
+  else if (s == 1 && l == 3) launch_fused_t<T, S, 1, 3>(h, c);
+  else if (s == 2 && l == 1) launch_fused_t<T, S, 2, 1>(h, c);
+  else if (s == 2 && l == 2) launch_fused_t<T, S, 2, 2>(h, c);
+  else if (s == 2 && l == 3) launch_fused_t<T, S, 2, 3>(h, c);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }
@@ -187,16 +187,16 @@ hipError_t launch_cfl(evh_ctx *h) {
 #endif
 
 #if EVH_FUSED_EXACT
-hipError_t launch_fused_exact(evh_ctx *h, double dt) { return launch_fused_prec<double, double>(h, dt); }
+hipError_t launch_fused_exact(evh_ctx *h, const StepCtl &c) { return launch_fused_prec<double, double>(h, c); }
 #elif EVH_FUSED_PREC == 32
-hipError_t launch_fused_f32(evh_ctx *h, double dt) { return launch_fused_prec<float, float>(h, dt); }
+hipError_t launch_fused_f32(evh_ctx *h, const StepCtl &c) { return launch_fused_prec<float, float>(h, c); }
 #else
-hipError_t launch_fused_f64(evh_ctx *h, double dt) { return launch_fused_prec<double, double>(h, dt); }
+hipError_t launch_fused_f64(evh_ctx *h, const StepCtl &c) { return launch_fused_prec<double, double>(h, c); }
 
-hipError_t launch_fused_step(evh_ctx *h, double dt) {
-  if (h->cfg.precision == EVH_FP32_MIXED) return launch_fused_f32(h, dt);
-  if (h->mode == EVH_MODE_FUSED_EXACT) return launch_fused_exact(h, dt);
-  return launch_fused_f64(h, dt);
+hipError_t launch_fused_step(evh_ctx *h, const StepCtl &c) {
+  if (h->cfg.precision == EVH_FP32_MIXED) return launch_fused_f32(h, c);
+  if (h->mode == EVH_MODE_FUSED_EXACT) return launch_fused_exact(h, c);
+  return launch_fused_f64(h, c);
 }
 #endif
 

@@ -79,9 +79,14 @@ struct GGeo {
 
 __device__ __forceinline__ int wrap(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
+// a run on the device that takes no further step (run: its slot; nullptr otherwise)
+__device__ __forceinline__ bool stopped(const RunSlot *run) { return run && run->stop; }
+
 // ---- mean density: Kahan per thread, pairwise tree per block, then one block
 template <typename S>
-__global__ void __launch_bounds__(256) k_rho_partials(const S *__restrict__ q, long long n, double *part) {
+__global__ void __launch_bounds__(256) k_rho_partials(const S *__restrict__ q, long long n, double *part,
+                                                      const RunSlot *run) {
+  if (stopped(run)) return;
   __shared__ double red[256];
   // four compensated sums over four interleaved streams, so that four loads
   // are in flight per thread; then their compensated total
@@ -123,7 +128,8 @@ __global__ void __launch_bounds__(256) k_rho_partials(const S *__restrict__ q, l
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-__global__ void __launch_bounds__(kSumBlocks) k_rho_mean(double *part, double n3) {
+__global__ void __launch_bounds__(kSumBlocks) k_rho_mean(double *part, double n3, const RunSlot *run) {
+  if (stopped(run)) return;
   __shared__ double red[kSumBlocks];
   red[threadIdx.x] = part[threadIdx.x];
   __syncthreads();
@@ -137,7 +143,8 @@ __global__ void __launch_bounds__(kSumBlocks) k_rho_mean(double *part, double n3
 // the mean density from the block totals of the previous call's x pass
 // (Neumaier sums per thread, then a pairwise tree)
 __global__ void __launch_bounds__(kSumBlocks) k_rho_mean_from(const double *__restrict__ sums, int nsums, double n3,
-                                                            double *part) {
+                                                            double *part, const RunSlot *run) {
+  if (stopped(run)) return;
   __shared__ double red[kSumBlocks];
   double s = 0.0, c = 0.0;
   for (int i = threadIdx.x; i < nsums; i += kSumBlocks) {
@@ -441,7 +448,8 @@ enum { kPencilGreenZ, kPencilFwdY, kPencilInvY };
 template <int LN, int MODE>
 __global__ void __launch_bounds__(kPencilThreads) __attribute__((amdgpu_waves_per_eu(kPencilWaves, kPencilWaves)))
 k_pencils(double2 *__restrict__ spec, Pencils pc, const double2 *__restrict__ tw,
-          const double *__restrict__ sin2, GParams G, int nx, int ny, int nz) {
+          const double *__restrict__ sin2, GParams G, int nx, int ny, int nz, const RunSlot *run) {
+  if (stopped(run)) return;
   __shared__ double2 X[kPencilElems];
   PencilTile pt;
   pt.X = X;
@@ -471,7 +479,8 @@ template <typename S, int LN, bool SC>
 __global__ void __launch_bounds__(kPencilThreads) __attribute__((amdgpu_waves_per_eu(kPencilWaves, kPencilWaves)))
 k_xfwd(const S *__restrict__ rho, double2 *__restrict__ spec, long long pitch, long long npairs,
        const double2 *__restrict__ tw, GParams G, double cosmo_grav, const double *__restrict__ mean_part,
-       double *__restrict__ rho_sum) {
+       double *__restrict__ rho_sum, const RunSlot *run) {
+  if (stopped(run)) return;
   constexpr int N = 1 << LN, TK = 1 << (kPencilLog - LN), NH = N / 2 + 1;
   using TI = TileIndex<LN, true>;
   __shared__ double2 X[tile_elems<true>()];
@@ -523,7 +532,8 @@ k_xfwd(const S *__restrict__ rho, double2 *__restrict__ spec, long long pitch, l
 template <int LN>
 __global__ void __launch_bounds__(kPencilThreads) __attribute__((amdgpu_waves_per_eu(kPencilWaves, kPencilWaves)))
 k_xinv(const double2 *__restrict__ spec, double *__restrict__ phi, long long pitch, long long npairs,
-       const double2 *__restrict__ tw, GParams G) {
+       const double2 *__restrict__ tw, GParams G, const RunSlot *run) {
+  if (stopped(run)) return;
   constexpr int N = 1 << LN, TK = 1 << (kPencilLog - LN);
   __shared__ double2 X[tile_elems<true>()];
   PencilTile pt;
@@ -573,11 +583,12 @@ __device__ __forceinline__ int cell_limits(const KParams &P, double q[6], double
 // ---- gravintegration + grav_force (gravitation.f90:172-254)
 template <typename S, bool EXACT>
 __global__ void __launch_bounds__(GT) k_gravint(KParams P, GParams Gp, GGeo G, S *__restrict__ q,
-                                                const double *__restrict__ phi, double dt, Status *st,
+                                                const double *__restrict__ phi, StepCtl C,
                                                 S *__restrict__ tout) {
   __shared__ double F[GRY * GRX];
   const int lin = xcd_tile(blockIdx.x, G.ntiles);
-  if (lin < 0) return;  // padding block (whole block exits before any barrier)
+  double dt;
+  if (!step_begin(P, C, dt) || lin < 0) return;  // no step, or a padding block (whole blocks, before any barrier)
   const int tile = lin % (G.tiles_x * G.tiles_y), chunk = lin / (G.tiles_x * G.tiles_y);
   const int x0 = (tile % G.tiles_x) * GX, y0 = (tile / G.tiles_x) * GY;
   const int z0 = chunk * G.zchunk, z1 = min(z0 + G.zchunk, G.nz);
@@ -636,7 +647,7 @@ __global__ void __launch_bounds__(GT) k_gravint(KParams P, GParams Gp, GGeo G, S
 #pragma unroll
       for (int m = 0; m < 6; m++) qs[m] = double(S(qc[m]));
       const int e = cell_limits<EXACT>(P, qs, v, t);
-      if (e) report_next(st, e, (unsigned long long)c);
+      if (e) report_next(C.lim, e, (unsigned long long)c);
       vmin = dmin(vmin, v);
       if (tout) tout[c] = S(t);
     }
@@ -645,7 +656,7 @@ __global__ void __launch_bounds__(GT) k_gravint(KParams P, GParams Gp, GGeo G, S
     pc = pn;
   }
   for (int off = 32; off > 0; off >>= 1) vmin = dmin(vmin, __shfl_xor(vmin, off));
-  if ((tid & 63) == 0) atomic_min_pos(&st->vmin_bits, vmin);
+  if ((tid & 63) == 0) atomic_min_pos(&C.lim->vmin_bits, vmin);
 }
 
 GParams make_gparams(const evh_ctx *h) {
@@ -710,13 +721,13 @@ Pencils make_pencils(int n, int nxh, long long s_elem, long long s_outer) {
 // of kx columns and outer index
 template <int MODE, int LN = 1>
 void launch_pencils(const Pencils &pc, int nouter, hipStream_t st, double2 *spec, const double2 *tw,
-                    const double *sin2, const GParams &gp, int nx, int ny, int nz) {
+                    const double *sin2, const GParams &gp, int nx, int ny, int nz, const RunSlot *run) {
   if constexpr (LN <= kPencilLog) {
     if (pc.ln == LN)
       hipLaunchKernelGGL((k_pencils<LN, MODE>), dim3(nouter * pc.ktiles), dim3(kPencilThreads), 0, st, spec, pc,
-                         tw, sin2, gp, nx, ny, nz);
+                         tw, sin2, gp, nx, ny, nz, run);
     else
-      launch_pencils<MODE, LN + 1>(pc, nouter, st, spec, tw, sin2, gp, nx, ny, nz);
+      launch_pencils<MODE, LN + 1>(pc, nouter, st, spec, tw, sin2, gp, nx, ny, nz, run);
   }
 }
 
@@ -724,18 +735,19 @@ void launch_pencils(const Pencils &pc, int nouter, hipStream_t st, double2 *spec
 // tile of row pairs
 template <typename S, int LN = 1>
 void launch_xfwd(int ln, const S *rho, double2 *spec, long long pitch, long long npairs, hipStream_t st,
-                 const double2 *tw, const GParams &gp, double cosmo_grav, const double *mean_part, double *rho_sum) {
+                 const double2 *tw, const GParams &gp, double cosmo_grav, const double *mean_part, double *rho_sum,
+                 const RunSlot *run) {
   if constexpr (LN <= kPencilLog) {
     constexpr int TK = 1 << (kPencilLog - LN);
     const dim3 grid((unsigned)((npairs + TK - 1) / TK));
     if (ln == LN && gp.supercomoving)
       hipLaunchKernelGGL((k_xfwd<S, LN, true>), grid, dim3(kPencilThreads), 0, st, rho, spec, pitch, npairs, tw, gp,
-                         cosmo_grav, mean_part, rho_sum);
+                         cosmo_grav, mean_part, rho_sum, run);
     else if (ln == LN)
       hipLaunchKernelGGL((k_xfwd<S, LN, false>), grid, dim3(kPencilThreads), 0, st, rho, spec, pitch, npairs, tw, gp,
-                         cosmo_grav, mean_part, rho_sum);
+                         cosmo_grav, mean_part, rho_sum, run);
     else
-      launch_xfwd<S, LN + 1>(ln, rho, spec, pitch, npairs, st, tw, gp, cosmo_grav, mean_part, rho_sum);
+      launch_xfwd<S, LN + 1>(ln, rho, spec, pitch, npairs, st, tw, gp, cosmo_grav, mean_part, rho_sum, run);
   }
 }
 // blocks of the x pass (the tiles of row pairs), one density total each
@@ -747,14 +759,14 @@ int xfwd_blocks(int nx, long long npairs) {
 }
 template <int LN = 1>
 void launch_xinv(int ln, const double2 *spec, double *phi, long long pitch, long long npairs, hipStream_t st,
-                 const double2 *tw, const GParams &gp) {
+                 const double2 *tw, const GParams &gp, const RunSlot *run) {
   if constexpr (LN <= kPencilLog) {
     constexpr int TK = 1 << (kPencilLog - LN);
     if (ln == LN)
       hipLaunchKernelGGL((k_xinv<LN>), dim3((unsigned)((npairs + TK - 1) / TK)), dim3(kPencilThreads), 0, st, spec,
-                         phi, pitch, npairs, tw, gp);
+                         phi, pitch, npairs, tw, gp, run);
     else
-      launch_xinv<LN + 1>(ln, spec, phi, pitch, npairs, st, tw, gp);
+      launch_xinv<LN + 1>(ln, spec, phi, pitch, npairs, st, tw, gp, run);
   }
 }
 
@@ -768,11 +780,11 @@ void append_twiddles(std::vector<double2> &tw, int n) {
 }
 
 template <typename S, bool EXACT>
-void launch_gravint_t(evh_ctx *h, double dt) {
+void launch_gravint_t(evh_ctx *h, const StepCtl &c) {
   const GGeo g = make_ggeo(h);
   const int blocks = xcd_blocks(g.ntiles);
   hipLaunchKernelGGL((k_gravint<S, EXACT>), dim3(blocks), dim3(GT), 0, h->stream, h->kp, make_gparams(h), g,
-                     (S *)h->qbuf[h->cur], h->phi, dt, h->st, (S *)h->tbuf);
+                     (S *)h->qbuf[h->cur], h->phi, c, (S *)h->tbuf);
 }
 
 }  // namespace
@@ -882,10 +894,13 @@ void gravity_release(evh_ctx *h) {
   h->sin2 = h->rho_part = nullptr;
 }
 
-hipError_t launch_gravpotential(evh_ctx *h, double cosmo) {
+// c: the step's control block; in a run on the device (power-of-two grids only) the
+// passes do nothing once the run has stopped
+hipError_t launch_gravpotential(evh_ctx *h, double cosmo, const StepCtl &c) {
   const long long n = h->grid.n();
   const GParams gp = make_gparams(h);
   const bool f32 = h->cfg.precision == EVH_FP32_MIXED;
+  const RunSlot *run = c.in ? c.out : nullptr;
   // The mean density only sets the (0,0,0) mode of the source, which the
   // Green's function zeroes; it keeps the transform's input small.  The
   // x pass of this library's transforms sums the densities it reads, and a
@@ -895,15 +910,15 @@ hipError_t launch_gravpotential(evh_ctx *h, double cosmo) {
   const bool reuse = h->xyz_pencils && h->rho_sums_valid;
   if (!gp.supercomoving && reuse) {
     hipLaunchKernelGGL(k_rho_mean_from, dim3(1), dim3(kSumBlocks), 0, h->stream, h->rho_sums, h->rho_nsums, gp.n3,
-                       h->rho_part);
+                       h->rho_part, run);
   } else if (!gp.supercomoving) {
     if (f32)
       hipLaunchKernelGGL(k_rho_partials<float>, dim3(kSumBlocks), dim3(256), 0, h->stream,
-                         (const float *)h->qbuf[h->cur], n, h->rho_part);
+                         (const float *)h->qbuf[h->cur], n, h->rho_part, run);
     else
       hipLaunchKernelGGL(k_rho_partials<double>, dim3(kSumBlocks), dim3(256), 0, h->stream,
-                         (const double *)h->qbuf[h->cur], n, h->rho_part);
-    hipLaunchKernelGGL(k_rho_mean, dim3(1), dim3(kSumBlocks), 0, h->stream, h->rho_part, gp.n3);
+                         (const double *)h->qbuf[h->cur], n, h->rho_part, run);
+    hipLaunchKernelGGL(k_rho_mean, dim3(1), dim3(kSumBlocks), 0, h->stream, h->rho_part, gp.n3, run);
   }
   const double cosmo_grav = cosmo * gp.grav;
   const int nx = h->grid.nx, ny = h->grid.ny, nz = h->grid.nz, nxh = nx / 2 + 1;
@@ -918,15 +933,15 @@ hipError_t launch_gravpotential(evh_ctx *h, double cosmo) {
     while ((1 << lnx) < nx) lnx++;
     if (f32)
       launch_xfwd<float>(lnx, (const float *)h->qbuf[h->cur], spec, h->spec_pitch, npairs, h->stream, twx, gp,
-                         cosmo_grav, h->rho_part, h->rho_sums);
+                         cosmo_grav, h->rho_part, h->rho_sums, run);
     else
       launch_xfwd<double>(lnx, (const double *)h->qbuf[h->cur], spec, h->spec_pitch, npairs, h->stream, twx, gp,
-                          cosmo_grav, h->rho_part, h->rho_sums);
+                          cosmo_grav, h->rho_part, h->rho_sums, run);
     h->rho_sums_valid = !gp.supercomoving;
-    launch_pencils<kPencilFwdY>(py, nz, h->stream, spec, twy, h->sin2, gp, nx, ny, nz);
-    launch_pencils<kPencilGreenZ>(pz, ny, h->stream, spec, twz, h->sin2, gp, nx, ny, nz);
-    launch_pencils<kPencilInvY>(py, nz, h->stream, spec, twy, h->sin2, gp, nx, ny, nz);
-    launch_xinv(lnx, spec, h->phi, h->spec_pitch, npairs, h->stream, twx, gp);
+    launch_pencils<kPencilFwdY>(py, nz, h->stream, spec, twy, h->sin2, gp, nx, ny, nz, run);
+    launch_pencils<kPencilGreenZ>(pz, ny, h->stream, spec, twz, h->sin2, gp, nx, ny, nz, run);
+    launch_pencils<kPencilInvY>(py, nz, h->stream, spec, twy, h->sin2, gp, nx, ny, nz, run);
+    launch_xinv(lnx, spec, h->phi, h->spec_pitch, npairs, h->stream, twx, gp, run);
     return hipGetLastError();
   }
   if (f32)
@@ -943,7 +958,7 @@ hipError_t launch_gravpotential(evh_ctx *h, double cosmo) {
   if (h->pencils) {
     const Pencils pz = make_pencils(nz, nxh, h->spec_plane, h->spec_pitch);
     launch_pencils<kPencilGreenZ>(pz, ny, h->stream, (double2 *)h->spec, (const double2 *)h->twiddle, h->sin2, gp,
-                                  nx, ny, nz);
+                                  nx, ny, nz, run);
   } else {
     const long long nspec = (long long)nxh * ny * nz;
     hipLaunchKernelGGL(k_green, dim3(grid_of(nspec)), dim3(256), 0, h->stream, (double2 *)h->spec, nx, ny, nz,
@@ -954,11 +969,11 @@ hipError_t launch_gravpotential(evh_ctx *h, double cosmo) {
 }
 
 // the caller resets the CFL minimum before
-hipError_t launch_gravintegration(evh_ctx *h, double dt) {
+hipError_t launch_gravintegration(evh_ctx *h, const StepCtl &c) {
   const bool exact = h->mode != EVH_MODE_FUSED && h->cfg.precision == EVH_FP64;
-  if (h->cfg.precision == EVH_FP32_MIXED) launch_gravint_t<float, false>(h, dt);
-  else if (exact) launch_gravint_t<double, true>(h, dt);
-  else launch_gravint_t<double, false>(h, dt);
+  if (h->cfg.precision == EVH_FP32_MIXED) launch_gravint_t<float, false>(h, c);
+  else if (exact) launch_gravint_t<double, true>(h, c);
+  else launch_gravint_t<double, false>(h, c);
   return hipGetLastError();
 }
 

@@ -59,6 +59,11 @@ __host__ __device__ __forceinline__ const KParams::Single &consts(const KParams 
 __device__ __forceinline__ float uniform(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
+__device__ __forceinline__ double uniform_value(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
 __device__ __forceinline__ double uniform(double v) { return v; }  // FP64 kernels have no scalar registers to spare
 
 // Device status block: first error (code, linear cell) and min reductions.
