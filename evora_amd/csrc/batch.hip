@@ -45,8 +45,12 @@ struct BoxDev {
   int pad;
 };
 
+// The counters lie on cache lines of their own: the blocks of each XCD take
+// their items from one, and meet at the others only when it is drained.
 struct Queues {
-  unsigned next[kXcds];  // items taken from each XCD's queue
+  struct alignas(128) Count {
+    unsigned next;  // items taken from this XCD's queue
+  } count[kXcds];
   int start[kXcds + 1];  // queue j covers items [start[j], start[j+1])
 };
 
@@ -58,12 +62,16 @@ struct BoxState {
   Status *st;  // per-box status: errors, CFL minimum
 };
 
-__device__ __forceinline__ int take_item(Queues *qs, int xcd) {
-  for (int i = 0; i < kXcds; i++) {
-    const int j = (xcd + i) % kXcds;
+// The next item of a block: from its own XCD's queue, then from the others';
+// `from` counts the queues it has found drained.  Device-wide, not
+// system-wide atomics, and no look before the increment: an item took 54 ns of
+// everybody's time before (35 M cells in 24 boxes, 4-plane items, FP32-mixed:
+// 3.9 ms per step).
+__device__ __forceinline__ int take_item(Queues *qs, int xcd, int &from) {
+  for (; from < kXcds; from++) {
+    const int j = (xcd + from) % kXcds;
     const int len = qs->start[j + 1] - qs->start[j];
-    if ((int)__atomic_load_n(&qs->next[j], __ATOMIC_RELAXED) >= len) continue;
-    const int idx = (int)atomicAdd(&qs->next[j], 1u);
+    const int idx = (int)__hip_atomic_fetch_add(&qs->count[j].next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (idx < len) return qs->start[j] + idx;
   }
   return -1;
@@ -86,12 +94,18 @@ __global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((
   __shared__ core::Smem<T, TX, TY> sm;
   __shared__ int s_item;
   const int xcd = blockIdx.x % kXcds;
+  int from = 0;                 // thread 0's
+  int b = -1, lo = 0, hi = 0;   // the box of the last item and its items [lo, hi): mostly the next one's too
   for (;;) {
-    if (threadIdx.x == 0) s_item = take_item(qs, xcd);
+    if (threadIdx.x == 0) s_item = take_item(qs, xcd, from);
     __syncthreads();
-    const int item = s_item;
+    const int item = __builtin_amdgcn_readfirstlane(s_item);
     if (item < 0) break;  // every queue drained: the whole block leaves
-    const int b = box_of(boxes, nbox, item);
+    if (item < lo || item >= hi) {
+      b = box_of(boxes, nbox, item);
+      lo = boxes[b].tile0;
+      hi = lo + boxes[b].G.ntiles;
+    }
     if (bs.active[b]) {
       // k_batch_dt has flipped the side of every box that steps: the new
       // state goes to that buffer, the current one is read from the other
@@ -100,7 +114,7 @@ __global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((
       const Geo G = bx.G;
       const bool to1 = bs.side[b] != 0;
       core::march<T, S, SOLVER, LIMITER, TX, TY, false>(P, G, to1 ? q0 : q1, to1 ? q1 : q0, bx.qoff, b, bs.dt[b],
-                                                    &bs.st[b], &bs.st[b], item - bx.tile0, sm);
+                                                    &bs.st[b], &bs.st[b], item - lo, sm);
     }
     __syncthreads();  // s_item is rewritten only after every lane has used it
   }
@@ -109,7 +123,7 @@ __global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((
 #if EVH_FUSED_PREC == 64
 __global__ void k_batch_dt(int nbox, BoxState bs, Queues *qs) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (blockIdx.x == 0 && threadIdx.x < kXcds) qs->next[threadIdx.x] = 0;
+  if (blockIdx.x == 0 && threadIdx.x < kXcds) qs->count[threadIdx.x].next = 0;
   if (b >= nbox) return;
   Status &s = bs.st[b];
   bs.active[b] = 0;
@@ -142,20 +156,26 @@ __global__ void k_batch_dt(int nbox, BoxState bs, Queues *qs) {
   s.vmin_bits = (unsigned long long)__double_as_longlong(1e6);  // timestep.f90:35
 }
 
-// exact primitive + CFL of one box (first step after an upload)
+// exact primitive + CFL of boxes box0 + blockIdx.y that are running (their
+// first step after an upload, or of a call)
 template <typename S>
-__global__ void __launch_bounds__(256) k_batch_cfl(KParams P, long long n, const S *__restrict__ q, Status *st) {
+__global__ void __launch_bounds__(256) k_batch_cfl(const BoxDev *__restrict__ boxes, int box0,
+                                                   const S *__restrict__ q0, const S *__restrict__ q1, BoxState bs) {
+  const int b = box0 + blockIdx.y;
+  if (!bs.go[b]) return;  // the same in the whole block
+  const KParams P = boxes[b].P;
+  const long long n = boxes[b].G.n;
+  const S *__restrict__ q = (bs.side[b] ? q1 : q0) + boxes[b].qoff;
   double vmin = 1e6;
   for (long long c = blockIdx.x * 256LL + threadIdx.x; c < n; c += (long long)gridDim.x * 256) {
     double qc[6], wc[5];
 #pragma unroll
     for (int m = 0; m < 6; m++) qc[m] = double(q[m * n + c]);
     const int e = q2w(P, qc, wc);
-    if (e) report_next(st, e, (unsigned long long)c);
+    if (e) report_next(&bs.st[b], e, (unsigned long long)c);
     vmin = dmin(vmin, cfl_cell(P, wc));
   }
-  for (int off = 32; off > 0; off >>= 1) vmin = dmin(vmin, __shfl_xor(vmin, off));
-  if ((threadIdx.x & 63) == 0) atomic_min_pos(&st->vmin_bits, vmin);
+  block_min_pos<256>(&bs.st[b].vmin_bits, vmin);
 }
 #endif
 
@@ -242,6 +262,7 @@ struct evh_batch {
   std::vector<char> cfl_needed;
   // launch shape
   int tile_ty = 12, wpe_hi = 1, zchunk = 64, blocks_per_cu = 2;
+  bool auto_chunk = true;  // no z chunk set: by the boxes (batch_chunk)
   int tx = 16, ty = 12;  // the column tile that tile_ty stands for (pick_tile)
   // one step of the ensemble, captured once (the kernels read each box's
   // buffer side from device memory)
@@ -300,14 +321,25 @@ __global__ void k_b_soa_to_aos(const S *__restrict__ src, double *__restrict__ d
     for (int m = 0; m < 6; m++) dst[6 * c + m] = double(src[m * n + base + c]);
 }
 
-__global__ void k_b_reset_status(Status *st, int box) {
-  if (threadIdx.x == 0) {
-    st[box].code = 0;
-    st[box].cell = 0;
-    st[box].next_code = 0;
-    st[box].next_cell = 0;
-    st[box].vmin_bits = (unsigned long long)__double_as_longlong(1e6);
-  }
+__global__ void k_b_reset_status(Status *st, int box0, int n) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < n) clear_status(st + box0 + b);
+}
+
+// the CFL limits of the running ones of n boxes from box0 on, in one launch
+hipError_t launch_batch_cfl(bool f32, const BoxDev *boxes, int box0, int n, long long max_cells, const void *q0,
+                            const void *q1, const BoxState &bs, hipStream_t stream) {
+  hipLaunchKernelGGL(k_b_reset_status, dim3((n + 63) / 64), dim3(64), 0, stream, bs.st, box0, n);
+  // about 2048 blocks in all: each ends with an atomic on its box's limit
+  const long long per = std::max(1LL, std::min((max_cells + 255) / 256, std::max(2048LL / n, 64LL)));
+  const dim3 grid((unsigned)per, (unsigned)n);
+  if (f32)
+    hipLaunchKernelGGL(k_batch_cfl<float>, grid, dim3(256), 0, stream, boxes, box0, (const float *)q0,
+                       (const float *)q1, bs);
+  else
+    hipLaunchKernelGGL(k_batch_cfl<double>, grid, dim3(256), 0, stream, boxes, box0, (const double *)q0,
+                       (const double *)q1, bs);
+  return hipGetLastError();
 }
 
 int gridsz(long long work) {
@@ -329,6 +361,22 @@ void pick_tile(const evh_config *cfgs, int nbox, int tile_ty, int *tx, int *ty) 
   if (wide_tile(n32, n16)) {
     *tx = 32;
     *ty = 6;
+  }
+}
+
+// z planes per item when the tuning leaves them open: 64, halved while the
+// boxes together give fewer than six items for each of the `slots` resident
+// blocks (the last ones to finish leave the others idle), and below 8 only
+// while there is less than one.  Measured, FP32-mixed, 24 boxes of 64 to 192
+// (35 M cells): 0.94 ms per step with 32 planes, 0.98 with 64 and 1.09 with 128;
+// 32 boxes of 16 to 48: FP64 0.106 ms with 8 and 0.174 with 64, FP32-mixed 0.063
+// with 4 and 0.151 with 64.
+int batch_chunk(const evh_config *cfgs, int nbox, int tx, int ty, int slots) {
+  int zc = 64;
+  for (;; zc /= 2) {
+    long long items = 0;
+    for (int i = 0; i < nbox; i++) items += tiles_of(cfgs[i].nx, cfgs[i].ny, tx, ty) * ((cfgs[i].nz + zc - 1) / zc);
+    if (zc == 4 || items >= 6LL * slots || (zc <= 8 && items >= slots)) return zc;
   }
 }
 
@@ -368,8 +416,10 @@ int rebuild_items(evh_batch *b) {
   std::vector<BoxDev> h(b->nbox);
   Queues q;
   pick_tile(b->cfgs.data(), b->nbox, b->tile_ty, &b->tx, &b->ty);
+  const int zc = b->auto_chunk ? batch_chunk(b->cfgs.data(), b->nbox, b->tx, b->ty, b->blocks_per_cu * b->num_cu)
+                               : b->zchunk;
   b->nitems = describe_boxes(b->cfgs.data(), b->kps.data(), b->ncell.data(), b->qoff.data(), b->nbox, b->tx, b->ty,
-                             b->zchunk, h.data(), &q);
+                             zc, h.data(), &q);
   BHIP(hipMemcpy(b->boxes_d, h.data(), sizeof(BoxDev) * b->nbox, hipMemcpyHostToDevice));
   BHIP(hipMemcpy(b->qs_d, &q, sizeof(Queues), hipMemcpyHostToDevice));
   if (b->gexec) {
@@ -420,17 +470,10 @@ int refresh_sides(evh_batch *b) {
 int prepare(evh_batch *b) {
   for (int i = 0; i < b->nbox; i++) {
     if (!b->cfl_needed[i]) continue;
-    hipLaunchKernelGGL(k_b_reset_status, dim3(1), dim3(64), 0, b->stream, b->bs.st, i);
-    const long long n = b->ncell[i];
-    if (b->precision == EVH_FP32_MIXED)
-      hipLaunchKernelGGL(k_batch_cfl<float>, dim3(gridsz(n)), dim3(256), 0, b->stream, b->kps[i], n,
-                         (const float *)box_q(b, i), b->bs.st + i);
-    else
-      hipLaunchKernelGGL(k_batch_cfl<double>, dim3(gridsz(n)), dim3(256), 0, b->stream, b->kps[i], n,
-                         (const double *)box_q(b, i), b->bs.st + i);
-    BHIP(hipGetLastError());
     const int one = 1;
     BHIP(hipMemcpyAsync(b->bs.go + i, &one, sizeof(int), hipMemcpyHostToDevice, b->stream));
+    BHIP(launch_batch_cfl(b->precision == EVH_FP32_MIXED, b->boxes_d, i, 1, b->ncell[i], b->qbuf[0], b->qbuf[1], b->bs,
+                          b->stream));
     b->cfl_needed[i] = 0;
   }
   BHIP(hipStreamSynchronize(b->stream));
@@ -690,6 +733,7 @@ int evh_batch_set_tuning(evh_batch *b, int tile_ty, int wpe_hi, int zchunk, int 
   b->tile_ty = tile_ty;
   b->wpe_hi = wpe_hi;
   b->zchunk = zchunk;
+  b->auto_chunk = false;
   b->blocks_per_cu = blocks_per_cu;
   return rebuild_items(b);
 }
@@ -709,30 +753,30 @@ int evh_batch_autotune(evh_batch *b, int trial_steps, char *log, int loglen) {
   if (r) return r;
   Snapshot snap;
   if ((r = save_state(b, snap))) return r;
-  const int tys[] = {8, 12}, zcs[] = {32, 64, 128}, bpcs[] = {1, 2, 3, 4};
+  const int tys[] = {8, 12}, zcs[] = {4, 8, 16, 32, 64, 128}, bpcs[] = {1, 2, 3, 4};
   double best = 1e300;
   int bt[4] = {b->tile_ty, b->wpe_hi, b->zchunk, b->blocks_per_cu};
   std::string text = "# batch autotune: nbox=" + std::to_string(b->nbox) + " cells=" + std::to_string(b->total) +
                      " trial_steps=" + std::to_string(trial_steps) + "\n";
   for (int ty : tys)
-    for (int hi = 0; hi <= 1; hi++)
-      for (int zc : zcs)
-        for (int bpc : bpcs) {
-          if ((r = evh_batch_set_tuning(b, ty, hi, zc, bpc))) return r;
-          if ((r = restore_state(b, snap))) return r;
-          float ms = 0.f;
-          if ((r = evh_batch_run(b, 1, 0, &ms))) return r;  // warm-up step
-          if ((r = evh_batch_run(b, trial_steps, 0, &ms))) return r;
-          const double per = ms / trial_steps;
-          char line[160];
-          std::snprintf(line, sizeof line, "tile_ty=%d wpe_hi=%d zchunk=%d blocks_per_cu=%d ms_per_step=%.4f\n", ty, hi,
-                        zc, bpc, per);
-          text += line;
-          if (per < best) {
-            best = per;
-            bt[0] = ty; bt[1] = hi; bt[2] = zc; bt[3] = bpc;
-          }
+    for (int zc : zcs)
+      for (int bpc : bpcs) {
+        const int hi = 1;  // one register budget either way
+        if ((r = evh_batch_set_tuning(b, ty, hi, zc, bpc))) return r;
+        if ((r = restore_state(b, snap))) return r;
+        float ms = 0.f;
+        if ((r = evh_batch_run(b, 1, 0, &ms))) return r;  // warm-up step
+        if ((r = evh_batch_run(b, trial_steps, 0, &ms))) return r;
+        const double per = ms / trial_steps;
+        char line[160];
+        std::snprintf(line, sizeof line, "tile_ty=%d wpe_hi=%d zchunk=%d blocks_per_cu=%d ms_per_step=%.4f\n", ty, hi, zc,
+                      bpc, per);
+        text += line;
+        if (per < best) {
+          best = per;
+          bt[0] = ty; bt[1] = hi; bt[2] = zc; bt[3] = bpc;
         }
+      }
   char line[160];
   std::snprintf(line, sizeof line, "best: tile_ty=%d wpe_hi=%d zchunk=%d blocks_per_cu=%d ms_per_step=%.4f\n", bt[0],
                 bt[1], bt[2], bt[3], best);
@@ -847,9 +891,14 @@ int evh_batch_run_noalloc(const evh_config *cfgs, int nbox, void *q0, void *q1, 
     off += ncell[i];
   }
   // the launch shape evh_batch_create starts with
-  const int zc = 64, bpc = f32 ? 4 : 2;
+  int devid = 0, cu = 256;
+  if ((e = hipGetDevice(&devid)) == hipSuccess)
+    e = hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, devid);
+  if (e != hipSuccess) return na_fail(err, errlen, EVH_ERR_HIP, hipGetErrorString(e));
+  const int bpc = f32 ? 4 : 2;
   int tx, ty;
   pick_tile(cfgs, nbox, 12, &tx, &ty);
+  const int zc = batch_chunk(cfgs, nbox, tx, ty, bpc * cu);
   describe_boxes(cfgs, kps, ncell, qoff, nbox, tx, ty, zc, img.boxes, &img.qs);
   for (int i = 0; i < nbox; i++) {
     img.t[i] = t[i];
@@ -872,23 +921,11 @@ int evh_batch_run_noalloc(const evh_config *cfgs, int nbox, void *q0, void *q1, 
   bs.err_step = dev->err_step;
   bs.side = dev->side;
   bs.st = dev->st;
-  int devid = 0, cu = 256;
-  if ((e = hipGetDevice(&devid)) == hipSuccess)
-    e = hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, devid);
   if (e == hipSuccess) e = hipMemcpy(dev, &img, sizeof img, hipMemcpyHostToDevice);
   // the first CFL limit of every running box from its current state
-  for (int i = 0; i < nbox && e == hipSuccess; i++) {
-    if (!img.go[i]) continue;
-    hipLaunchKernelGGL(k_b_reset_status, dim3(1), dim3(64), 0, 0, bs.st, i);
-    const long long n = ncell[i];
-    if (f32)
-      hipLaunchKernelGGL(k_batch_cfl<float>, dim3(gridsz(n)), dim3(256), 0, 0, kps[i], n,
-                         (const float *)(side[i] ? q1 : q0) + 6 * qoff[i], bs.st + i);
-    else
-      hipLaunchKernelGGL(k_batch_cfl<double>, dim3(gridsz(n)), dim3(256), 0, 0, kps[i], n,
-                         (const double *)(side[i] ? q1 : q0) + 6 * qoff[i], bs.st + i);
-    e = hipGetLastError();
-  }
+  long long most = 0;
+  for (int i = 0; i < nbox; i++) most = ncell[i] > most ? ncell[i] : most;
+  if (e == hipSuccess) e = launch_batch_cfl(f32, dev->boxes, 0, nbox, most, q0, q1, bs, 0);
   const evh_config &c0 = cfgs[0];
   for (int k = 0; k < nsteps && e == hipSuccess; k++) {
     hipLaunchKernelGGL(k_batch_dt, dim3((nbox + 255) / 256), dim3(256), 0, 0, nbox, bs, &dev->qs);

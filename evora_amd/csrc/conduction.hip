@@ -260,14 +260,9 @@ __global__ void __launch_bounds__(CT) k_conduct(KParams P, CGeo G, S *__restrict
     tm = tc;
     tc = tn;
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    vmin = dmin(vmin, __shfl_xor(vmin, off));
-    tvmin = dmin(tvmin, __shfl_xor(tvmin, off));
-  }
-  if ((tid & 63) == 0) {
-    atomic_min_pos(&C.lim->vmin_bits, vmin);
-    atomic_min_pos(&C.lim->tvmin_bits, tvmin);
-  }
+  block_min_pos<CT>(&C.lim->vmin_bits, vmin);
+  __syncthreads();  // the same LDS again
+  block_min_pos<CT>(&C.lim->tvmin_bits, tvmin);
 }
 
 // T of every cell of q (the state did not come out of a fused sweep)
@@ -293,8 +288,7 @@ __global__ void __launch_bounds__(256) k_thermal_min(KParams P, long long n, con
     if (e) report_next(st, e, (unsigned long long)c);
     v = dmin(v, tv);
   }
-  for (int off = 32; off > 0; off >>= 1) v = dmin(v, __shfl_xor(v, off));
-  if ((threadIdx.x & 63) == 0) atomic_min_pos(&st->tvmin_bits, v);
+  block_min_pos<256>(&st->tvmin_bits, v);
 }
 
 __global__ void k_reset_tv(Status *st) {
@@ -330,7 +324,7 @@ template <typename S>
 void launch_thermal_min_s(evh_ctx *h) {
   hipLaunchKernelGGL(k_reset_tv, dim3(1), dim3(64), 0, h->stream, h->st);
   const long long n = h->grid.n();
-  const long long b = std::min((n + 255) / 256, 8192LL);
+  const long long b = std::min((n + 255) / 256, 2048LL);
   hipLaunchKernelGGL(k_thermal_min<S>, dim3((int)b), dim3(256), 0, h->stream, h->kp, n, (const S *)h->qbuf[h->cur],
                      h->st);
 }

@@ -73,8 +73,7 @@ __global__ void __launch_bounds__(256) k_cfl(KParams P, Geo G, const S *__restri
     if (e) report_next(st, e, (unsigned long long)c);
     vmin = dmin(vmin, cfl_cell(P, wc));
   }
-  for (int off = 32; off > 0; off >>= 1) vmin = dmin(vmin, __shfl_xor(vmin, off));
-  if ((threadIdx.x & 63) == 0) atomic_min_pos(&st->vmin_bits, vmin);
+  block_min_pos<256>(&st->vmin_bits, vmin);
 }
 
 Geo make_geo(const evh_ctx *h, int tx, int ty) {
@@ -175,7 +174,7 @@ bool fused_supported(const evh_config &c) { return c.nx >= 2 && c.ny >= 2 && c.n
 hipError_t launch_cfl(evh_ctx *h) {
   const Geo g = make_geo(h, 16, 12);
   long long b = (g.n + 255) / 256;
-  if (b > 8192) b = 8192;
+  if (b > 2048) b = 2048;
   if (h->cfg.precision == EVH_FP32_MIXED)
     hipLaunchKernelGGL(k_cfl<float>, dim3((int)b), dim3(256), 0, h->stream, h->kp, g, (const float *)h->qbuf[h->cur],
                        h->st);

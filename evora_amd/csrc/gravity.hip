@@ -655,8 +655,7 @@ __global__ void __launch_bounds__(GT) k_gravint(KParams P, GParams Gp, GGeo G, S
     pm = pc;
     pc = pn;
   }
-  for (int off = 32; off > 0; off >>= 1) vmin = dmin(vmin, __shfl_xor(vmin, off));
-  if ((tid & 63) == 0) atomic_min_pos(&C.lim->vmin_bits, vmin);
+  block_min_pos<GT>(&C.lim->vmin_bits, vmin);
 }
 
 GParams make_gparams(const evh_ctx *h) {

@@ -260,8 +260,7 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
     if (nerr) report_next(lim, nerr, (unsigned long long)(ex + G.nx * (long long)nerr_k));
   }
   if constexpr (kSpeedKey) vmin = fm::rcp(-vmin);
-  for (int off = 32; off > 0; off >>= 1) vmin = dmin(vmin, __shfl_xor(vmin, off));
-  if ((l & 63) == 0) atomic_min_pos(&lim->vmin_bits, vmin);
+  block_min_pos<NL>(&lim->vmin_bits, vmin);
 }
 
 }  // namespace core2d

@@ -96,6 +96,23 @@ __device__ __forceinline__ T dmin(T a, T b) { return a < b ? a : b; }
 template <typename T>
 __device__ __forceinline__ T dmax(T a, T b) { return a > b ? a : b; }
 
+// The minimum of a block's positive values into *a, with one atomic per block:
+// all blocks meet at one address, which takes about 10 ns each, so one per
+// wave made the limit of a 64 M-cell state wait for 33,000 of them (0.3 ms).
+// Every lane of the block's NT calls it, once per launch.
+template <int NT>
+__device__ __forceinline__ void block_min_pos(unsigned long long *a, double v) {
+  __shared__ double sh[NT / 64];
+  for (int off = 32; off > 0; off >>= 1) v = dmin(v, __shfl_xor(v, off));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int i = 1; i < NT / 64; i++) v = dmin(v, sh[i]);
+    atomic_min_pos(a, v);
+  }
+}
+
 // ---------------------------------------------------------------- comp.f90:45-85
 // pressure(q, press); q may be rewritten when dualenergy is on.
 template <typename T>

@@ -99,9 +99,7 @@ __global__ void __launch_bounds__(kBlock) k_hydrostep(KParams P, Grid G, const d
     for (int m = 0; m < 5; m++) wc[m] = w[m * nw + wi];
     v = dmin(v, cfl_cell(P, wc));
   }
-  // wavefront min, then one atomic per wavefront
-  for (int off = 32; off > 0; off >>= 1) v = dmin(v, __shfl_xor(v, off));
-  if ((threadIdx.x & 63) == 0) atomic_min_pos(&st->vmin_bits, v);
+  block_min_pos<kBlock>(&st->vmin_bits, v);
 }
 
 // ------------------------------------------------------------ compevo (muscl.f90:45-113)
