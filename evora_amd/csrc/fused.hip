@@ -84,7 +84,9 @@ Geo make_geo(const evh_ctx *h, int tx, int ty) {
   g.n = h->grid.n();
   g.tiles_x = (g.nx + tx - 1) / tx;
   g.tiles_y = (g.ny + ty - 1) / ty;
-  g.zchunk = h->zchunk > 0 ? h->zchunk : z_chunk((long long)g.tiles_x * g.tiles_y, g.nz, 64);
+  g.zchunk = h->zchunk > 0 ? h->zchunk
+                           : march_chunk(h->cfg.precision == EVH_FP32_MIXED ? kMarch32 : kMarch64,
+                                         (long long)g.tiles_x * g.tiles_y, g.nz, 128);
   if (g.zchunk > g.nz) g.zchunk = g.nz;
   g.nchunks = (g.nz + g.zchunk - 1) / g.zchunk;
   g.ntiles = g.tiles_x * g.tiles_y * g.nchunks;
@@ -102,7 +104,7 @@ void launch_ty(evh_ctx *h, const StepCtl &c) {
                      (S *)h->tbuf);
 }
 
-// the 2-D form: strips of 252 columns, chunks of up to 32 rows (the z chunk
+// the 2-D form: strips of 252 columns, chunks of up to 64 rows (the z chunk
 // of the tuning, when set), WPE waves per SIMD
 template <typename T, typename S, int SOLVER, int LIMITER, int WPE>
 void launch_2d(evh_ctx *h, const StepCtl &c) {
@@ -111,9 +113,7 @@ void launch_2d(evh_ctx *h, const StepCtl &c) {
   g.ny = h->grid.ny;
   g.n = h->grid.n();
   g.strips = (g.nx + core2d::NC - 1) / core2d::NC;
-  // 32 rows measured fastest at 8192^2 (FP64 2.10 ms against 2.14 with 64 and
-  // 2.27 with 128; FP32-mixed 0.94 with 32 or 64)
-  g.ychunk = h->zchunk > 0 ? h->zchunk : y_chunk(g.strips, g.ny, 32);
+  g.ychunk = h->zchunk > 0 ? h->zchunk : march_chunk(sizeof(T) == 4 ? kMarch2d32 : kMarch2d64, g.strips, g.ny, 64);
   if (g.ychunk > g.ny) g.ychunk = g.ny;
   g.nchunks = (g.ny + g.ychunk - 1) / g.ychunk;
   g.ntiles = g.strips * g.nchunks;

@@ -7,16 +7,16 @@
 // Lane l holds column x0 + l - 2, so lanes 0-1 and 254-255 hold the two
 // ghost columns on either side; the ghost rules of `bound` (boundary.f90)
 // are folded into the load index.  Per row k:
-//   S1  primitive of row k+1 (its raw q was loaded one row ahead); w of row
-//       k to LDS;
-//   S2  limited slopes in x (LDS neighbours) and y (rows k-1, k, k+1 in
+//   S1  w of row k to LDS;
+//   S2  primitive of row k+1 (its raw q was loaded one row ahead); limited slopes in x (LDS neighbours) and y (rows k-1, k, k+1 in
 //       registers), the 2-D predictor, the two states of every x face to
 //       LDS; the y face k-1/2 is solved from the top state of row k-1
 //       (carried) and the bottom state of row k, and row k-1 is finished as
-//       (q + dtx*(Fx)) + dty*(Fy), the reference's x, y order, and stored;
+//       (q + dtx*(Fx)) + dty*(Fy), the reference's x, y order, and stored,
+//       with the primitive and CFL limit of the cells that can change the
+//       minimum (and, with conduction, the temperature of all);
 //   S3  the x faces of row k, one per lane;
-//   S4  q(k) + dtx*(Fx) of row k, carried to row k+1; the primitive and CFL
-//       limit of the stored row k-1 (and its temperature, with conduction).
+//   S4  q(k) + dtx*(Fx) of row k, carried to row k+1.
 // Every lane does useful work in every stage except the four ghost lanes in
 // the solves and updates, and a cell takes two Riemann solves.
 #pragma once
@@ -111,12 +111,8 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
   // carried from row k-1: its partial update q + dtx*(Fx), the flux of its
   // bottom face, its top face state (the last two in LDS with LC)
   T part[6], fyb[LC ? 1 : 6], ytop[LC ? 1 : 5];
-  constexpr bool kSpeedKey = !EXACT && sizeof(T) == 8;
-  double vmin = kSpeedKey ? -1e-6 : 1e6;
+  core::CflMin<T, EXACT> cfl;
   int err = 0, err_k = 0, nerr = 0, nerr_k = 0;
-  T o[6];
-  bool pend = false;
-  long long oc = 0;
 
   S pre[6];
   const long long cx = col_off(P, G, gx);
@@ -143,14 +139,16 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
 
   for (int k = y0 - 1; k <= y1; k++) {
     const bool out_row = k >= y0 && k < y1;
-    // ---- S1: primitive of row k+1; w of row k to LDS
-    prim2<EXACT>(P, G, pre, gx, qn, wp, rp);
-    fetch2(G, qin, cx + row_off(P, G, k + 2), pre);
+    bool raise = false;
+    // ---- S1: w of row k to LDS
 #pragma unroll
     for (int m = 0; m < 5; m++) W[m][l] = wc[m];
     __syncthreads();
 
-    // ---- S2: slopes, predictor, face states; the y face k-1/2
+    // ---- S2: primitive of row k+1; slopes, predictor, face states; the y
+    // face k-1/2
+    prim2<EXACT>(P, G, pre, gx, qn, wp, rp);
+    fetch2(G, qin, cx + row_off(P, G, k + 2), pre);
     if (slopes) {
       T sx[5], sy[5], ev[5];
 #pragma unroll
@@ -189,15 +187,24 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
           const int e = Ph::template riemann<SOLVER, 2>(P, yt0, yb, fy);
           if (e && inside && !err) { err = e; err_k = k; }
           if (k - 1 >= y0 && inside) {
+            T o[6];
 #pragma unroll
             for (int m = 0; m < 6; m++) {
               if constexpr (LC) o[m] = Ph::mad(dty, sm.F[m][l] - fy[m], part[m]);
               else o[m] = Ph::mad(dty, fyb[m] - fy[m], part[m]);
             }
-            oc = (long long)gx + (long long)G.nx * (k - 1);
+            const long long oc = (long long)gx + (long long)G.nx * (k - 1);
 #pragma unroll
             for (int m = 0; m < 6; m++) qout[m * G.n + oc] = S(o[m]);
-            pend = true;
+            // the limits of the new state, for the cells that can change them
+            if (tout || !core::slower(P, o, cfl.thr)) {
+              T wn[5], rn;
+              const int ep = Ph::q2w(P, o, wn, rn);
+              if (ep && !nerr) { nerr = ep; nerr_k = k - 1; }
+              cfl.add(P, wn, rn);
+              if (tout) tout[oc] = S(Ph::temp(P, wn, rn));
+              raise = !tout;
+            }
           }
 #pragma unroll
           for (int m = 0; m < 6; m++) {
@@ -212,6 +219,7 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
         }
       }
     }
+    if (__builtin_amdgcn_ballot_w64(raise)) cfl.raise();
     __syncthreads();
 
     // ---- S3: the x face (l, l+1) of row k
@@ -229,21 +237,10 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
     }
     __syncthreads();
 
-    // ---- S4: q(k) + dtx*(Fx) of row k; the end of row k-1
+    // ---- S4: q(k) + dtx*(Fx) of row k, carried to row k+1
     if (out_row && inner) {
 #pragma unroll
       for (int m = 0; m < 6; m++) part[m] = Ph::mad(dtx, XB[m][l - 1] - XB[m][l], qc[m]);
-    }
-    if (pend) {
-      T on[6], wn[5], rn;
-#pragma unroll
-      for (int m = 0; m < 6; m++) on[m] = T(S(o[m]));
-      const int ep = Ph::q2w(P, on, wn, rn);
-      if (ep && !nerr) { nerr = ep; nerr_k = k - 1; }
-      if constexpr (kSpeedKey) vmin = dmin(vmin, -fast::cfl_speed(P, wn, rn));
-      else vmin = dmin(vmin, Ph::cfl_cell(P, wn, rn));
-      if (tout) tout[oc] = S(Ph::temp(P, wn, rn));
-      pend = false;
     }
     // rotate the column window
 #pragma unroll
@@ -259,8 +256,7 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
     if (err) report(st, err, (unsigned long long)(ex + G.nx * (long long)err_k));
     if (nerr) report_next(lim, nerr, (unsigned long long)(ex + G.nx * (long long)nerr_k));
   }
-  if constexpr (kSpeedKey) vmin = fm::rcp(-vmin);
-  block_min_pos<NL>(&lim->vmin_bits, vmin);
+  block_min_pos<NL>(&lim->vmin_bits, cfl.wave_min());
 }
 
 }  // namespace core2d

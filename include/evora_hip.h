@@ -176,8 +176,7 @@ int evh_synchronize(evh_ctx *h);
  * 16 x 12 or, in FP32-mixed, 32 x 6 where that covers the grid as well),
  * occupancy target (0 or 1; kept for callers, both give the one register
  * budget compiled per precision), z planes per block (rows on 2-D grids; 0,
- * the default: 64 planes or 32 rows, halved down to 4 while the grid gives
- * too few blocks).  Invalid values are rejected.  A z-slab with halo buffers
+ * the default: up to 128 planes or 64 rows, fewer on small grids).  Invalid values are rejected.  A z-slab with halo buffers
  * (evh_slab) runs tile height 12; its z chunk is the tuning's.  The results
  * do not depend on the launch shape. */
 int evh_set_tuning(evh_ctx *h, int tile_ty, int wpe_hi, int zchunk);
