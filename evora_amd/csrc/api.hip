@@ -611,7 +611,7 @@ int evh_download_phi(evh_ctx *h, double *phi) {
   if (!h->phi_valid) return fail(h, EVH_ERR_STATE, "no potential yet");
   int r = check_status(h);
   if (r) return r;
-  HIP_TRY(hipMemcpy(phi, h->phi, sizeof(double) * h->grid.n(), hipMemcpyDeviceToHost));
+  HIP_TRY(h->xfer.download_doubles(phi, h->phi, h->grid.n(), h->stream));
   return EVH_OK;
 }
 
