@@ -88,7 +88,7 @@ __global__ void k_clear_statuses(Status *st, int n) {
 }
 
 __global__ void k_run_start(RunSlot *r, double t) {
-  if (threadIdx.x == 0) *r = RunSlot{t, 1e99, 1, 0, 0, 0};
+  if (threadIdx.x == 0) *r = RunSlot{t, 1e99, 1e99, 1, 0, 0, 0};
 }
 
 // AoS chunk (cells x 6, double) -> SoA storage at cell offset `base`
@@ -649,8 +649,16 @@ int evh_step(evh_ctx *h, double *t, double tend, double *dt, int *go) {
 static int run_on_device(evh_ctx *h, int nsteps, double *t, double tend, double *dt, int *done) {
   constexpr int kRunBatch = 64;
   const bool hydro = !h->cfg.hydro_off, grav = h->cfg.gravity, cond = h->cfg.conduction;
+  const bool line = h->mode == EVH_MODE_STAGED;  // 1-D: one kernel with the staged kernels' arithmetic
   int r;
-  if ((r = evh_primitive(h))) return r;
+  if (line) {
+    if ((r = ensure_staged_arrays(h))) return r;
+    HIP_TRY(launch_reset_status(h, false));
+    HIP_TRY(launch_primitive(h));
+    HIP_TRY(launch_hydrostep(h));
+  } else if ((r = evh_primitive(h))) {
+    return r;
+  }
   if (cond && !h->tv_valid) {
     HIP_TRY(launch_thermal_min(h));
     h->tv_valid = true;
@@ -675,7 +683,7 @@ static int run_on_device(evh_ctx *h, int nsteps, double *t, double tend, double 
       Status *const replaced = h->st_all + 3;  // limits that a later kernel of the step replaces
       if (hydro) {
         c.lim = grav || cond ? replaced : c.st;
-        HIP_TRY(launch_fused_step(h, c));
+        HIP_TRY(line ? launch_line_step(h, c) : launch_fused_step(h, c));
         h->cur = 1 - h->cur;
         c.head = 0;
       }
@@ -713,8 +721,25 @@ static int run_on_device(evh_ctx *h, int nsteps, double *t, double tend, double 
     h->rho_sums_valid = sums0;
   }
   *t = end.t;
-  *dt = end.dt;
   *done = end.done;
+  if (line) {
+    if (end.done > 0) {  // w, evo and s of the last step, from the state it started from
+      *dt = end.last;
+      h->cur = 1 - h->cur;
+      HIP_TRY(launch_primitive(h));
+      HIP_TRY(launch_bound(h));
+      if (h->cfg.secondorder) HIP_TRY(launch_compevo(h, end.last));
+      h->cur = 1 - h->cur;
+      if ((r = surface_errors(h))) {  // a face of the last step taken
+        *done -= 1;
+        return r;
+      }
+    }
+    // stopped before a step: its routines name the cause
+    int go = 1;
+    return end.why && end.why != kRunEnd ? evh_step(h, t, tend, dt, &go) : EVH_OK;
+  }
+  *dt = end.dt;
   if (end.why == kRunNext) {
     if ((r = surface_errors(h))) return r;
     h->v_valid = false;
@@ -730,9 +755,11 @@ int evh_run(evh_ctx *h, int nsteps, double *t, double tend, double *dt, int *don
   int go = 1;
   *done = 0;
   // one wait at the end where every kernel of a step can take its dt from the
-  // device: not with the staged kernels, nor hipFFT's transforms; with the
-  // stages timed, each step is waited for as its events are
-  const bool device = h->mode != EVH_MODE_STAGED && !h->timing && !h->zslab[0] && !h->zslab[1] &&
+  // device: not with the staged kernels (but for 1-D hydro, which has one
+  // kernel of their arithmetic), nor hipFFT's transforms; with the stages
+  // timed, each step is waited for as its events are
+  const bool kernels = h->mode != EVH_MODE_STAGED || (h->cfg.onedimension && !h->cfg.hydro_off && !h->cfg.gravity && !h->cfg.conduction);
+  const bool device = kernels && !h->timing && !h->zslab[0] && !h->zslab[1] &&
                       (!h->cfg.gravity || h->xyz_pencils) && nsteps > 1;
   if (device) return run_on_device(h, nsteps, t, tend, dt, done);
   for (int k = 0; k < nsteps && go; k++) {

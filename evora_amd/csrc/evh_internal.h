@@ -130,6 +130,7 @@ hipError_t launch_bound(evh_ctx *h);
 hipError_t launch_hydrostep(evh_ctx *h);
 hipError_t launch_compevo(evh_ctx *h, double dt);
 hipError_t launch_sweep(evh_ctx *h, double dt);
+hipError_t launch_line_step(evh_ctx *h, const StepCtl &c);  // a whole 1-D step, cur -> other, CFL of the result
 
 // fused kernels (fused.hip)
 hipError_t launch_cfl(evh_ctx *h);                 // primitive + CFL min over cur q

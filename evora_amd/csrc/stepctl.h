@@ -24,6 +24,7 @@ namespace evh {
 // the run at the start of a step; two take turns
 struct RunSlot {
   double t, dt;
+  double last;  // dt of the last step taken
   int go;    // updatetime's flag: 0 after the step that reaches tend
   int stop;  // no step is taken any more
   int done;  // steps taken
@@ -102,6 +103,7 @@ __device__ __forceinline__ bool step_begin(const KParams &P, const StepCtl &C, d
   dt = uniform_value(s.dt);
   if (first) {
     s.t = s.t + s.dt;
+    s.last = s.dt;
     s.done += 1;
     *C.out = s;
     clear_status(C.reset);
