@@ -345,11 +345,11 @@ int evh_create(const evh_config *cfg, evh_ctx **out) {
   }
   if (h->cfg.gravity && (e = gravity_init(h)) != hipSuccess) return bail(e);
   if ((e = h->xfer.init(n)) != hipSuccess) return bail(e);
-  if ((e = hipMalloc(&h->st_all, 4 * sizeof(Status))) != hipSuccess) return bail(e);
+  if ((e = hipMalloc(&h->st_all, 4 * sizeof(Status) + 2 * sizeof(RunSlot))) != hipSuccess) return bail(e);
   h->st = h->st_all;
-  if ((e = hipMalloc(&h->runs, 2 * sizeof(RunSlot))) != hipSuccess) return bail(e);
-  if ((e = hipHostMalloc(&h->st_host, sizeof(Status))) != hipSuccess) return bail(e);
+  h->runs = (RunSlot *)(h->st_all + 4);
   if ((e = hipHostMalloc(&h->run_host, sizeof(evh_ctx::RunHost))) != hipSuccess) return bail(e);
+  h->st_host = &h->run_host->now;
   if ((e = hipMalloc(&h->partials, sizeof(double) * 6 * kSumBlocks)) != hipSuccess) return bail(e);
   h->dev_bytes += h->xfer.device_bytes() + (long long)(4 * sizeof(Status) + 2 * sizeof(RunSlot)) + (long long)sizeof(double) * 6 * kSumBlocks;
   hipLaunchKernelGGL(k_clear_statuses, dim3(1), dim3(64), 0, h->stream, h->st_all, 4);
@@ -369,8 +369,6 @@ int evh_destroy(evh_ctx *h) {
   if (h->s) hipFree(h->s);
   h->xfer.release();
   if (h->st_all) hipFree(h->st_all);
-  if (h->runs) hipFree(h->runs);
-  if (h->st_host) hipHostFree(h->st_host);
   if (h->run_host) hipHostFree(h->run_host);
   if (h->partials) hipFree(h->partials);
   for (auto p : h->zhalo) if (p) hipFree(p);

@@ -89,9 +89,10 @@ struct evh_ctx {
   // status blocks on the device: three that take turns and one for what a
   // later kernel of the same step replaces; st: the current state's
   evh::Status *st_all = nullptr, *st = nullptr;
-  evh::Status *st_host = nullptr;  // pinned
-  evh::RunSlot *runs = nullptr;    // device: the two slots of a run of several steps
+  evh::RunSlot *runs = nullptr;    // device, behind the status blocks: the two slots of a run of several steps
+  evh::Status *st_host = nullptr;  // run_host->now
   struct RunHost {
+    evh::Status now;
     evh::Status st[3];
     evh::RunSlot runs[2];
   } *run_host = nullptr;  // pinned
