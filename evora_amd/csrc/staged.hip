@@ -189,32 +189,36 @@ __global__ void __launch_bounds__(kBlock) k_sweep(KParams P, Grid G, double *__r
 // All of the above for a grid of one row, q to the other buffer, with the
 // limits of the new state: in a run of steps nothing else is launched, where
 // the routines one by one are seven launches and three waits.  A small row is
-// bound by latency: 1000 cells (Sod) 57 -> 7.5 us per step.  A block takes
+// bound by latency: 1000 cells (Sod) 57 -> 7.0 us per step.  A block takes
 // kLine cells and two more on each side, so that every value but the fluxes'
 // operands is formed by the lane that owns the cell, in the arithmetic and
 // order of the kernels above: q, limits and errors are theirs bit for bit.
-// w, evo and s are not stored; a row of 5e6 cells takes 0.20 ms (96 bytes a
-// cell: 2.4 TB/s) for 1.50.
+// w, evo and s are not stored; a row of 5e6 cells takes 0.19 ms (96 bytes a
+// cell: 2.5 TB/s) for 1.50.
 constexpr int kLine = kBlock - 4;
 
 template <int SOLVER, int LIMITER>
 __global__ void __launch_bounds__(kBlock) k_line_step(KParams P, const double *__restrict__ qin,
                                                       double *__restrict__ qout, StepCtl C) {
   __shared__ double W[5][kBlock], U[5][kBlock], F[6][kBlock];  // primitive, state left of the next face, flux of the cell's left face
-  double dt;
-  if (!step_begin(P, C, dt)) return;
   const int lane = threadIdx.x;
   const long long n = P.nx;
+  double q[6], dt;
+  const auto fetch = [&](long long i) {
+    if (i >= n + 2) return;
+    const int c = ghost_src((int)i, (int)n, P.boundtype == 2);
+#pragma unroll
+    for (int m = 0; m < 6; m++) q[m] = qin[m * n + c];
+  };
+  fetch(blockIdx.x * (long long)kLine + lane - 2);  // on its way while dt is formed
+  if (!step_begin(P, C, dt)) return;
   const double dt2 = -0.5 * dt, delta = dt * P.dxinv;
   double v = 1e6;
   for (long long x0 = (long long)blockIdx.x * kLine; x0 < n; x0 += (long long)gridDim.x * kLine) {
     const long long i = x0 + lane - 2;  // -2 .. n + 1: two ghosts on each side, as bound fills them
     const bool cell = i >= 0 && i < n;
-    double q[6], w[5], lo[5];
+    double w[5], lo[5];
     if (i < n + 2) {
-      const int c = ghost_src((int)i, (int)n, P.boundtype == 2);
-#pragma unroll
-      for (int m = 0; m < 6; m++) q[m] = qin[m * n + c];
       (void)q2w(P, q, w);
       if (P.boundtype == 3 && i >= n)
 #pragma unroll
@@ -261,6 +265,7 @@ __global__ void __launch_bounds__(kBlock) k_line_step(KParams P, const double *_
       if (e) report_next(C.lim, e, (unsigned long long)i);
       v = dmin(v, cfl_cell(P, w));
     }
+    fetch(i + (long long)gridDim.x * kLine);
   }
   block_min_pos<kBlock>(&C.lim->vmin_bits, v);
 }
