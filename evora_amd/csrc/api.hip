@@ -345,14 +345,14 @@ int evh_create(const evh_config *cfg, evh_ctx **out) {
   }
   if (h->cfg.gravity && (e = gravity_init(h)) != hipSuccess) return bail(e);
   if ((e = h->xfer.init(n)) != hipSuccess) return bail(e);
-  if ((e = hipMalloc(&h->st_all, 4 * sizeof(Status) + 2 * sizeof(RunSlot))) != hipSuccess) return bail(e);
+  if ((e = hipMalloc(&h->st_all, 3 * sizeof(Status) + 2 * sizeof(RunSlot))) != hipSuccess) return bail(e);
   h->st = h->st_all;
-  h->runs = (RunSlot *)(h->st_all + 4);
+  h->runs = (RunSlot *)(h->st_all + 3);
   if ((e = hipHostMalloc(&h->run_host, sizeof(evh_ctx::RunHost))) != hipSuccess) return bail(e);
   h->st_host = &h->run_host->now;
   if ((e = hipMalloc(&h->partials, sizeof(double) * 6 * kSumBlocks)) != hipSuccess) return bail(e);
-  h->dev_bytes += h->xfer.device_bytes() + (long long)(4 * sizeof(Status) + 2 * sizeof(RunSlot)) + (long long)sizeof(double) * 6 * kSumBlocks;
-  hipLaunchKernelGGL(k_clear_statuses, dim3(1), dim3(64), 0, h->stream, h->st_all, 4);
+  h->dev_bytes += h->xfer.device_bytes() + (long long)(3 * sizeof(Status) + 2 * sizeof(RunSlot)) + (long long)sizeof(double) * 6 * kSumBlocks;
+  hipLaunchKernelGGL(k_clear_statuses, dim3(1), dim3(64), 0, h->stream, h->st_all, 3);
   if ((e = hipStreamSynchronize(h->stream)) != hipSuccess) return bail(e);
   *out = h;
   return EVH_OK;
@@ -678,16 +678,15 @@ static int run_on_device(evh_ctx *h, int nsteps, double *t, double tend, double 
       c.tend = tend;
       c.hydro = hydro ? 1 : 0;
       c.head = 1;
-      Status *const replaced = h->st_all + 3;  // limits that a later kernel of the step replaces
       if (hydro) {
-        c.lim = grav || cond ? replaced : c.st;
+        c.lim = grav || cond ? nullptr : c.st;  // none that a later kernel of the step replaces
         HIP_TRY(line ? launch_line_step(h, c) : launch_fused_step(h, c));
         h->cur = 1 - h->cur;
         c.head = 0;
       }
       if (grav) {
         HIP_TRY(launch_gravpotential(h, h->cosmo, c));
-        c.lim = cond ? replaced : c.st;
+        c.lim = cond ? nullptr : c.st;
         HIP_TRY(launch_gravintegration(h, c));
         c.head = 0;
       }

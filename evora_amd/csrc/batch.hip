@@ -113,8 +113,10 @@ __global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((
       const KParams P = bx.P;
       const Geo G = bx.G;
       const bool to1 = bs.side[b] != 0;
-      core::march<T, S, SOLVER, LIMITER, TX, TY, false>(P, G, to1 ? q0 : q1, to1 ? q1 : q0, bx.qoff, b, bs.dt[b],
-                                                    &bs.st[b], &bs.st[b], item - lo, sm);
+      Status *const st = &bs.st[b];
+      __builtin_assume(st != nullptr);
+      core::march<T, S, SOLVER, LIMITER, TX, TY, false>(P, G, to1 ? q0 : q1, to1 ? q1 : q0, bx.qoff, b, bs.dt[b], st, st,
+                                                    item - lo, sm);
     }
     __syncthreads();  // s_item is rewritten only after every lane has used it
   }

@@ -86,8 +86,7 @@ struct evh_ctx {
   evh::Xfer xfer;
 
   // reductions
-  // status blocks on the device: three that take turns and one for what a
-  // later kernel of the same step replaces; st: the current state's
+  // status blocks on the device, three that take turns; st: the current state's
   evh::Status *st_all = nullptr, *st = nullptr;
   evh::RunSlot *runs = nullptr;    // device, behind the status blocks: the two slots of a run of several steps
   evh::Status *st_host = nullptr;  // run_host->now

@@ -647,7 +647,7 @@ __global__ void __launch_bounds__(GT) k_gravint(KParams P, GParams Gp, GGeo G, S
 #pragma unroll
       for (int m = 0; m < 6; m++) qs[m] = double(S(qc[m]));
       const int e = cell_limits<EXACT>(P, qs, v, t);
-      if (e) report_next(C.lim, e, (unsigned long long)c);
+      if (e && C.lim) report_next(C.lim, e, (unsigned long long)c);
       vmin = dmin(vmin, v);
       if (tout) tout[c] = S(t);
     }
@@ -655,7 +655,7 @@ __global__ void __launch_bounds__(GT) k_gravint(KParams P, GParams Gp, GGeo G, S
     pm = pc;
     pc = pn;
   }
-  block_min_pos<GT>(&C.lim->vmin_bits, vmin);
+  if (C.lim) block_min_pos<GT>(&C.lim->vmin_bits, vmin);
 }
 
 GParams make_gparams(const evh_ctx *h) {

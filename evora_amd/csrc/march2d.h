@@ -111,7 +111,7 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
   // carried from row k-1: its partial update q + dtx*(Fx), the flux of its
   // bottom face, its top face state (the last two in LDS with LC)
   T part[6], fyb[LC ? 1 : 6], ytop[LC ? 1 : 5];
-  core::CflMin<T, EXACT> cfl;
+  core::CflMin<T, EXACT> cfl(lim != nullptr);
   int err = 0, err_k = 0, nerr = 0, nerr_k = 0;
 
   S pre[6];
@@ -201,7 +201,7 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
               T wn[5], rn;
               const int ep = Ph::q2w(P, o, wn, rn);
               if (ep && !nerr) { nerr = ep; nerr_k = k - 1; }
-              cfl.add(P, wn, rn);
+              if (!tout || cfl.wanted()) cfl.add(P, wn, rn);
               if (tout) tout[oc] = S(Ph::temp(P, wn, rn));
               raise = !tout;
             }
@@ -254,9 +254,9 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
   if (err || nerr) {  // the lane's own column (clamped into the grid) locates the error
     const long long ex = min(max(gx, 0), G.nx - 1);
     if (err) report(st, err, (unsigned long long)(ex + G.nx * (long long)err_k));
-    if (nerr) report_next(lim, nerr, (unsigned long long)(ex + G.nx * (long long)nerr_k));
+    if (lim && nerr) report_next(lim, nerr, (unsigned long long)(ex + G.nx * (long long)nerr_k));
   }
-  block_min_pos<NL>(&lim->vmin_bits, cfl.wave_min());
+  if (lim) block_min_pos<NL>(&lim->vmin_bits, cfl.wave_min());
 }
 
 }  // namespace core2d

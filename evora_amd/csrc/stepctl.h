@@ -35,7 +35,7 @@ enum : int { kRunEnd = 1, kRunCode, kRunNext, kRunDt };
 struct StepCtl {
   double dt;           // the step's dt where the host gives it (in == nullptr)
   Status *st;          // takes the step's errors
-  Status *lim;         // takes the limits (and next errors) of the new state
+  Status *lim;         // takes the limits (and next errors) of the new state; nullptr: a later kernel of the step forms them
   const Status *prev;  // the limits and errors of the state the step starts from
   Status *reset;       // cleared for the next step (nullptr: none)
   const RunSlot *in;   // a run on the device: the run so far
