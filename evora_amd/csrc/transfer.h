@@ -107,40 +107,40 @@ class CopyTeam {
 };
 
 struct Xfer {
-  double *dstage = nullptr;            // device: kBuffers * chunk_cells * 6 doubles
-  void *pin[kBuffers] = {};            // pinned host: chunk_cells * 6 doubles each
+  double *dstage = nullptr;            // device: buffers * chunk_cells * 6 doubles
+  char *pinned = nullptr;              // pinned host: as much
   hipEvent_t ev[kBuffers] = {};
-  long long chunk_cells = 0;
+  long long chunk_cells = 0, buffers = 0;  // chunks of the largest grid fill up to kBuffers of them
 
-  // device staging for grids of up to max_cells cells
+  // device staging for grids of up to max_cells cells: the buffers hold the
+  // largest chunk that chunk_units gives
   hipError_t init(long long max_cells) {
-    chunk_cells = std::max(1LL, std::min(max_cells, kChunkBytes / kCellBytes));
+    chunk_cells = kChunkBytes / kCellBytes;
+    chunk_cells = std::min(std::max(1LL, max_cells), chunk_units(max_cells, kCellBytes));
+    buffers = std::min((long long)kBuffers, (max_cells + chunk_cells - 1) / chunk_cells);
     hipError_t e = hipMalloc(&dstage, device_bytes());
     for (auto &x : ev)
       if (e == hipSuccess) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
     return e;
   }
-  long long device_bytes() const { return kBuffers * chunk_cells * kCellBytes; }
+  long long device_bytes() const { return buffers * chunk_cells * kCellBytes; }
   void release() {
     if (dstage) (void)hipFree(dstage);
-    for (auto &p : pin) {
-      if (p) (void)hipHostFree(p);
-      p = nullptr;
-    }
+    if (pinned) (void)hipHostFree(pinned);
+    pinned = nullptr;
     for (auto &x : ev) {
       if (x) (void)hipEventDestroy(x);
       x = nullptr;
     }
     dstage = nullptr;
   }
+  // one allocation, of what a transfer can turn over: pinning takes 0.1 ms and
+  // more each time (64^3 context: first upload 0.9 ms with four buffers of the
+  // whole state's size, 0.6 ms with these; 128^2 0.13 -> 0.09)
   hipError_t ensure_pinned() {
-    for (auto &p : pin)
-      if (!p) {
-        hipError_t e = hipHostMalloc(&p, chunk_cells * kCellBytes, hipHostMallocDefault);
-        if (e != hipSuccess) return e;
-      }
-    return hipSuccess;
+    return pinned ? hipSuccess : hipHostMalloc((void **)&pinned, device_bytes(), hipHostMallocDefault);
   }
+  char *pin(int b) const { return pinned + (long long)b * kCellBytes * chunk_cells; }
   double *stage(int b) const { return dstage + (long long)b * 6 * chunk_cells; }
 
   // units of `bytes` each per chunk for a transfer of n: an eighth of it, so
@@ -154,17 +154,17 @@ struct Xfer {
   // layout kernel of one chunk on stream s
   template <typename F>
   hipError_t upload(const double *q, long long n, hipStream_t s, F launch) {
+    const long long chunk = chunk_units(n, kCellBytes);
     hipError_t e = ensure_pinned();
     if (e != hipSuccess) return e;
     CopyTeam team((size_t)(n * kCellBytes));
-    const long long chunk = chunk_units(n, kCellBytes);
     long long i = 0;
     for (long long base = 0; base < n; base += chunk, i++) {
       const int b = (int)(i % kBuffers);
       const long long cells = std::min(chunk, n - base);
-      if (i >= kBuffers && (e = hipEventSynchronize(ev[b])) != hipSuccess) return e;  // pin[b] consumed
-      team.copy(pin[b], q + 6 * base, cells * kCellBytes);
-      if ((e = hipMemcpyAsync(stage(b), pin[b], cells * kCellBytes, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+      if (i >= kBuffers && (e = hipEventSynchronize(ev[b])) != hipSuccess) return e;  // pin(b) consumed
+      team.copy(pin(b), q + 6 * base, cells * kCellBytes);
+      if ((e = hipMemcpyAsync(stage(b), pin(b), cells * kCellBytes, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
       if ((e = hipEventRecord(ev[b], s)) != hipSuccess) return e;
       if ((e = launch(stage(b), cells, base)) != hipSuccess) return e;
     }
@@ -192,10 +192,10 @@ struct Xfer {
   // on stream s at device address src
   template <typename F>
   hipError_t stream_down(char *out, long long n, long long bytes, hipStream_t s, F fill) {
+    const long long chunk = chunk_units(n, bytes), chunks = (n + chunk - 1) / chunk;
     hipError_t e = ensure_pinned();
     if (e != hipSuccess) return e;
     CopyTeam team((size_t)(n * bytes));
-    const long long chunk = chunk_units(n, bytes), chunks = (n + chunk - 1) / chunk;
     // chunk i is enqueued kBuffers - 1 chunks before it is copied out, into a
     // buffer whose last chunk has been
     for (long long i = 0; i < chunks + kBuffers - 1; i++) {
@@ -204,7 +204,7 @@ struct Xfer {
         const long long base = i * chunk, units = std::min(chunk, n - base);
         const void *src = nullptr;
         if ((e = fill(b, units, base, &src)) != hipSuccess) return e;
-        if ((e = hipMemcpyAsync(pin[b], src, units * bytes, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+        if ((e = hipMemcpyAsync(pin(b), src, units * bytes, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
         if ((e = hipEventRecord(ev[b], s)) != hipSuccess) return e;
       }
       const long long j = i - (kBuffers - 1);
@@ -212,7 +212,7 @@ struct Xfer {
         const int b = (int)(j % kBuffers);
         const long long base = j * chunk;
         if ((e = hipEventSynchronize(ev[b])) != hipSuccess) return e;
-        team.copy(out + base * bytes, pin[b], std::min(chunk, n - base) * bytes);
+        team.copy(out + base * bytes, pin(b), std::min(chunk, n - base) * bytes);
       }
     }
     return hipSuccess;
