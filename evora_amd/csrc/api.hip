@@ -314,11 +314,10 @@ int evh_create(const evh_config *cfg, evh_ctx **out) {
   h->grid = Grid{cfg->nx, cfg->ny, cfg->nz};
   h->qelem = mixed(h) ? sizeof(float) : sizeof(double);
   h->mode = fused_supported(*cfg) ? EVH_MODE_FUSED : EVH_MODE_STAGED;
-  // launch shape measured fastest on MI355X for the 512^3 blast (16x12 tiles,
-  // 64-plane chunks, the higher waves-per-SIMD budget: FP64 runs at 2
-  // waves/SIMD, FP32 at 4)
+  // launch shape measured fastest on MI355X: 192-column tiles (FP32 at 4
+  // waves per SIMD, FP64 at 2)
   h->tile_ty = 12;
-  h->zchunk = 0;  // automatic: 64 planes, fewer on small grids
+  h->zchunk = 0;  // automatic (march_chunk)
   h->wpe_hi = 1;
 
   auto bail = [&](hipError_t e) {

@@ -19,8 +19,8 @@
 //       lanes solve their z face k-1/2 (riemann.f90) and finish plane k-1
 //       as (q + dtx*(Fx) + dty*(Fy)) + dtz*(Fz), the reference's x, y, z
 //       order (muscl.f90:191-272, integration :287), store it, and take the
-//       primitive and the CFL limit of those of its cells that can change
-//       the minimum for the next hydrostep (timestep.f90:26-57; CflMin).
+//       CFL limit of its new state for the next hydrostep
+//       (timestep.f90:26-57; CflMin).
 //   S3  x and y faces of plane k: interior lane (i,j) solves its left and
 //       bottom faces, the ring wave the TY right-edge and TX top-edge faces
 //       in one solve.  Each flux overwrites the two states it came from.
@@ -34,14 +34,13 @@
 // instruction takes about 5 cycles of its SIMD, and the SIMDs that hold
 // interior waves only have one to issue 98% of the time); FP32-mixed, the
 // L1's requests to L2 for the ring.  512^3 HLLC blast, FP64: 6.36 ms with both
-// roles in one loop (219 VGPRs), the carry in LDS and every cell's limit
-// formed; 5.62 ms (23.9 G cell updates/s) with a loop per role, so that
-// neither holds the other's values (205 VGPRs with the carry in registers,
-// 32 of 135 LDS operations per plane gone, 46 KB of LDS instead of 72),
-// third-order reciprocals and roots, the star flux from its jump conditions,
-// the predictor from shared factors, and the limit only where it can count.
-// FP32-mixed: 3.33 -> 2.95 ms (45.5 G), with its constants in scalar
-// registers (16 B/lane of spills gone).
+// roles in one loop (219 VGPRs) and the carry in LDS; 5.46 ms (24.6 G cell
+// updates/s) with a loop per role, so that neither holds the other's values
+// (the carry in registers, 32 of 135 LDS operations per plane gone, 46 KB of
+// LDS instead of 72), third-order reciprocals and roots, the star flux from
+// its jump conditions, the predictor from shared factors, and the limit from
+// q.  FP32-mixed: 3.33 -> 2.58 ms (52 G), with its constants in scalar
+// registers (16 B/lane of spills gone) and the 32 x 6 tile.
 #pragma once
 
 #include "evh_internal.h"
@@ -453,65 +452,43 @@ __device__ __forceinline__ void store_w(T (*W)[EA], int slot, const T w[5]) {
 }
 
 // ---- the CFL minimum of the new state
-// Most cells cannot set the step's CFL minimum: their fastest signal is
-// slower than one already found.  `slower` tells so without the primitive:
-// with a lower bound thr of the largest signal speed max_d (|u_d| + a) / dx_d
-// found so far in this step, a cell whose |m_d| + a rho < thr dx_d rho in
-// every direction, with (a rho)^2 = g p rho = g g1 (rho E - m^2/2), changes
-// neither the minimum nor the error state (p > 0, by a margin above the
-// rounding of any form; with dual energy also p from E, not from the
-// entropy).  About 16 operations against 50 for the primitive and the limit;
-// thr carries a margin of 5e-6, far above the rounding of this test, so
-// the minimum is the same to the last bit.  false for NaN.
-template <typename T>
-__device__ __forceinline__ bool slower(const KParams &P, const T q[6], T thr) {
-  const auto &C = consts(P, T());
-  const T er = q[4] * q[0];
-  const T m2 = fm::fma(q[3], q[3], fm::fma(q[2], q[2], q[1] * q[1]));
-  const T x = fm::fma(T(-0.5), m2, er);
-  const T a = thr * q[0];
-  const T d = dmin(dmin(fm::fma(a, C.dx, -fm::fabs(q[1])), fm::fma(a, C.dy, -fm::fabs(q[2]))),
-                   fm::fma(a, C.dz, -fm::fabs(q[3])));
-  return x > C.calm * er && d > T(0) && d * d > C.ggm * fm::fma(T(1e-6), er, x);
-}
-
-// the largest of the wave's positive values, as a scalar
-__device__ __forceinline__ float wave_max_pos(float v) {
-  int x = __builtin_bit_cast(int, v);
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false));  // row_shr 1, 2, 4, 8
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false));
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false));  // row_bcast 15, 31
-  x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false));
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(x, 63));
-}
-
-// The running minimum of one lane, min_c 1 / max_d (|u_d| + a) / dx_d, and
-// the wave's bound for `slower`.  The FP64 fast form keeps -max_d (..) per
-// cell and inverts once per lane; a lane without cells gives 1e6 either way.
+// The running minimum of one lane, min_c 1 / max_d (|u_d| + a) / dx_d.  Every
+// cell counts: a test of 16 operations that told which cells cannot set the
+// minimum spared most of a field that varies from cell to cell, but none of a
+// uniform medium, whose cells all have its largest speed, and cost more there:
+// 256^3 shock and cloud FP64 0.784 ms with it, 0.741 without; FP32-mixed 0.390,
+// 0.371; 512^3 blast in 1% noise 5.43, 5.46; FP32-mixed 2.51, 2.58.
+//
+// The FP64 fast form keeps -max_d (..) per cell and inverts once per lane,
+// and where p comes from E by a margin above the rounding of any form (and p
+// > 0, so that nothing is to be reported) takes it from q without the
+// primitive: (a rho)^2 = g g1 (rho E - m^2/2), max_d (|m_d| + a rho) / dx_d
+// times 1/rho, 25 operations for 47, both to a few ulp (times E/p, as with
+// p = g1 (E - kin)).  A lane without cells gives 1e6.
 template <typename T, bool EXACT>
 struct CflMin {
   static constexpr bool kSpeedKey = !EXACT && sizeof(T) == 8;
-  static constexpr float kMargin = 0.999995f;
   double v = kSpeedKey ? -1e-6 : 1e6;
-  T thr = T(1e-6f * kMargin);
-  // no limit is wanted (gravity or conduction changes the state and forms it):
-  // a bound that no signal reaches, so that no cell takes the primitive for it.
-  // 128^3 FP64 steps with gravity 0.218 -> 0.214 ms, with conduction 0.163 ->
-  // 0.159; 256^3 1.32 -> 1.31 and 1.035 -> 1.028
-  __device__ __forceinline__ explicit CflMin(bool wanted) {
-    if (!wanted) thr = T(__builtin_inff());
-  }
-  __device__ __forceinline__ bool wanted() const { return thr < T(__builtin_inff()); }
   __device__ __forceinline__ void add(const KParams &P, const T w[5], T rinv) {
     if constexpr (kSpeedKey) v = dmin(v, -fast::cfl_speed(P, w, rinv));
     else v = dmin(v, Phys<EXACT>::cfl_cell(P, w, rinv));
   }
-  __device__ __forceinline__ void raise() {  // all lanes of the wave
-    const float s = kSpeedKey ? float(-v) : fm::rcp(float(v));
-    const T t = T(wave_max_pos(s) * kMargin);
-    thr = t > thr ? t : thr;
+  // from q; false where it takes the primitive (and for NaN)
+  __device__ __forceinline__ bool add(const KParams &P, const T q[6]) {
+    if constexpr (kSpeedKey) {
+      const double er = q[4] * q[0];
+      const double m2 = fm::fma(q[3], q[3], fm::fma(q[2], q[2], q[1] * q[1]));
+      const double x = fm::fma(-0.5, m2, er);
+      if (!(x > P.calm * er)) return false;
+      const double a2 = P.ggm * x, ar = fm::div_sqrt_pos(a2, a2);
+      const double sx = (fm::fabs(q[1]) + ar) * P.dxinv;
+      const double sy = (fm::fabs(q[2]) + ar) * P.dyinv;
+      const double sz = (fm::fabs(q[3]) + ar) * P.dzinv;
+      v = dmin(v, -(dmax(dmax(sx, sy), sz) * fm::rcp(q[0])));
+      return true;
+    } else {
+      return false;
+    }
   }
   // the wave's minimum, in every lane
   __device__ __forceinline__ double wave_min() {
@@ -547,7 +524,7 @@ struct Place {
 template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, bool EXACT, bool SLAB>
 __device__ __forceinline__ void march_columns(const KParams &P, const Geo &G, const Place &L,
                                               const S *__restrict__ qin, S *__restrict__ qout, double dt,
-                                              Smem<T, TX, TY> &sm, S *__restrict__ tout, CflMin<T, EXACT> &cfl,
+                                              Smem<T, TX, TY> &sm, S *__restrict__ tout, const Status *lim, CflMin<T, EXACT> &cfl,
                                               LaneErrors &er, int tid) {
   using TS = TileShape<TX, TY>;
   constexpr int EW = TS::EW;
@@ -654,17 +631,13 @@ __device__ __forceinline__ void march_columns(const KParams &P, const Geo &G, co
 #pragma unroll
             for (int m = 0; m < 6; m++) (qout + (m * G.n + op))[own_xy] = S(o[m]);
           }
-          // the limits of the new state, for the cells that can change them
-          const bool need = inside && (tout || !slower(P, o, cfl.thr));
-          if (__builtin_amdgcn_ballot_w64(need)) {
-            if (need) {
-              T wn[5], rn;
-              const int ep = Phys<EXACT>::q2w(P, o, wn, rn);
-              if (ep && !er.nerr) { er.nerr = ep; er.nerr_k = k - 1; }
-              if (!tout || cfl.wanted()) cfl.add(P, wn, rn);
-              if (tout) (tout + op)[own_xy] = S(Phys<EXACT>::temp(P, wn, rn));
-            }
-            if (!tout) cfl.raise();
+          // the limits (and temperature) of the new state, where they are wanted
+          if (inside && (tout || (lim && !cfl.add(P, o)))) {
+            T wn[5], rn;
+            const int ep = Phys<EXACT>::q2w(P, o, wn, rn);
+            if (ep && !er.nerr) { er.nerr = ep; er.nerr_k = k - 1; }
+            if (lim) cfl.add(P, wn, rn);
+            if (tout) (tout + op)[own_xy] = S(Phys<EXACT>::temp(P, wn, rn));
           }
         }
 #pragma unroll
@@ -897,8 +870,8 @@ __device__ __forceinline__ void march(const KParams &P, const Geo &G, const S *_
   LaneErrors er;
   int gx, gy;  // the lane's own column, which locates its errors
   if (wave < NI / 64) {
-    CflMin<T, EXACT> cfl(lim != nullptr);
-    march_columns<T, S, SOLVER, LIMITER, TX, TY, EXACT, SLAB>(P, G, L, qin, qout, dt, sm, tout, cfl, er, tid);
+    CflMin<T, EXACT> cfl;
+    march_columns<T, S, SOLVER, LIMITER, TX, TY, EXACT, SLAB>(P, G, L, qin, qout, dt, sm, tout, lim, cfl, er, tid);
     const double v = cfl.wave_min();
     if ((tid & 63) == 0) sm.vmin[wave] = v;
     gx = L.x0 + tid % TX;

@@ -111,7 +111,7 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
   // carried from row k-1: its partial update q + dtx*(Fx), the flux of its
   // bottom face, its top face state (the last two in LDS with LC)
   T part[6], fyb[LC ? 1 : 6], ytop[LC ? 1 : 5];
-  core::CflMin<T, EXACT> cfl(lim != nullptr);
+  core::CflMin<T, EXACT> cfl;
   int err = 0, err_k = 0, nerr = 0, nerr_k = 0;
 
   S pre[6];
@@ -139,7 +139,6 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
 
   for (int k = y0 - 1; k <= y1; k++) {
     const bool out_row = k >= y0 && k < y1;
-    bool raise = false;
     // ---- S1: w of row k to LDS
 #pragma unroll
     for (int m = 0; m < 5; m++) W[m][l] = wc[m];
@@ -196,14 +195,13 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
             const long long oc = (long long)gx + (long long)G.nx * (k - 1);
 #pragma unroll
             for (int m = 0; m < 6; m++) qout[m * G.n + oc] = S(o[m]);
-            // the limits of the new state, for the cells that can change them
-            if (tout || !core::slower(P, o, cfl.thr)) {
+            // the limits (and temperature) of the new state, where they are wanted
+            if (tout || (lim && !cfl.add(P, o))) {
               T wn[5], rn;
               const int ep = Ph::q2w(P, o, wn, rn);
               if (ep && !nerr) { nerr = ep; nerr_k = k - 1; }
-              if (!tout || cfl.wanted()) cfl.add(P, wn, rn);
+              if (lim) cfl.add(P, wn, rn);
               if (tout) tout[oc] = S(Ph::temp(P, wn, rn));
-              raise = !tout;
             }
           }
 #pragma unroll
@@ -219,7 +217,6 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
         }
       }
     }
-    if (__builtin_amdgcn_ballot_w64(raise)) cfl.raise();
     __syncthreads();
 
     // ---- S3: the x face (l, l+1) of row k

@@ -3,8 +3,9 @@
 // This is the reference-structured form of the step: primitive writes w,
 // bound fills the ghosts, hydrostep reduces the CFL limit, compevo writes
 // evo and s, and the sweep applies the x, then y, then z flux differences to
-// q.  It serves 1-D and 2-D grids (whose compevo association differs,
-// muscl.f90:60-88) and checks each routine on its own against the oracle.
+// q.  It serves 1-D grids (whose compevo association differs, muscl.f90:60-68)
+// and checks each routine on its own against the oracle.  A run of 1-D steps
+// takes k_line_step, which is all of it in one pass.
 // Built with -ffp-contract=off: results equal the reference's bit for bit
 // except for the pow() feeding the passive entropy component.
 #include "evh_internal.h"

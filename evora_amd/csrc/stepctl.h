@@ -9,8 +9,8 @@
 // hydrostep, thermalstep and updatetime do (timestep.f90:26-57,72-104,
 // 147-171), every block from the same values and one of them storing the
 // result for the next step.  A step after the end, or after an error, does
-// nothing.  128^2 2-D Kelvin-Helmholtz: 31 -> 14 us per step; 64^3 blast: 62
-// -> 43 us.
+// nothing.  128^2 2-D Kelvin-Helmholtz: 31 -> 17 us per step (12 with its
+// shorter chunks); 64^3: 62 -> 43 us (30 with them).
 //
 // Three status blocks take turns: a step reads the limits of the state it
 // starts from in one, leaves those of its own new state in the next, and

@@ -1,8 +1,8 @@
-"""The launch shapes and the CFL filter of the march: FP32's 32 x 6 column tile
+"""The launch shapes and the CFL limit of the march: FP32's 32 x 6 column tile
 at its edges and with chunks from one plane to all of them, against the
 16 x 8 tile bit for bit; the limit of a new state with one cell faster than
-the rest, against the limit of the same state uploaded (formed without the
-filter); the potential's download over more than one buffer."""
+the rest, against the limit of the same state uploaded (formed from its
+primitive); the potential's download over more than one buffer."""
 import numpy as np
 import pytest
 
@@ -40,7 +40,7 @@ def test_wide_tile_equals_the_other(nx, ny, nz, bound, solver, limiter):
 @pytest.mark.parametrize("dual", [False, True])
 @pytest.mark.parametrize("axis", [0, 1, 2])
 @pytest.mark.parametrize("mach", [0.1, 8.0, 40.0])
-def test_filtered_limit(mode, precision, tol, nz, dual, axis, mach):
+def test_limit_of_a_new_state(mode, precision, tol, nz, dual, axis, mach):
     """One cell moves at up to Mach 40 (with dual energy its pressure comes
     from the entropy there), the rest at a tenth of its speed."""
     if nz == 1 and axis == 2:
