@@ -35,11 +35,15 @@ constexpr long long kCellBytes = 6 * 8;  // one cell of q in the reference layou
 // Threads that copy memory together, for the length of one transfer.
 class CopyTeam {
  public:
-  // one thread per 2 MB of the transfer, 16 at most; if the system gives
-  // fewer, those copy it all
+  // one thread per 8 MB of a transfer of 32 MB or more, 8 at most; if the
+  // system gives fewer, those copy it all.  More threads are no faster on an
+  // idle host (64^3, 12.6 MB: 0.57 ms either way; 128^3 2.66 and 2.67 ms with one per
+  // 2 MB, 16 at most), and where another library's threads spin on every CPU
+  // each one may wait a scheduler's slice of 4 ms: 18 MB after a step loop
+  // 2.1 ms against 4.0, 96 MB 13.0 against 16.0.
   explicit CopyTeam(size_t total) {
-    const unsigned most = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    const unsigned n = (unsigned)std::min<size_t>(most, total >> 21);
+    const unsigned most = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
+    const unsigned n = total < (32u << 20) ? 1u : (unsigned)std::min<size_t>(most, total >> 23);
     try {
       for (unsigned i = 1; i < n; i++) threads_.emplace_back([this, i] { work(i); });
     } catch (const std::exception &) {
