@@ -88,7 +88,14 @@ __global__ void k_clear_statuses(Status *st, int n) {
 }
 
 __global__ void k_run_start(RunSlot *r, double t) {
-  if (threadIdx.x == 0) *r = RunSlot{t, 1e99, 1e99, 1, 0, 0, 0};
+  if (threadIdx.x < 2) r[threadIdx.x] = RunSlot{t, 1e99, 1e99, 1, 0, 0, 0};
+}
+
+// the head of a step whose first kernels do not form dt themselves: without
+// hydro the potential's passes come first, and ask whether the step is taken
+__global__ void k_step_head(KParams P, StepCtl C) {
+  double dt;
+  (void)step_begin(P, C, dt);
 }
 
 // AoS chunk (cells x 6, double) -> SoA storage at cell offset `base`
@@ -684,10 +691,13 @@ static int run_on_device(evh_ctx *h, int nsteps, double *t, double tend, double 
         c.head = 0;
       }
       if (grav) {
+        if (!hydro) {
+          hipLaunchKernelGGL(k_step_head, dim3(1), dim3(64), 0, h->stream, h->kp, c);
+          c.head = 0;
+        }
         HIP_TRY(launch_gravpotential(h, h->cosmo, c));
         c.lim = cond ? nullptr : c.st;
         HIP_TRY(launch_gravintegration(h, c));
-        c.head = 0;
       }
       if (cond) {
         if (!hydro) HIP_TRY(launch_temp(h));

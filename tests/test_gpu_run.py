@@ -104,3 +104,28 @@ def test_run_stops_as_steps_do(what):
     for x, y in zip(*got):
         assert np.array_equal(np.asarray(x, dtype=object), np.asarray(y, dtype=object)) if isinstance(x, tuple) \
             else np.array_equal(x, y), (x, y)
+
+
+@pytest.mark.parametrize("precision,mode", [(hydro.FP64, hydro.MODE_FUSED), (hydro.FP64, hydro.MODE_FUSED_EXACT),
+                                            (hydro.FP32_MIXED, hydro.MODE_FUSED)])
+def test_run_without_hydro_takes_each_steps_own_potential(precision, mode):
+    """Gravity and conduction without hydro: the potential's passes lead the
+    step.  The first run of a context, one that ends with steps to spare, and
+    one from another state after it: each step has the potential of its own
+    state, and a step after the end forms none."""
+    p = ics.conduction_params(16, hydro=False, gravity=True)
+    q0 = 10 * ics.conduction_blob(p)
+    q1 = ics.conduction_blob(p, seed=3)
+    out = []
+    for drive in (_run, _steps):
+        with hydro.Hydro(p, precision=precision, mode=mode) as h:
+            h.upload_q(q0)
+            a = drive(h, 2, 0.0, 1e30)
+            first = (h.download_q(), h.download_phi())
+            b = drive(h, 100, a[0], a[0] + 2.5 * a[1])
+            end = (h.download_q(), h.download_phi())
+            h.upload_q(q1)
+            c = drive(h, 2, 0.0, 1e30)
+            out.append((a, b, c, *first, *end, h.download_q(), h.download_phi()))
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
