@@ -294,7 +294,8 @@ KParams make_kparams(const evh_config &c) {
   k.ggm = k.g * k.g1;
   // 4e-6 is above the FP32 rounding of E - kin; with dual energy p comes from
   // E while kin <= de_thresh1 E
-  k.calm = 4e-6 + (k.dualenergy ? std::fmax(0.0, 1.0 - k.de_thresh1) : 0.0);
+  // (for g <= 1 no cell has p > 0 by it)
+  k.calm = !(k.g1 > 0.0) ? INFINITY : 4e-6 + (k.dualenergy ? std::fmax(0.0, 1.0 - k.de_thresh1) : 0.0);
   k.f = {float(k.g), float(k.g1), float(k.g1inv), float(k.gg1), float(k.de_thresh1), float(k.kin_frac64),
          float(k.temp0), float(k.dxinv), float(k.dyinv), float(k.dzinv),
          float(k.dx), float(k.dy), float(k.dz), float(k.ggm), float(k.calm)};

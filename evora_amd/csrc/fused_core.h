@@ -479,7 +479,8 @@ struct CflMin {
       const double er = q[4] * q[0];
       const double m2 = fm::fma(q[3], q[3], fm::fma(q[2], q[2], q[1] * q[1]));
       const double x = fm::fma(-0.5, m2, er);
-      if (!(x > P.calm * er)) return false;
+      // with rho < 0, or E < 0 and calm >= 1, an x above calm rho E is no pressure above 0
+      if (!(q[0] > 0.0 && x > P.calm * fm::fabs(er))) return false;
       const double a2 = P.ggm * x, ar = fm::div_sqrt_pos(a2, a2);
       const double sx = (fm::fabs(q[1]) + ar) * P.dxinv;
       const double sy = (fm::fabs(q[2]) + ar) * P.dyinv;

@@ -1,0 +1,66 @@
+"""The limits a sweep leaves for the next step, in states that no step should
+start from: the fast FP64 form takes most cells' CFL limit from q without the
+primitive, and has to find every cell the primitive finds."""
+import numpy as np
+import pytest
+
+from evora_amd import hydro, ics
+from evora_amd.batch import Batch
+from evora_amd.params import HydroParams
+
+pytestmark = pytest.mark.gpu
+
+HOT = (13, 4)  # x, y of the cell that empties
+
+
+def _hot_cell(nz, cfl=0.4, **kw):
+    """Gas at rest with one hot, dense cell, which a step far beyond the CFL
+    limit drains below zero, symmetrically, so that its momentum stays 0."""
+    p = HydroParams(nx=24, ny=10, nz=nz, solver=2, limiter=1, boundtype=1, cfl=cfl, atomic=True, secondorder=False, **kw)
+    one = np.ones((nz, 10, 24))
+    rho, pres = one.copy(), one.copy()
+    rho[nz // 2, HOT[1], HOT[0]], pres[nz // 2, HOT[1], HOT[0]] = 10.0, 100.0
+    return p, ics.prim_to_q(p.derive(), rho, 0 * one, 0 * one, 0 * one, pres)
+
+
+def _only_invalid(q, nz, sign_rho):
+    """Whether the hot cell alone has no pressure, with E < 0 and rho of the given sign."""
+    bad = np.argwhere(q[..., 4] - 0.5 * (q[..., 1:4] ** 2).sum(-1) / q[..., 0] <= 0).tolist()
+    c = q[nz // 2, HOT[1], HOT[0]]
+    return bad == [[nz // 2, HOT[1], HOT[0]]] and c[4] < 0 and sign_rho * c[0] > 0
+
+
+# factor: of the CFL limit's dt; with a dual-energy threshold of 1 every cell
+# of moving gas takes p from the entropy, and E < 0 at rest is the only stop
+CASES = [(8, {}, 12.0, -1), (1, {}, 12.0, -1), (8, {"dualenergy": True, "de_thresh": 1.0}, 0.79, 1),
+         (1, {"dualenergy": True, "de_thresh": 1.0}, 0.975, 1)]
+
+
+@pytest.mark.parametrize("nz,kw,factor,sign_rho", CASES)
+@pytest.mark.parametrize("mode", [hydro.MODE_FUSED, hydro.MODE_FUSED_EXACT])
+def test_cell_without_pressure_is_found(nz, kw, factor, sign_rho, mode):
+    p, q0 = _hot_cell(nz, **kw)
+    with hydro.Hydro(p, mode=mode) as h:
+        h.upload_q(q0)
+        h.primitive()
+        dt = factor * h.hydrostep(1e99) / p.cfl
+        h.compevo(dt)
+        h.sweep(dt)
+        as_meant = _only_invalid(h.download_q(), nz, sign_rho)
+        assert as_meant
+        h.primitive()
+        with pytest.raises(hydro.EvoraError) as e:
+            h.hydrostep(1e99)
+    assert e.value.code == 1 and e.value.cell == (HOT[0] + 1, HOT[1] + 1, nz // 2 + 1)
+
+
+def test_cell_without_pressure_is_found_in_a_batch():
+    nz, kw, factor, _ = CASES[0]
+    p, q0 = _hot_cell(nz, cfl=factor)
+    with Batch([p, p]) as b:
+        b.upload_q(0, np.ones(q0.shape) * q0[0, 0, 0])
+        b.upload_q(1, q0)
+        with pytest.raises(hydro.EvoraError) as e:
+            b.run(2, graph=False)
+        assert e.value.code == 1 and e.value.box == 1 and e.value.cell == (HOT[0] + 1, HOT[1] + 1, nz // 2 + 1)
+        assert b.times()[2].tolist() == [2, 1]
