@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(256) k_batch_cfl(const BoxDev *__restrict__ bo
     for (int m = 0; m < 6; m++) qc[m] = double(q[m * n + c]);
     const int e = q2w(P, qc, wc);
     if (e) report_next(&bs.st[b], e, (unsigned long long)c);
-    vmin = dmin(vmin, cfl_cell(P, wc));
+    vmin = min_limit(vmin, cfl_cell(P, wc));
   }
   block_min_pos<256>(&bs.st[b].vmin_bits, vmin);
 }

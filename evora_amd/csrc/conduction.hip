@@ -253,8 +253,8 @@ __global__ void __launch_bounds__(CT) k_conduct(KParams P, CGeo G, S *__restrict
       for (int m = 0; m < 6; m++) qs[m] = double(S(qc[m]));
       const int ep = M::limits(P, qs, v, tv);
       if (ep) report_next(C.lim, ep, (unsigned long long)c);
-      vmin = dmin(vmin, v);
-      tvmin = dmin(tvmin, tv);
+      vmin = min_limit(vmin, v);
+      tvmin = min_limit(tvmin, tv);
     }
     __syncthreads();  // T is rewritten for the next plane only after every lane has read it
     tm = tc;
@@ -286,7 +286,7 @@ __global__ void __launch_bounds__(256) k_thermal_min(KParams P, long long n, con
     for (int m = 0; m < 6; m++) qc[m] = double(q[m * n + c]);
     const int e = M::limits(P, qc, vc, tv);  // pressure(q) of timestep.f90:87
     if (e) report_next(st, e, (unsigned long long)c);
-    v = dmin(v, tv);
+    v = min_limit(v, tv);
   }
   block_min_pos<256>(&st->tvmin_bits, v);
 }

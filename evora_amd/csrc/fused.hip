@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(256) k_cfl(KParams P, Geo G, const S *__restri
     for (int m = 0; m < 6; m++) qc[m] = double(q[m * G.n + c]);
     const int e = q2w(P, qc, wc);
     if (e) report_next(st, e, (unsigned long long)c);
-    vmin = dmin(vmin, cfl_cell(P, wc));
+    vmin = min_limit(vmin, cfl_cell(P, wc));
   }
   block_min_pos<256>(&st->vmin_bits, vmin);
 }

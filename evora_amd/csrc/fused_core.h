@@ -470,8 +470,8 @@ struct CflMin {
   static constexpr bool kSpeedKey = !EXACT && sizeof(T) == 8;
   double v = kSpeedKey ? -1e-6 : 1e6;
   __device__ __forceinline__ void add(const KParams &P, const T w[5], T rinv) {
-    if constexpr (kSpeedKey) v = dmin(v, -fast::cfl_speed(P, w, rinv));
-    else v = dmin(v, Phys<EXACT>::cfl_cell(P, w, rinv));
+    if constexpr (kSpeedKey) v = min_limit(v, -fast::cfl_speed(P, w, rinv));
+    else v = min_limit(v, Phys<EXACT>::cfl_cell(P, w, rinv));
   }
   // from q; false where it takes the primitive (and for NaN)
   __device__ __forceinline__ bool add(const KParams &P, const T q[6]) {
@@ -485,7 +485,7 @@ struct CflMin {
       const double sx = (fm::fabs(q[1]) + ar) * P.dxinv;
       const double sy = (fm::fabs(q[2]) + ar) * P.dyinv;
       const double sz = (fm::fabs(q[3]) + ar) * P.dzinv;
-      v = dmin(v, -(dmax(dmax(sx, sy), sz) * fm::rcp(q[0])));
+      v = min_limit(v, -(dmax(dmax(sx, sy), sz) * fm::rcp(q[0])));
       return true;
     } else {
       return false;
@@ -494,7 +494,7 @@ struct CflMin {
   // the wave's minimum, in every lane
   __device__ __forceinline__ double wave_min() {
     if constexpr (kSpeedKey) v = fm::rcp(-v);
-    for (int off = 32; off > 0; off >>= 1) v = dmin(v, __shfl_xor(v, off));
+    for (int off = 32; off > 0; off >>= 1) v = min_limit(v, __shfl_xor(v, off));
     return v;
   }
 };
@@ -889,7 +889,7 @@ __device__ __forceinline__ void march(const KParams &P, const Geo &G, const S *_
   if (lim && threadIdx.x == 0) {
     double v = sm.vmin[0];
 #pragma unroll
-    for (int i = 1; i < NI / 64; i++) v = dmin(v, sm.vmin[i]);
+    for (int i = 1; i < NI / 64; i++) v = min_limit(v, sm.vmin[i]);
     atomic_min_pos(&lim->vmin_bits, v);
   }
   if (er.err || er.nerr) {  // clamped into the box

@@ -648,7 +648,7 @@ __global__ void __launch_bounds__(GT) k_gravint(KParams P, GParams Gp, GGeo G, S
       for (int m = 0; m < 6; m++) qs[m] = double(S(qc[m]));
       const int e = cell_limits<EXACT>(P, qs, v, t);
       if (e && C.lim) report_next(C.lim, e, (unsigned long long)c);
-      vmin = dmin(vmin, v);
+      vmin = min_limit(vmin, v);
       if (tout) tout[c] = S(t);
     }
     __syncthreads();  // F is rewritten for the next plane only after every lane has read it

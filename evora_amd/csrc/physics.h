@@ -96,6 +96,10 @@ __device__ __forceinline__ T dmin(T a, T b) { return a < b ? a : b; }
 template <typename T>
 __device__ __forceinline__ T dmax(T a, T b) { return a > b ? a : b; }
 
+// The smaller of two limits.  A cell that is no number sets no limit and hides
+// no other's, whichever lane or wave it falls to (v_min_f64 takes the number).
+__device__ __forceinline__ double min_limit(double a, double b) { return __builtin_fmin(a, b); }
+
 // The minimum of a block's positive values into *a, with one atomic per block:
 // all blocks meet at one address, which takes about 10 ns each, so one per
 // wave made the limit of a 64 M-cell state wait for 33,000 of them (0.3 ms).
@@ -103,12 +107,12 @@ __device__ __forceinline__ T dmax(T a, T b) { return a > b ? a : b; }
 template <int NT>
 __device__ __forceinline__ void block_min_pos(unsigned long long *a, double v) {
   __shared__ double sh[NT / 64];
-  for (int off = 32; off > 0; off >>= 1) v = dmin(v, __shfl_xor(v, off));
+  for (int off = 32; off > 0; off >>= 1) v = min_limit(v, __shfl_xor(v, off));
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int i = 1; i < NT / 64; i++) v = dmin(v, sh[i]);
+    for (int i = 1; i < NT / 64; i++) v = min_limit(v, sh[i]);
     atomic_min_pos(a, v);
   }
 }

@@ -98,7 +98,7 @@ __global__ void __launch_bounds__(kBlock) k_hydrostep(KParams P, Grid G, const d
     double wc[5];
 #pragma unroll
     for (int m = 0; m < 5; m++) wc[m] = w[m * nw + wi];
-    v = dmin(v, cfl_cell(P, wc));
+    v = min_limit(v, cfl_cell(P, wc));
   }
   block_min_pos<kBlock>(&st->vmin_bits, v);
 }
@@ -264,7 +264,7 @@ __global__ void __launch_bounds__(kBlock) k_line_step(KParams P, const double *_
       }
       const int e = q2w(P, q, w);
       if (e) report_next(C.lim, e, (unsigned long long)i);
-      v = dmin(v, cfl_cell(P, w));
+      v = min_limit(v, cfl_cell(P, w));
     }
     fetch(i + (long long)gridDim.x * kLine);
   }

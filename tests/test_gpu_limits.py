@@ -64,3 +64,26 @@ def test_cell_without_pressure_is_found_in_a_batch():
             b.run(2, graph=False)
         assert e.value.code == 1 and e.value.box == 1 and e.value.cell == (HOT[0] + 1, HOT[1] + 1, nz // 2 + 1)
         assert b.times()[2].tolist() == [2, 1]
+
+
+@pytest.mark.parametrize("where", [63, 64, 126, 127, 255, 300])
+@pytest.mark.parametrize("precision,mode", [(hydro.FP64, hydro.MODE_FUSED), (hydro.FP64, hydro.MODE_FUSED_EXACT),
+                                            (hydro.FP64, hydro.MODE_STAGED), (hydro.FP32_MIXED, hydro.MODE_FUSED)])
+def test_cell_that_is_no_number_hides_no_limit(precision, mode, where):
+    """The limits come from the fastest cell, the first one here, wherever in
+    its wave or its block's other waves a density is no number."""
+    p = ics.conduction_params(16, nx=128, ny=4, nz=4)
+    one = np.ones((4, 4, 128))
+    pres = one.copy()
+    pres[0, 0, 0] = 100.0
+    q = ics.prim_to_q(p.derive(), one, 0 * one, 0 * one, 0 * one, pres)
+    got = []
+    for w in (None, where):
+        if w is not None:
+            q.reshape(-1, 6)[w, 0] = np.nan
+        with hydro.Hydro(p, precision=precision, mode=mode) as h:
+            h.upload_q(q)
+            h.primitive()
+            h.bound()
+            got.append((h.hydrostep(1e99), h.thermalstep(1e99)))
+    assert got[0] == got[1]
