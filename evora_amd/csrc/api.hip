@@ -658,9 +658,10 @@ static int run_on_device(evh_ctx *h, int nsteps, double *t, double tend, double 
   int r;
   if (line) {
     if ((r = ensure_staged_arrays(h))) return r;
+    // the limit alone: the step applies the dual-energy correction to q itself,
+    // and a q corrected twice may take the other branch
     HIP_TRY(launch_reset_status(h, false));
-    HIP_TRY(launch_primitive(h));
-    HIP_TRY(launch_hydrostep(h));
+    HIP_TRY(launch_cfl(h));
   } else if ((r = evh_primitive(h))) {
     return r;
   }

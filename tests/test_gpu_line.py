@@ -76,3 +76,30 @@ def test_line_stops_as_staged_steps_do(what):
                 h.upload_q(q0)
                 got[-1] += drive(h, 5)
     assert got[0] == got[1], got
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_line_corrects_the_first_state_once(seed):
+    """Dual energy, with an entropy that gives twice the pressure of E: the
+    corrected E is back under the threshold, so that a second correction would
+    take p from it.  Runs of one step (2 asked for, the end within the first)
+    and of four."""
+    n = 4000
+    p = ics.sod_params(n, solver=2, limiter=1, boundtype=2, cfl=0.4, dualenergy=True, de_thresh=0.1)
+    r = np.random.default_rng(seed).uniform(-0.1, 0.1, (2, 1, 1, n))
+    rho, u = 1 + r[0], 2 + r[1]
+    kin = 0.5 * rho * u * u  # kin / E = 1 / 1.1, just over the threshold of 0.9
+    q = ics.prim_to_q(p.derive(), rho, u, 0 * u, 0 * u, 2.0 / 3.0 * 0.1 * kin)
+    q[..., 5] *= 2
+    out = []
+    for drive in (hydro.Hydro.run, _steps):
+        got = []
+        for steps, tend in ((2, 1e-9), (4, 1e99)):
+            with hydro.Hydro(p) as h:
+                h.upload_q(q)
+                a = drive(h, steps, 0.0, tend)
+                got += [a, h.download_q(), h.download_w(), *h.download_evo_s()]
+        out.append(got)
+    assert out[0][0][2] == 1
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
