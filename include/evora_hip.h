@@ -117,7 +117,9 @@ int evh_download_phi(evh_ctx *h, double *phi);    /* the potential phi(nx,ny,nz)
  * gravity of main.f90:157-164 when gravity is on, with the expansion factor
  * of the last evh_gravpotential call, 1 at first), with updatetime
  * (timestep.f90:163-169): t, dt, go in/out.  evh_run repeats it nsteps
- * times (or until go turns 0), syncing only for dt. */
+ * times (or until go turns 0).  Where it can it forms dt and t on the device
+ * and looks at the run only every few steps, up to 64 (not with hipFFT's
+ * transforms, the staged kernels on 2-D and 3-D grids, or timed stages). */
 int evh_step(evh_ctx *h, double *t, double tend, double *dt, int *go);
 int evh_run(evh_ctx *h, int nsteps, double *t, double tend, double *dt, int *done);
 

@@ -3,6 +3,8 @@ the same steps taken one by one through evh_step (each with its own read of
 the limits): the same states, times and limits bit for bit, the same number
 of steps, the same stops; over more steps than one batch of launches, in runs
 that end early, after errors, and continued afterwards."""
+import time
+
 import numpy as np
 import pytest
 
@@ -129,3 +131,31 @@ def test_run_without_hydro_takes_each_steps_own_potential(precision, mode):
             out.append((a, b, c, *first, *end, h.download_q(), h.download_phi()))
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("name,steps", [("jeans", 1), ("jeans", 3), ("kh2d", 3)])
+def test_run_to_an_output_time_launches_few_steps_beyond_it(name, steps):
+    """A run asked for very many steps that ends after a few takes no longer
+    than the steps one by one, but for its own start (half as long again).
+    64 steps launched at once took 2.5 to 12 times as long."""
+    if name == "jeans":
+        p = ics.jeans_params(64)
+        q0 = ics.jeans(p, jeans_length=2.0)
+    else:
+        p = HydroParams(nx=128, ny=128, nz=1, solver=2, limiter=2, boundtype=2, cfl=0.4, atomic=False, tend=1e30)
+        q0 = ics.kh_reference(p)
+    best = []
+    for drive in (_run, _steps):
+        with hydro.Hydro(p) as h:
+            h.upload_q(q0)
+            t, dt, _ = drive(h, 5, 0.0, 1e30)
+            took = []
+            for _ in range(20):
+                h.synchronize()
+                t0 = time.perf_counter()
+                t, _, done = drive(h, 10**6, t, t + (steps - 0.5) * dt)
+                h.synchronize()
+                took.append(time.perf_counter() - t0)
+                assert done == steps
+            best.append(min(took))
+    assert best[0] < 1.5 * best[1], best
