@@ -377,13 +377,15 @@ struct Phys<true> {
 // in z the prefetch of plane nz + 2 after the last plane (never used; it
 // would fall outside the grid for nz = 2).  A column's offset is fixed for
 // the whole march, so only the plane's is formed per plane.
-// (An element index below 2^31: a plane of more cells would not leave room for
-// the state in device memory.)
-__device__ __forceinline__ int col_offset(const KParams &P, const Geo &G, int gx, int gy) {
+// A column's offset is an element index below 2^32 and takes all 32 bits: a
+// plane of more than 2^31 cells fits the 288 GB (FP32-mixed with nz = 2: both
+// buffers take 96 bytes per cell of it, 206 GB), one of 2^32 (412 GB) does not.
+using Col = unsigned;
+__host__ __device__ __forceinline__ Col col_offset(const KParams &P, const Geo &G, int gx, int gy) {
   const bool per = P.boundtype == 2;
   const int cx = gx < -2 ? -2 : (gx > G.nx + 1 ? G.nx + 1 : gx);
   const int cy = gy < -2 ? -2 : (gy > G.ny + 1 ? G.ny + 1 : gy);
-  return ghost_src(cx, G.nx, per) + G.nx * ghost_src(cy, G.ny, per);
+  return Col(ghost_src(cx, G.nx, per)) + Col(G.nx) * Col(ghost_src(cy, G.ny, per));
 }
 __device__ __forceinline__ long long plane_offset(const KParams &P, const Geo &G, int gz) {
   const int cz = gz < -2 ? -2 : (gz > G.nz + 1 ? G.nz + 1 : gz);
@@ -393,7 +395,7 @@ __device__ __forceinline__ long long plane_offset(const KParams &P, const Geo &G
 // raw q of the column at offset c of the plane at offset `plane` (the same in
 // all lanes)
 template <typename S>
-__device__ __forceinline__ void fetch_at(const Geo &G, const S *__restrict__ q, long long plane, int c, S raw[6]) {
+__device__ __forceinline__ void fetch_at(const Geo &G, const S *__restrict__ q, long long plane, Col c, S raw[6]) {
 #pragma unroll
   for (int m = 0; m < 6; m++) raw[m] = (q + (m * G.n + plane))[c];
 }
@@ -406,7 +408,7 @@ __device__ __forceinline__ void fetch_at(const Geo &G, const S *__restrict__ q, 
 // the kernels without the test.
 template <bool SLAB, typename S>
 __device__ __forceinline__ void fetch_plane(const KParams &P, const Geo &G, const S *__restrict__ q, int gz,
-                                            int c, S raw[6]) {
+                                            Col c, S raw[6]) {
   if constexpr (SLAB) {
     const long long pl = (long long)G.nx * G.ny;
     const S *h = nullptr;
@@ -551,7 +553,7 @@ __device__ __forceinline__ void march_columns(const KParams &P, const Geo &G, co
   T wm[5], wc[5], wp[5], qc[6], qn[6];
   T rc, rp;
   S pre[6];
-  const int own_xy = col_offset(P, G, gx, gy);
+  const Col own_xy = col_offset(P, G, gx, gy);
   {
     S ra[6], rb[6];  // all three planes in flight together
     fetch_plane<SLAB>(P, G, qin, z0 - 2, own_xy, ra);
@@ -708,7 +710,7 @@ __device__ __forceinline__ void march_ring(const KParams &P, const Geo &G, const
   bool owns[NP], second[NP], wall[NP], wall2[NP], isx[NP];
   T half[NP], *out[NP];
   int ostride[NP], me[NP], slot2[NP];
-  int own_xy[NP], r2_xy[NP];
+  Col own_xy[NP], r2_xy[NP];
   T wm[NP][5], wc[NP][5], wp[NP][5], rc[NP], rp[NP], rw2[NP][5], tq[6], tr;
   S pre[NP][6], pre2[NP][6];
 #pragma unroll

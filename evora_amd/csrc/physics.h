@@ -317,7 +317,7 @@ __device__ __forceinline__ int riemann(const KParams &P, const T wl[5], const T 
 // cell in [0, n).  Zero-gradient ghosts mirror (w(lx-2) = w(lx+1),
 // boundary.f90:36-37); periodic wraps.  Composing the per-axis maps
 // reproduces the x -> y -> z fill over full extents (edges and corners).
-__device__ __forceinline__ int ghost_src(int g, int n, bool periodic) {
+__host__ __device__ __forceinline__ int ghost_src(int g, int n, bool periodic) {
   if (g < 0) return periodic ? g + n : -1 - g;
   if (g >= n) return periodic ? g - n : 2 * n - 1 - g;
   return g;
