@@ -496,7 +496,7 @@ struct CflMin {
   // the wave's minimum, in every lane
   __device__ __forceinline__ double wave_min() {
     if constexpr (kSpeedKey) v = fm::rcp(-v);
-    for (int off = 32; off > 0; off >>= 1) v = min_limit(v, __shfl_xor(v, off));
+    for (int off = 32; off > 0; off >>= 1) v = min_limits(v, __shfl_xor(v, off));
     return v;
   }
 };
@@ -891,7 +891,7 @@ __device__ __forceinline__ void march(const KParams &P, const Geo &G, const S *_
   if (lim && threadIdx.x == 0) {
     double v = sm.vmin[0];
 #pragma unroll
-    for (int i = 1; i < NI / 64; i++) v = min_limit(v, sm.vmin[i]);
+    for (int i = 1; i < NI / 64; i++) v = min_limits(v, sm.vmin[i]);
     atomic_min_pos(&lim->vmin_bits, v);
   }
   if (er.err || er.nerr) {  // clamped into the box
