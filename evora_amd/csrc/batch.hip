@@ -116,7 +116,7 @@ __global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((
       Status *const st = &bs.st[b];
       __builtin_assume(st != nullptr);
       core::march<T, S, SOLVER, LIMITER, TX, TY, false>(P, G, to1 ? q0 : q1, to1 ? q1 : q0, bx.qoff, b, bs.dt[b], st, st,
-                                                    nullptr, item - lo, sm);
+                                                    item - lo, sm);
     }
     __syncthreads();  // s_item is rewritten only after every lane has used it
   }

@@ -45,7 +45,7 @@ __global__ void __launch_bounds__((core::TileShape<TX, TY>::NT)) __attribute__((
   const int lin = xcd_tile(blockIdx.x, G.ntiles);
   double dt;
   if (!step_begin(P, C, dt) || lin < 0) return;  // no step, or a padding block (whole blocks, before any barrier)
-  core::march<T, S, SOLVER, LIMITER, TX, TY, kExact, SLAB>(P, G, qin, qout, 0, 0, dt, C.st, C.lim, C.prev, lin, sm, tout);
+  core::march<T, S, SOLVER, LIMITER, TX, TY, kExact, SLAB>(P, G, qin, qout, 0, 0, dt, C.st, C.lim, lin, sm, tout);
 }
 
 // 2-D grids (nz = 1): row strips marching along y (march2d.h)
@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(core2d::NL) __attribute__((amdgpu_waves_per_eu
   const int lin = xcd_tile(blockIdx.x, G.ntiles);
   double dt;
   if (!step_begin(P, C, dt) || lin < 0) return;  // no step, or a padding block (whole blocks, before any barrier)
-  core2d::march2d<T, S, SOLVER, LIMITER, kExact>(P, G, qin, qout, dt, C.st, C.lim, C.prev, lin, sm, tout);
+  core2d::march2d<T, S, SOLVER, LIMITER, kExact>(P, G, qin, qout, dt, C.st, C.lim, lin, sm, tout);
 }
 
 // primitive + CFL min over q without materialising w (first step, after

@@ -844,9 +844,8 @@ __device__ __forceinline__ void march_ring(const KParams &P, const Geo &G, const
 
 // One tile `lin` (x fastest, then y, then z chunk) of the box whose q starts
 // at element qoff of qin_all/qout_all.  st takes the step's errors, lim (unless
-// null) the CFL minimum and the negative pressures of the new state; prev (or null)
-// is the block of the step before.  Errors carry the box index above bit 40 of
-// the cell.
+// null) the CFL minimum and the negative pressures of the new state; errors carry the box
+// index above bit 40 of the cell.
 // With tout (single box only), the temperature of each new cell is stored
 // there too, for the conduction pass that follows the sweep.  SLAB: the grid
 // is a z-slab whose ghost planes may come from halo buffers (Geo::zlo, zhi).
@@ -855,7 +854,7 @@ __device__ __forceinline__ void march_ring(const KParams &P, const Geo &G, const
 template <typename T, typename S, int SOLVER, int LIMITER, int TX, int TY, bool EXACT, bool SLAB = false>
 __device__ __forceinline__ void march(const KParams &P, const Geo &G, const S *__restrict__ qin_all,
                                       S *__restrict__ qout_all, long long qoff, int box, double dt, Status *st,
-                                      Status *lim, const Status *prev, int lin, Smem<T, TX, TY> &sm,
+                                      Status *lim, int lin, Smem<T, TX, TY> &sm,
                                       S *__restrict__ tout = nullptr) {
   using TS = TileShape<TX, TY>;
   constexpr int NI = TS::NI;
@@ -898,7 +897,7 @@ __device__ __forceinline__ void march(const KParams &P, const Geo &G, const S *_
   if (er.err || er.nerr) {  // clamped into the box
     const unsigned long long tag = (unsigned long long)box << 40;  // box index above the cell index
     const long long ex = min(max(gx, 0), G.nx - 1), ey = min(max(gy, 0), G.ny - 1);
-    if (er.err) report(st, prev, er.err, tag | (unsigned long long)(ex + G.nx * (ey + (long long)G.ny * er.err_k)));
+    if (er.err) report(st, er.err, tag | (unsigned long long)(ex + G.nx * (ey + (long long)G.ny * er.err_k)));
     if (lim && er.nerr) report_next(lim, er.nerr, tag | (unsigned long long)(ex + G.nx * (ey + (long long)G.ny * er.nerr_k)));
   }
 }

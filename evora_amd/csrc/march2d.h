@@ -84,7 +84,7 @@ __device__ __forceinline__ void prim2(const KParams &P, const Geo2 &G, const S r
 // and with tout the temperature of each new cell is stored.
 template <typename T, typename S, int SOLVER, int LIMITER, bool EXACT>
 __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *__restrict__ qin,
-                                        S *__restrict__ qout, double dt, Status *st, Status *lim, const Status *prev,
+                                        S *__restrict__ qout, double dt, Status *st, Status *lim,
                                         int lin, Smem2<T> &sm, S *__restrict__ tout) {
   using Ph = core::Phys<EXACT>;
   T(&W)[5][NL] = sm.W;
@@ -250,7 +250,7 @@ __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *
 
   if (err || nerr) {  // the lane's own column (clamped into the grid) locates the error
     const long long ex = min(max(gx, 0), G.nx - 1);
-    if (err) report(st, prev, err, (unsigned long long)(ex + G.nx * (long long)err_k));
+    if (err) report(st, err, (unsigned long long)(ex + G.nx * (long long)err_k));
     if (lim && nerr) report_next(lim, nerr, (unsigned long long)(ex + G.nx * (long long)nerr_k));
   }
   if (lim) block_min_pos<NL>(&lim->vmin_bits, cfl.wave_min());

@@ -82,13 +82,6 @@ __device__ __forceinline__ void report(Status *st, int code, unsigned long long 
   if (atomicCAS(&st->code, 0, code) == 0) atomicExch(&st->cell, cell);
 }
 
-// An error of a step whose predecessor's block is `before` (nullptr: none): one
-// that is still unread there is the first, whoever comes first here.
-__device__ __forceinline__ void report(Status *st, const Status *before, int code, unsigned long long cell) {
-  const bool older = before && before->code;
-  report(st, older ? before->code : code, older ? before->cell : cell);
-}
-
 __device__ __forceinline__ void report_next(Status *st, int code, unsigned long long cell) {
   if (atomicCAS(&st->next_code, 0ull, (unsigned long long)code) == 0ull) atomicExch(&st->next_cell, cell);
 }
