@@ -77,6 +77,8 @@ __global__ void k_clear_code(Status *st) {
   if (threadIdx.x == 0) {
     st->code = 0;
     st->cell = 0;
+    st->old_code = 0;
+    st->old_cell = 0;
     st->next_code = 0;
     st->next_cell = 0;
     st->vmin_bits = (unsigned long long)__double_as_longlong(kVInit);
@@ -197,9 +199,8 @@ hipError_t timer_end(evh_ctx *h, int stage) {
 
 // Surface the device-side errors of a status block read into st_host.
 int surface_errors(evh_ctx *h) {
-  if (h->st_host->code) {
-    const int code = h->st_host->code;
-    const long long cell = (long long)h->st_host->cell;
+  if (const int code = first_code(*h->st_host)) {
+    const long long cell = (long long)first_cell(*h->st_host);
     hipLaunchKernelGGL(k_clear_code, dim3(1), dim3(64), 0, h->stream, h->st);
     hipStreamSynchronize(h->stream);
     h->v_valid = false;

@@ -69,14 +69,17 @@ __device__ __forceinline__ double uniform(double v) { return v; }  // FP64 kerne
 // Device status block: first error (code, linear cell) and min reductions.
 struct Status {
   int code;           // first error code seen (0 = none)
-  int pad;
+  int old_code;       // an error of an earlier step that nobody has read yet
   unsigned long long cell;  // linear index of an offending cell (x fastest), or ~0
   unsigned long long vmin_bits;   // CFL min of dx/(|u|+a) (positive double bits)
   unsigned long long next_code;   // error found while computing the next step's primitive
   unsigned long long next_cell;
   unsigned long long tvmin_bits;  // conduction limit: min of rho / kappa (positive double bits)
-  unsigned long long pad_;
+  unsigned long long old_cell;
 };
+// the first error of a block
+__host__ __device__ __forceinline__ int first_code(const Status &s) { return s.old_code ? s.old_code : s.code; }
+__host__ __device__ __forceinline__ unsigned long long first_cell(const Status &s) { return s.old_code ? s.old_cell : s.cell; }
 
 __device__ __forceinline__ void report(Status *st, int code, unsigned long long cell) {
   if (atomicCAS(&st->code, 0, code) == 0) atomicExch(&st->cell, cell);

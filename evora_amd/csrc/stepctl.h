@@ -48,6 +48,8 @@ struct StepCtl {
 __device__ __forceinline__ void clear_status(Status *s) {
   s->code = 0;
   s->cell = 0;
+  s->old_code = 0;
+  s->old_cell = 0;
   s->next_code = 0;
   s->next_cell = 0;
   s->vmin_bits = (unsigned long long)__double_as_longlong(1e6);   // timestep.f90:35
@@ -61,7 +63,10 @@ __device__ __forceinline__ bool step_begin(const KParams &P, const StepCtl &C, d
   dt = C.dt;
   if (!C.in) {
     if (first && C.reset) clear_status(C.reset);
-    if (first && C.prev && C.prev->code) report(C.st, C.prev->code, C.prev->cell);  // errors stay until read
+    if (first && C.prev) {  // errors stay until read, and before those that other blocks report meanwhile
+      C.st->old_code = first_code(*C.prev);
+      C.st->old_cell = first_cell(*C.prev);
+    }
     return true;
   }
   if (!C.head) {
@@ -74,7 +79,7 @@ __device__ __forceinline__ bool step_begin(const KParams &P, const StepCtl &C, d
     if (!s.go) {
       s.why = kRunEnd;
       s.dt = C.in->dt;
-    } else if (C.prev->code) {
+    } else if (first_code(*C.prev)) {
       s.why = kRunCode;
     } else if (C.prev->next_code) {
       s.why = kRunNext;

@@ -58,3 +58,30 @@ def test_calls_out_of_order():
         with pytest.raises(hydro.EvoraError) as ei:
             h.bound()
         assert ei.value.code == 10
+
+
+@pytest.mark.parametrize("nz", [1, 24])
+@pytest.mark.parametrize("mode", [hydro.MODE_FUSED, hydro.MODE_FUSED_EXACT])
+def test_first_error_stays_until_read(mode, nz):
+    """Sweeps without a read between them: a cell of the first sweep's errors is
+    reported, although the next sweeps find others further out, in blocks that
+    end in any order."""
+    p = HydroParams(nx=96, ny=64, nz=nz, solver=2, limiter=1, boundtype=1, cfl=0.4, atomic=True)
+    d = p.derive()
+    one = np.ones((nz, 64, 96))
+    u = 0 * one
+    x0, y0, z0 = 40, 30, nz // 2
+    u[z0, y0, x0 - 3:x0 + 4] = np.linspace(-1, 1, 7)  # gas that parts: at a large dt the predicted pressure is negative
+    for _ in range(5):
+        with hydro.Hydro(p, mode=mode) as h:
+            h.upload_q(ics.prim_to_q(d, one, u, 0 * one, 0 * one, one))
+            h.primitive()
+            dt = 40 * h.hydrostep(1e99)
+            for _ in range(4):
+                h.compevo(dt)
+                h.sweep(dt)
+            with pytest.raises(hydro.EvoraError) as ei:
+                h.hydrostep(1e99)
+        assert ei.value.code == 2
+        x, y, z = ei.value.cell
+        assert abs(x - 1 - x0) <= 4 and abs(y - 1 - y0) <= 1 and abs(z - 1 - z0) <= 1, ei.value.cell
