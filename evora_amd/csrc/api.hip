@@ -292,14 +292,16 @@ KParams make_kparams(const evh_config &c) {
   k.c_cond = c.c_cond;
   k.temp0 = c.temp0;
   k.kappa0 = c.kappa0;
-  k.ggm = k.g * k.g1;
-  // 4e-6 is above the FP32 rounding of E - kin; with dual energy p comes from
-  // E while kin <= de_thresh1 E
-  // (for g <= 1 no cell has p > 0 by it)
-  k.calm = !(k.g1 > 0.0) ? INFINITY : 4e-6 + (k.dualenergy ? std::fmax(0.0, 1.0 - k.de_thresh1) : 0.0);
+  k.ggm = 0.5 * (k.g * k.g1);
+  // E - kin > c E is 2 rho E - m^2 > c / (1 - c) m^2 where rho E > 0.  4e-6 is
+  // far above the rounding of E - kin in FP64, and small beside the margin of
+  // dual energy, with which p comes from E while kin <= de_thresh1 E.  Never
+  // where c takes all of E, or g <= 1, by which p > 0 has E < kin.
+  const double c4 = 4e-6 + (k.dualenergy ? std::fmax(0.0, 1.0 - k.de_thresh1) : 0.0);
+  k.calm = k.g1 > 0.0 && c4 < 1.0 ? c4 / (1.0 - c4) : INFINITY;
   k.f = {float(k.g), float(k.g1), float(k.g1inv), float(k.gg1), float(k.de_thresh1), float(k.kin_frac64),
          float(k.temp0), float(k.dxinv), float(k.dyinv), float(k.dzinv),
-         float(k.dx), float(k.dy), float(k.dz), float(k.ggm), float(k.calm)};
+         float(k.dx), float(k.dy), float(k.dz)};
   return k;
 }
 

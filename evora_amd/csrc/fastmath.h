@@ -166,6 +166,15 @@ __device__ __forceinline__ double div_sqrt_pos(double n, double x) {
   return __builtin_fma(a * e, __builtin_fma(e, 0.375, 0.5), a);
 }
 
+// sqrt(x) for positive, normal x, from the rsq estimate: the third-order step
+// on the exact residual of g = x y, so that only the last fma rounds
+__device__ __forceinline__ double sqrt_near(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double g = x * y;
+  const double t = __builtin_fma(-g, g, x) * y;
+  return __builtin_fma(t, __builtin_fma(t * y, 0.375, 0.5), g);
+}
+
 // a*b + c fused, and |a|, in either type.  The builds of the march are
 // compiled without contraction and place every fused operation by hand, so
 // that each inlined call site of the same expression rounds alike.

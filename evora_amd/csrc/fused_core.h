@@ -461,33 +461,33 @@ __device__ __forceinline__ void store_w(T (*W)[EA], int slot, const T w[5]) {
 // 256^3 shock and cloud FP64 0.784 ms with it, 0.741 without; FP32-mixed 0.390,
 // 0.371; 512^3 blast in 1% noise 5.43, 5.46; FP32-mixed 2.51, 2.58.
 //
-// The FP64 fast form keeps -max_d (..) per cell and inverts once per lane,
-// and where p comes from E by a margin above the rounding of any form (and p
-// > 0, so that nothing is to be reported) takes it from q without the
-// primitive: (a rho)^2 = g g1 (rho E - m^2/2), max_d (|m_d| + a rho) / dx_d
-// times 1/rho, 25 operations for 47, both to a few ulp (times E/p, as with
-// p = g1 (E - kin)).  A lane without cells gives 1e6.
+// Where p comes from E by a margin above its rounding (and p > 0, so that
+// nothing is to be reported) the FP64 fast form takes the limit from q without
+// the primitive: rho / max_d (|m_d| + a rho) / dx_d with (a rho)^2 = g g1/2
+// (2 rho E - m^2), 27 operations for 47.  Six roundings, those of the square
+// halved by its root: against 80 bits, over gas at rest and in motion in 2-D
+// and 3-D, rms 0.9e-16 (times E/p, as with p = g1 (E - kin)), where the
+// primitive's arithmetic gives 1.0e-16 and the reciprocal of a speed from q,
+// without the residuals of root and quotient, 1.2e-16.  A lane without cells
+// gives 1e6.
 template <typename T, bool EXACT>
 struct CflMin {
-  static constexpr bool kSpeedKey = !EXACT && sizeof(T) == 8;
-  double v = kSpeedKey ? -1e-6 : 1e6;
+  double v = 1e6;
   __device__ __forceinline__ void add(const KParams &P, const T w[5], T rinv) {
-    if constexpr (kSpeedKey) v = min_limit(v, -fast::cfl_speed(P, w, rinv));
-    else v = min_limit(v, Phys<EXACT>::cfl_cell(P, w, rinv));
+    v = min_limit(v, Phys<EXACT>::cfl_cell(P, w, rinv));
   }
   // from q; false where it takes the primitive (and for NaN)
   __device__ __forceinline__ bool add(const KParams &P, const T q[6]) {
-    if constexpr (kSpeedKey) {
-      const double er = q[4] * q[0];
+    if constexpr (!EXACT && sizeof(T) == 8) {
       const double m2 = fm::fma(q[3], q[3], fm::fma(q[2], q[2], q[1] * q[1]));
-      const double x = fm::fma(-0.5, m2, er);
-      // with rho < 0, or E < 0 and calm >= 1, an x above calm rho E is no pressure above 0
-      if (!(q[0] > 0.0 && x > P.calm * fm::fabs(er))) return false;
-      const double a2 = P.ggm * x, ar = fm::div_sqrt_pos(a2, a2);
+      const double x = fm::fma(q[4] + q[4], q[0], -m2);
+      if (!(q[0] > 0.0 && x > P.calm * m2)) return false;  // x > 0 says rho E > 0
+      const double ar = fm::sqrt_near(P.ggm * x);
       const double sx = (fm::fabs(q[1]) + ar) * P.dxinv;
       const double sy = (fm::fabs(q[2]) + ar) * P.dyinv;
       const double sz = (fm::fabs(q[3]) + ar) * P.dzinv;
-      v = min_limit(v, -(dmax(dmax(sx, sy), sz) * fm::rcp(q[0])));
+      const double s = dmax(dmax(sx, sy), sz);
+      v = min_limit(v, fm::div_cr(q[0], s, fm::rcp(s)));
       return true;
     } else {
       return false;
@@ -495,7 +495,6 @@ struct CflMin {
   }
   // the wave's minimum, in every lane
   __device__ __forceinline__ double wave_min() {
-    if constexpr (kSpeedKey) v = fm::rcp(-v);
     for (int off = 32; off > 0; off >>= 1) v = min_limits(v, __shfl_xor(v, off));
     return v;
   }

@@ -41,13 +41,13 @@ struct KParams {
   int g1_third;       // |2/3 - g1| <= 1e-6: powers of g1 via the cube root
   int conduction;     // thermal conduction (simplekappa) on
   double c_cond, temp0, kappa0;
-  double ggm;   // g g1: (a rho)^2 = ggm (rho E - m^2/2)
-  double calm;  // share of rho E that rho E - m^2/2 exceeds where p > 0 comes from E in every form
+  double ggm;   // g g1/2: (a rho)^2 = ggm (2 rho E - m^2)
+  double calm;  // share of m^2 that 2 rho E - m^2 exceeds where p > 0 comes from E, and to be sure of it
   // the same rounded to single precision, for the FP32-mixed kernels: read
   // from here they stay in scalar registers, where a conversion in the kernel
   // (the vector unit's) would hold a vector register each for its whole loop
   struct Single {
-    float g, g1, g1inv, gg1, de_thresh1, kin_frac64, temp0, dxinv, dyinv, dzinv, dx, dy, dz, ggm, calm;
+    float g, g1, g1inv, gg1, de_thresh1, kin_frac64, temp0, dxinv, dyinv, dzinv, dx, dy, dz;
   } f;
 };
 
