@@ -264,7 +264,7 @@ struct evh_batch {
   std::vector<char> cfl_needed;
   // launch shape
   int tile_ty = 12, wpe_hi = 1, zchunk = 64, blocks_per_cu = 2;
-  bool auto_chunk = true;  // no z chunk set: by the boxes (batch_chunk)
+  bool auto_chunk = true;  // no z chunk set: zchunk is the boxes' (batch_chunk)
   int tx = 16, ty = 12;  // the column tile that tile_ty stands for (pick_tile)
   // one step of the ensemble, captured once (the kernels read each box's
   // buffer side from device memory)
@@ -418,10 +418,9 @@ int rebuild_items(evh_batch *b) {
   std::vector<BoxDev> h(b->nbox);
   Queues q;
   pick_tile(b->cfgs.data(), b->nbox, b->tile_ty, &b->tx, &b->ty);
-  const int zc = b->auto_chunk ? batch_chunk(b->cfgs.data(), b->nbox, b->tx, b->ty, b->blocks_per_cu * b->num_cu)
-                               : b->zchunk;
+  if (b->auto_chunk) b->zchunk = batch_chunk(b->cfgs.data(), b->nbox, b->tx, b->ty, b->blocks_per_cu * b->num_cu);
   b->nitems = describe_boxes(b->cfgs.data(), b->kps.data(), b->ncell.data(), b->qoff.data(), b->nbox, b->tx, b->ty,
-                             zc, h.data(), &q);
+                             b->zchunk, h.data(), &q);
   BHIP(hipMemcpy(b->boxes_d, h.data(), sizeof(BoxDev) * b->nbox, hipMemcpyHostToDevice));
   BHIP(hipMemcpy(b->qs_d, &q, sizeof(Queues), hipMemcpyHostToDevice));
   if (b->gexec) {

@@ -238,7 +238,8 @@ int evh_batch_run(evh_batch *b, int nsteps, int use_graph, float *ms);
 int evh_batch_times(evh_batch *b, double *t, double *dt, int *steps, int *go);
 /* launch shape as evh_set_tuning: tile height 8|12, occupancy target 0|1 (one
  * register budget either way), z chunk (64 until it is set, less for boxes
- * that together give too few items), blocks per CU */
+ * that together give too few items; evh_batch_get_tuning gives the one in
+ * force), blocks per CU */
 int evh_batch_set_tuning(evh_batch *b, int tile_ty, int wpe_hi, int zchunk, int blocks_per_cu);
 int evh_batch_get_tuning(evh_batch *b, int *tile_ty, int *wpe_hi, int *zchunk, int *blocks_per_cu);
 /* time every launch shape for trial_steps steps on a snapshot of the state,

@@ -183,3 +183,25 @@ def test_batch_configured_ensemble():
 def _prim(q, g1):
     rho = q[..., 0]
     return rho, g1 * (q[..., 4] - 0.5 * (q[..., 1] ** 2 + q[..., 2] ** 2 + q[..., 3] ** 2) / rho)
+
+
+def test_tuning_that_was_read_can_be_set_back():
+    """The shape that get_tuning gives is the one in force: set back, it leaves
+    the time of a step as it was (64 planes per item took twice as long
+    here)."""
+    rng = np.random.default_rng(3)
+    params = [HydroParams(nx=int(n[0]), ny=int(n[1]), nz=int(n[2]), solver=2, limiter=1, boundtype=1, cfl=0.3, atomic=True)
+              for n in rng.integers(16, 48, (32, 3))]
+    with Batch(params) as b:
+        for i, p in enumerate(params):
+            q = np.zeros((p.nz, p.ny, p.nx, 6))
+            q[..., 0], q[..., 4], q[..., 5] = 1.0, 1.5, 1.0
+            b.upload_q(i, q)
+        b.run(20)
+        took = [min(b.run(20) for _ in range(5))]
+        shape = b.get_tuning()
+        b.set_tuning(*shape)
+        b.run(20)
+        took.append(min(b.run(20) for _ in range(5)))
+        assert b.get_tuning() == shape
+    assert took[1] < 1.25 * took[0], (took, shape)
