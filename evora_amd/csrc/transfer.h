@@ -121,8 +121,9 @@ class CopyTeam {
 // the last of a download have nothing beside them.
 // Upload: in one piece up to 10 MB (5.3 MB: 200 us, 215 in two, 255 in five),
 // then about the root of the size in MB (12.6 MB: 4 MB; 42 MB: 8 to 12; 805 MB:
-// 24 to 32), through two buffers; more gain nothing, and the first touch of
-// one takes 0.34 ms per MB.
+// 24 to 32).  Two buffers would do, but it takes the whole pool in equal parts:
+// the first touch of its pages, 0.34 ms per MB, then falls to the first upload
+// and not to the first download too.
 // Download: an eighth, between 1 and 16 MB (5.3 MB: 266 us, 321 in one piece),
 // through four buffers where the pool has them: a fresh array takes its page
 // faults between the chunks, and they keep the link busy meanwhile (128^3 2.70
@@ -151,7 +152,9 @@ inline ChunkPlan chunk_plan(long long n, long long bytes, bool up, long long poo
   const long long most = pool / bytes;
   long long units = chunk_units(n, bytes, up);
   if (units < n ? 2 * units > most : units > most) units = std::max(1LL, most / 2);
-  return {units, (int)std::min(up ? 2LL : (long long)kBuffers, most / units)};
+  const long long parts = (2 * most + units) / (2 * units);
+  if (up && units < n && parts <= kBuffers) units = most / parts;
+  return {units, (int)std::min((long long)kBuffers, most / units)};
 }
 
 struct Xfer {
