@@ -37,7 +37,7 @@ struct evh_ctx {
   int mode = EVH_MODE_FUSED;
   int zchunk = 0;   // z planes per fused block (0: default)
   int tile_ty = 12;    // fused tile height: 8 or 12
-  bool wpe_hi = true;  // register budget for the higher of the two occupancy targets
+  bool wpe_hi = true;  // the occupancy target as set, for evh_get_tuning: one register budget either way
   hipStream_t stream = nullptr;
   hipEvent_t events[8] = {};
 
@@ -82,7 +82,7 @@ struct evh_ctx {
   // staged path arrays (allocated on first use)
   double *w = nullptr, *evo = nullptr, *s = nullptr;
 
-  // host transfers (pinned, double-buffered chunks)
+  // host transfers (chunks through pinned buffers)
   evh::Xfer xfer;
 
   // reductions

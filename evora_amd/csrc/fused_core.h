@@ -34,12 +34,12 @@
 // instruction takes about 5 cycles of its SIMD, and the SIMDs that hold
 // interior waves only have one to issue 98% of the time); FP32-mixed, the
 // L1's requests to L2 for the ring.  512^3 HLLC blast, FP64: 6.36 ms with both
-// roles in one loop (219 VGPRs) and the carry in LDS; 5.46 ms (24.6 G cell
+// roles in one loop (219 VGPRs) and the carry in LDS; 5.49 ms (24.4 G cell
 // updates/s) with a loop per role, so that neither holds the other's values
 // (the carry in registers, 32 of 135 LDS operations per plane gone, 46 KB of
 // LDS instead of 72), third-order reciprocals and roots, the star flux from
 // its jump conditions, the predictor from shared factors, and the limit from
-// q.  FP32-mixed: 3.33 -> 2.58 ms (52 G), with its constants in scalar
+// q.  FP32-mixed: 3.33 -> 2.62 ms (51 G), with its constants in scalar
 // registers (16 B/lane of spills gone) and the 32 x 6 tile.
 #pragma once
 

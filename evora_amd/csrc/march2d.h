@@ -13,8 +13,8 @@
 //       LDS; the y face k-1/2 is solved from the top state of row k-1
 //       (carried) and the bottom state of row k, and row k-1 is finished as
 //       (q + dtx*(Fx)) + dty*(Fy), the reference's x, y order, and stored,
-//       with the primitive and CFL limit of the cells that can change the
-//       minimum (and, with conduction, the temperature of all);
+//       with the CFL limit of its cells (core::CflMin) and, with
+//       conduction, their temperature;
 //   S3  the x faces of row k, one per lane;
 //   S4  q(k) + dtx*(Fx) of row k, carried to row k+1.
 // Every lane does useful work in every stage except the four ghost lanes in
@@ -79,9 +79,10 @@ __device__ __forceinline__ void prim2(const KParams &P, const Geo2 &G, const S r
   }
 }
 
-// One strip-chunk `lin` (strips fastest).  As core::march: vmin_dst receives
-// the CFL minimum of the new state, errors are reported once after the march,
-// and with tout the temperature of each new cell is stored.
+// One strip-chunk `lin` (strips fastest).  As core::march: st takes the step's
+// errors, lim (unless null) the CFL minimum and the negative pressures of the
+// new state, errors are reported once after the march, and with tout the
+// temperature of each new cell is stored.
 template <typename T, typename S, int SOLVER, int LIMITER, bool EXACT>
 __device__ __forceinline__ void march2d(const KParams P, const Geo2 G, const S *__restrict__ qin,
                                         S *__restrict__ qout, double dt, Status *st, Status *lim,

@@ -5,10 +5,10 @@
 // previous step left: read on the host, it costs a wait, a copy and the
 // launches behind it, about 20 us, more than a small grid's kernel.  In a run
 // of several steps (evh_run) the host therefore only launches: the first
-// kernel of each step (its head) forms dt, t and the end of the run as
-// hydrostep, thermalstep and updatetime do (timestep.f90:26-57,72-104,
-// 147-171), every block from the same values and one of them storing the
-// result for the next step.  A step after the end, or after an error, does
+// kernel of each step (its head; one of its own where the potential's passes
+// come first) forms dt, t and the end of the run as hydrostep, thermalstep and
+// updatetime do (timestep.f90:26-57,72-104,147-171), every block from the same
+// values and one of them storing the result for the next step.  A step after the end, or after an error, does
 // nothing.  128^2 2-D Kelvin-Helmholtz: 31 -> 17 us per step (12 with its
 // shorter chunks); 64^3: 62 -> 43 us (30 with them).
 //

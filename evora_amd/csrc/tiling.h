@@ -30,9 +30,10 @@ inline int xcd_blocks(int ntiles) { return kXcds * ((ntiles + kXcds - 1) / kXcds
 // cover a plane of the grid (or of all boxes together).  The wide tile's ring
 // has half the columns beyond its x sides, each of which costs the L1 a
 // request of a whole line for one value, and more columns in all.  FP32 is
-// bound by those requests: 512^3 2.51 ms wide against 2.78, 384^3 1.15 against
-// 1.26, 256^3 0.361 against 0.387.  FP64 is bound by instruction issue, the
-// ring's included: 512^3 5.55 ms wide against 5.39, 256^3 0.765 against 0.735.
+// bound by those requests: 512^3 2.64 ms wide against 2.86, 384^3 1.23 against
+// 1.31, 256^3 0.429 against 0.440 (7 to 19 steps of a blast, events).  FP64 is
+// bound by instruction issue, the ring's included: 512^3 5.65 ms wide against
+// 5.49, 384^3 2.45 against 2.39, 256^3 0.838 against 0.805.
 inline long long tiles_of(int nx, int ny, int tx, int ty) {
   return (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
 }
