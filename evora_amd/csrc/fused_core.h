@@ -464,7 +464,7 @@ __device__ __forceinline__ void store_w(T (*W)[EA], int slot, const T w[5]) {
 // Where p comes from E by a margin above its rounding (and p > 0, so that
 // nothing is to be reported) the FP64 fast form takes the limit from q without
 // the primitive: rho / max_d (|m_d| + a rho) / dx_d with (a rho)^2 = g g1/2
-// (2 rho E - m^2), 27 operations for 47.  Six roundings, those of the square
+// (2 rho E - m^2), 28 operations for 47.  Six roundings, those of the square
 // halved by its root: against 80 bits, over gas at rest and in motion in 2-D
 // and 3-D, rms 0.9e-16 (times E/p, as with p = g1 (E - kin)), where the
 // primitive's arithmetic gives 1.0e-16 and the reciprocal of a speed from q,
@@ -481,7 +481,8 @@ struct CflMin {
     if constexpr (!EXACT && sizeof(T) == 8) {
       const double m2 = fm::fma(q[3], q[3], fm::fma(q[2], q[2], q[1] * q[1]));
       const double x = fm::fma(q[4] + q[4], q[0], -m2);
-      if (!(q[0] > 0.0 && x > P.calm * m2)) return false;  // x > 0 says rho E > 0
+      // x > 0 says rho E > 0; x that has over- or underflown takes the primitive
+      if (!(x > fm::fma(P.calm, m2, 1e-290) && x < 1e300 * q[0])) return false;
       const double ar = fm::sqrt_near(P.ggm * x);
       const double sx = (fm::fabs(q[1]) + ar) * P.dxinv;
       const double sy = (fm::fabs(q[2]) + ar) * P.dyinv;

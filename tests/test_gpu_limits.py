@@ -122,3 +122,27 @@ def test_limit_of_the_fast_form_is_as_near_as_six_roundings():
     one = 2.0 ** -52 / np.sqrt(12) * np.sqrt(3 / (8 * np.log(2)))
     rms = float(np.sqrt(np.mean(np.square(err))))
     assert rms <= np.sqrt(5 + 2 / 4) * one, rms
+
+
+@pytest.mark.parametrize("nz", [1, 4])
+@pytest.mark.parametrize("scale", [1e154, 1e-152])
+def test_limit_does_not_depend_on_the_unit_of_density(scale, nz):
+    """Density and pressure in another unit leave every speed as it is: also
+    where 2 rho E leaves the range of the type (rho p g, which the solvers
+    form, does not)."""
+    p = HydroParams(nx=20, ny=12, nz=nz, solver=2, limiter=1, boundtype=2, cfl=0.3, atomic=True)
+    d = p.derive()
+    r = np.random.default_rng(2)
+    rho, pres = r.uniform(0.95, 1.0, (2, nz, 12, 20))
+    v = r.uniform(-0.05, 0.05, (3, nz, 12, 20))
+    got = []
+    for unit in (1.0, scale):
+        with hydro.Hydro(p) as h:
+            h.upload_q(ics.prim_to_q(d, unit * rho, *v, unit * 0.7 * pres))
+            h.primitive()
+            dt = 0.2 * h.hydrostep(1e99)
+            h.compevo(dt)
+            h.sweep(dt)
+            h.primitive()
+            got.append(h.hydrostep(1e99))
+    assert got[1] == pytest.approx(got[0], rel=1e-13)
